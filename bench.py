@@ -53,10 +53,11 @@ METRIC = "Ginteractions/s Hermite-4 N=128K, mixed vs FP64 GPU at rel. force err 
 TRAFFIC_PROFILE = os.path.join(ROOT, "profiles", "force_h4_mixed_traffic.md")
 DRIVER = os.path.join(ROOT, "sapporo2_amd", "bench", "g6_blocksteps")
 FLOP_PER_INTERACTION = 60.0          # test_gravity_block.cpp:271
-# Algorithmic bytes of the HBM-bound kernels (Hermite-4).  Predictor, per j-particle: reads
+# Algorithmic bytes of the HBM-bound kernels (Hermite-4).  Predictor (its launch also applies
+# the updates and copies the call's inputs from host memory), per j-particle: reads
 # t, m, x, v, a, j (14 doubles) and the id; writes the working-precision record (48 B mixed,
 # 64 B FP64) and, mixed only, the FP64 predicted position and velocity kept for read-back.
-# Scatter, per staged update followed by a prediction in the same call: reads the staged row
+# Scatter (a launch of its own only where updates change ids), per staged update: reads the row
 # (16 doubles and the address/id pair), writes the 16 raw fields and the id.
 PREDICT_BYTES = {"mixed": 116 + 48 + 48, "fp64": 116 + 64}
 SCATTER_BYTES = 136 + 128 + 4

@@ -125,14 +125,15 @@ int sapamd_retrieve_predicted_j_particles(sapamd_engine *e, int n, const int *ad
 int sapamd_graph_count(sapamd_engine *e);
 float sapamd_last_force_ms(sapamd_engine *e);
 float sapamd_last_predict_ms(sapamd_engine *e);
-/* j-update scatter kernel time of the last call (timing on; 0 when the call had
- * no updates) and, in *nupd (may be NULL), the number of updates it applied */
+/* time of the launch that applied the last call's j-updates (timing on) and, in
+ * *nupd (may be NULL), their number; 0 when the call had none or applied them in
+ * the predictor's launch (updates that change no id) */
 float sapamd_last_scatter_ms(sapamd_engine *e, int *nupd);
 /* finalize kernel time of the last call (timing on): reduction of the partial
  * sums, list sort, and the result and list writes into host memory */
 float sapamd_last_finalize_ms(sapamd_engine *e);
-/* device time of the last force call from the first kernel after its input
- * copies to the end of the finalize kernel (copies excluded) */
+/* device time of the last force call from its first kernel to the end of the
+ * finalize kernel */
 float sapamd_last_device_ms(sapamd_engine *e);
 int sapamd_last_config(sapamd_engine *e, int *P, int *S, int *jchunk);
 /* Launch-shape table (sapporo2_amd/autotune.py output; loaded at open from

@@ -8,6 +8,7 @@
 #include <algorithm>
 #include <atomic>
 #include <chrono>
+#include <climits>
 #include <cmath>
 #include <condition_variable>
 #include <cstdio>
@@ -38,6 +39,7 @@ constexpr int IBUF_FIELDS = 10;  // xi 3, vi 3, ai 3, h2 1
 // Staged j-update rows are copied to the device as soon as this many are
 // pending, while the caller is still staging (the copy overlaps its loop).
 constexpr int EARLY_FLUSH_ROWS = 4096;
+constexpr int BATCH_ROWS = 16384;  // rows a batch stages at a time
 // Upload block of a single-system call, one host->device copy: the call
 // descriptor, then the i ids, then the i doubles.  The ids region is sized by
 // the power-of-two bucket of ni, so every offset depends on the bucket only
@@ -70,10 +72,10 @@ bool host_coherent() {
   return v ? atoi(v) != 0 : true;
 }
 template <typename T>
-hipError_t hmap(T** h, T** d, size_t n) {
+hipError_t hmap(T** h, T** d, size_t n, bool coherent) {
   *h = *d = nullptr;
   if (n == 0) n = 1;
-  const unsigned flags = hipHostMallocMapped | (host_coherent() ? hipHostMallocCoherent : hipHostMallocNonCoherent);
+  const unsigned flags = hipHostMallocMapped | (coherent ? hipHostMallocCoherent : hipHostMallocNonCoherent);
   const hipError_t e = hipHostMalloc(reinterpret_cast<void**>(h), n * sizeof(T), flags);
   if (e != hipSuccess) return e;
   return hipHostGetDevicePointer(reinterpret_cast<void**>(d), *h, 0);
@@ -151,7 +153,7 @@ int Engine::open(int device, int order, int precision) {
   for (auto& s : stage_) HIPCHK(hipEventCreateWithFlags(&s.ev, hipEventDisableTiming), "hipEventCreate");
   HIPCHK(hipEventCreateWithFlags(&ev_desc_, hipEventDisableTiming), "hipEventCreate");
   HIPCHK(dmalloc(&pack_ctr_d_, 1), "pack counter");
-  HIPCHK(hmalloc(&call_h_, CALL_DOUBLES), "pinned call block");
+  HIPCHK(hmap(&call_h_, &call_hd_, CALL_DOUBLES, true), "pinned call block");
   HIPCHK(dmalloc(&call_d_, CALL_DOUBLES), "call block");
   desc_h_ = reinterpret_cast<CallDesc*>(call_h_);
   desc_d_ = reinterpret_cast<CallDesc*>(call_d_);
@@ -165,8 +167,8 @@ int Engine::open(int device, int order, int precision) {
 
   nj_max_ = NJ_INITIAL;
   max_addr_ = -1;
-  slot_of_.assign(nj_max_, -1);
-  staged_addr_.clear();
+  addr_.assign(nj_max_, AddrState{});
+  new_ids_ = false;
   nstaged_ = 0;
   cur_ = 0;
   predict_ = false;
@@ -184,7 +186,7 @@ int Engine::close() {
   (void)hipSetDevice(device_);
   (void)hipStreamSynchronize(stream_);
   drop_graphs();
-  hfree(call_h_); dfree(call_d_);
+  hfree(call_h_); dfree(call_d_); call_hd_ = nullptr;
   desc_h_ = nullptr; desc_d_ = nullptr;
   if (ev_desc_) (void)hipEventDestroy(ev_desc_);
   ev_desc_ = nullptr;
@@ -192,7 +194,9 @@ int Engine::close() {
   dfree(st_.raw); dfree(st_.id); dfree(st_.rec); dfree(st_.ppos); dfree(st_.pvel); dfree(st_.pacc); dfree(st_.idr);
   st_.cap = 0;
   for (auto& s : stage_) {
-    hfree(s.d); s.cap = 0; s.busy = false;
+    hfree(s.d); s.dd = nullptr; s.cap = 0; s.busy = s.by_call = false;
+    hfree(s.bits); s.bits_d = nullptr; s.words = 0;
+    s.addr.clear();
     if (s.ev) (void)hipEventDestroy(s.ev);
     s.ev = nullptr;
   }
@@ -217,8 +221,7 @@ int Engine::close() {
   if (stream_) (void)hipStreamDestroy(stream_);
   stream_ = nullptr;
   open_ = inflight_ = have_results_ = ngb_fetched_ = jhost_valid_ = false;
-  slot_of_.clear();
-  staged_addr_.clear();
+  addr_.clear();
   nstaged_ = 0;
   return 0;
 }
@@ -289,15 +292,44 @@ int Engine::grow_staging(int need) {
   const int nr = raw_fields(order_) + 1;  // row: fields, then the (address, id) pair
   for (auto& s : stage_) {
     if (s.cap >= need) continue;
-    if (s.busy && s.seq > done_seq_) HIPCHK(hipEventSynchronize(s.ev), "staging wait");
-    s.busy = false;
+    if (wait_stage(s) != 0) return -1;
     const int nc = std::max(need, s.cap * 2);
-    double* d = nullptr;
-    HIPCHK(hmalloc(&d, (size_t)nc * nr), "pinned staging");
+    double *d = nullptr, *dd = nullptr;
+    HIPCHK(hmap(&d, &dd, (size_t)nc * nr, true), "pinned staging");
     if (s.cap > 0 && &s == &stage_[cur_] && nstaged_ > 0) memcpy(d, s.d, sizeof(double) * (size_t)nstaged_ * nr);
     hfree(s.d);
     s.d = d;
+    s.dd = dd;
     s.cap = nc;
+  }
+  return ensure_bits(nj_max_);
+}
+
+// Waits until the device has read what the stage last handed over.
+int Engine::wait_stage(Stage& s) {
+  if (s.busy && s.seq > done_seq_) {
+    if (!s.by_call) HIPCHK(hipEventSynchronize(s.ev), "staging wait");
+    else if (inflight_ && wait_results() != 0) return -1;
+  }
+  s.busy = false;
+  return 0;
+}
+
+// Address bit sets of both stages for at least `need` addresses.
+int Engine::ensure_bits(int need) {
+  const size_t nw = ((size_t)need + 63) / 64 * 2;  // whole 64-address tiles
+  for (auto& s : stage_) {
+    if (s.words >= nw) continue;
+    if (wait_stage(s) != 0) return -1;
+    const size_t nc = std::max(nw, s.words + s.words / 2);
+    unsigned *b = nullptr, *bd = nullptr;
+    HIPCHK(hmap(&b, &bd, nc, true), "pinned update bits");
+    if (s.words) memcpy(b, s.bits, s.words * sizeof(unsigned));
+    memset(b + s.words, 0, (nc - s.words) * sizeof(unsigned));
+    hfree(s.bits);
+    s.bits = b;
+    s.bits_d = bd;
+    s.words = nc;
   }
   return 0;
 }
@@ -315,13 +347,43 @@ int Engine::set_no_time() {
   return 0;
 }
 
-// Reference set_j_particle (sapporohostclass.cpp:434-558): stage the update;
-// re-setting an address before the next flush overwrites its slot; the
-// logical capacity grows by 10% and addresses beyond that are rejected.
-int Engine::set_j_particle(int addr, int id, double tj, double dtj, double mass, const double a[3],
-                           const double jrk[3], const double v[3], const double x[3],
-                           const double snp[3], const double crk[3], double eps) {
-  if (!open_) return fail("set_j_particle: library not open");
+namespace {
+// Row of one update: the raw fields in RawField order, then (address, id).
+inline void fill_row(double* u, int order, int addr, int id, double tj, double dtj, double mass, const double* a,
+                     const double* jrk, const double* v, const double* x, const double* snp, const double* crk,
+                     double eps) {
+  u[RF_T] = tj; u[RF_DT] = dtj; u[RF_M] = mass; u[RF_EPS] = eps;
+  for (int d = 0; d < 3; ++d) {
+    u[RF_X + d] = x ? x[d] : 0.0;
+    u[RF_VX + d] = v ? v[d] : 0.0;
+    u[RF_AX + d] = a ? a[d] : 0.0;
+    u[RF_JX + d] = jrk ? jrk[d] : 0.0;
+    if (order >= ORDER_H6) {
+      u[RF_SX + d] = snp ? snp[d] : 0.0;
+      u[RF_CX + d] = crk ? crk[d] : 0.0;
+    }
+  }
+  const int pair[2] = {addr, id};
+  memcpy(u + raw_fields(order), pair, sizeof(pair));
+}
+}  // namespace
+
+// Makes the current stage ready for its first row: a stage still read by an
+// earlier flush is waited for; copies of this flush's own rows (early flushes)
+// need no wait, since a rewritten row is copied again behind them.
+int Engine::open_stage() {
+  if (nstaged_ != 0) return 0;
+  Stage& sg = stage_[cur_];
+  if (sg.busy && wait_stage(sg) != 0) return -1;
+  par_for(sg.addr.size(), [&](size_t b, size_t e) {
+    for (size_t k = b; k < e; ++k) __atomic_store_n(&sg.bits[sg.addr[k] >> 5], 0u, __ATOMIC_RELAXED);
+  });
+  sg.addr.clear();
+  return 0;
+}
+
+// Capacity for an address beyond the host maps.
+int Engine::admit(int addr) {
   if (addr < 0) return fail("set_j_particle: negative address");
   if (addr >= nj_max_) {
     fprintf(stderr, "sapporo2_amd: increasing nj_max from %d for address %d\n", nj_max_, addr);
@@ -332,46 +394,55 @@ int Engine::set_j_particle(int addr, int id, double tj, double dtj, double mass,
       return fail("set_j_particle: address out of order");
     }
   }
-  if ((int)slot_of_.size() < nj_max_) slot_of_.resize(nj_max_, -1);
+  return grow_maps();
+}
+
+// Row of the current stage for an update of addr (-1 on error); the caller
+// fills it.
+inline int Engine::stage_row(int addr, int id) {
+  if ((unsigned)addr >= addr_.size() && admit(addr) != 0) return -1;
+  if (nstaged_ == 0 && open_stage() != 0) return -1;
   Stage* sg = &stage_[cur_];
-  // a stage still read by the copy of an earlier flush is waited for before its
-  // first row is rewritten; copies of this flush's own rows (early flushes)
-  // need no wait: a rewritten row is copied again behind them
-  if (nstaged_ == 0 && sg->busy) {
-    if (sg->seq > done_seq_) HIPCHK(hipEventSynchronize(sg->ev), "staging wait");
-    sg->busy = false;
-  }
-  int k = slot_of_[addr];
+  AddrState& as = addr_[addr];
+  int k = as.slot;
+  new_ids_ |= k == SLOT_NEW || as.id != id;
+  as.id = id;
   if (k < 0) {
     if (nstaged_ >= sg->cap) {
       if (grow_staging(nstaged_ + 1) != 0) return -1;
       sg = &stage_[cur_];
     }
     k = nstaged_++;
-    slot_of_[addr] = k;
-    staged_addr_.push_back(addr);
+    as.slot = k;
+    sg->addr.push_back(addr);
+    sg->bits[addr >> 5] |= 1u << (addr & 31);
   } else if (k < flushed_) {
     flushed_ = k;  // already copied: copy again from this row
   }
-  const int nf = raw_fields(order_);
-  double* u = sg->d + (size_t)k * (nf + 1);
-  u[RF_T] = tj; u[RF_DT] = dtj; u[RF_M] = mass; u[RF_EPS] = eps;
-  for (int d = 0; d < 3; ++d) {
-    u[RF_X + d] = x ? x[d] : 0.0;
-    u[RF_VX + d] = v ? v[d] : 0.0;
-    u[RF_AX + d] = a ? a[d] : 0.0;
-    u[RF_JX + d] = jrk ? jrk[d] : 0.0;
-    if (order_ >= ORDER_H6) {
-      u[RF_SX + d] = snp ? snp[d] : 0.0;
-      u[RF_CX + d] = crk ? crk[d] : 0.0;
-    }
-  }
-  const int pair[2] = {addr, id};
-  memcpy(u + nf, pair, sizeof(pair));
   if (addr > max_addr_) max_addr_ = addr;
   jhost_valid_ = false;
+  return k;
+}
+
+// Reference set_j_particle (sapporohostclass.cpp:434-558): stage the update;
+// re-setting an address before the next flush overwrites its slot; the
+// logical capacity grows by 10% and addresses beyond that are rejected.
+int Engine::set_j_particle(int addr, int id, double tj, double dtj, double mass, const double a[3],
+                           const double jrk[3], const double v[3], const double x[3],
+                           const double snp[3], const double crk[3], double eps) {
+  if (!open_) return fail("set_j_particle: library not open");
+  const int k = stage_row(addr, id);
+  if (k < 0) return -1;
+  fill_row(stage_[cur_].d + (size_t)k * (raw_fields(order_) + 1), order_, addr, id, tj, dtj, mass, a, jrk, v, x, snp,
+           crk, eps);
   if (nstaged_ - flushed_ >= EARLY_FLUSH_ROWS) return copy_staged();
   return 0;
+}
+
+// The per-address host maps for the logical capacity nj_max_.
+int Engine::grow_maps() {
+  addr_.resize(nj_max_);
+  return ensure_bits(nj_max_);
 }
 
 // Copies the staged rows [flushed_, nstaged_) of the current stage to the
@@ -396,6 +467,7 @@ int Engine::copy_staged() {
                         stream_), "update upload");
   HIPCHK(hipEventRecord(sg.ev, stream_), "event");
   sg.busy = true;
+  sg.by_call = false;
   sg.seq = ++rec_seq_;
   flushed_ = n;
   return 0;
@@ -407,34 +479,173 @@ int Engine::set_j_particles(int n, const int* addr, const int* id, const double*
   if (n < 0 || !addr || !id || !mass || !x) return fail("set_j_particles: bad arguments");
   if (!open_) return fail("set_j_particles: library not open");
   // the batch names all its addresses up front: grow the logical capacity once
-  int amax = -1;
-  for (int k = 0; k < n; ++k) amax = addr[k] > amax ? addr[k] : amax;
-  if (amax >= nj_max_) nj_max_ = amax + 1;
+  int amax = -1, amin = 0;
   for (int k = 0; k < n; ++k) {
-    const size_t o = 3 * (size_t)k;
-    const int rc = set_j_particle(addr[k], id[k], tj ? tj[k] : 0.0, dtj ? dtj[k] : 0.0, mass[k],
-                                  a ? a + o : nullptr, jrk ? jrk + o : nullptr, v ? v + o : nullptr, x + o,
-                                  snp ? snp + o : nullptr, crk ? crk + o : nullptr, eps ? eps[k] : 0.0);
-    if (rc != 0) return rc;
+    amax = std::max(amax, addr[k]);
+    amin = std::min(amin, addr[k]);
+  }
+  if (amax >= nj_max_) nj_max_ = amax + 1;
+  if ((int)addr_.size() < nj_max_ && grow_maps() != 0) return -1;
+  // On the host threads a block at a time: a block's copy is under way while the
+  // next one is staged.
+  for (int b = 0; b < n; b += BATCH_ROWS) {
+    const int e = std::min(n, b + BATCH_ROWS);
+    auto row = [&](int r, int k) {
+      const size_t o = 3 * (size_t)k;
+      fill_row(stage_[cur_].d + (size_t)r * (raw_fields(order_) + 1), order_, addr[k], id[k], tj ? tj[k] : 0.0,
+               dtj ? dtj[k] : 0.0, mass[k], a ? a + o : nullptr, jrk ? jrk + o : nullptr, v ? v + o : nullptr, x + o,
+               snp ? snp + o : nullptr, crk ? crk + o : nullptr, eps ? eps[k] : 0.0);
+    };
+    if (amin >= 0 && e - b >= (int)(2 * HOST_CHUNK)) {
+      const int rc = stage_block(e - b, addr + b, id + b, [&](int r, int k) { row(r, b + k); });
+      if (rc < 0) return -1;
+      if (rc > 0) continue;
+    }
+    for (int k = b; k < e; ++k) {
+      const int r = stage_row(addr[k], id[k]);
+      if (r < 0) return -1;
+      row(r, k);
+      if (nstaged_ - flushed_ >= EARLY_FLUSH_ROWS && copy_staged() != 0) return -1;
+    }
   }
   return 0;
 }
 
+// Stages n updates of distinct addresses, none of them staged yet, on the host
+// threads: update k takes row nstaged_ + k, filled by fill(row, k).  Returns 1
+// when done, 0 with nothing staged when an address was met twice (the caller
+// stages them in order: the last values win), -1 on error.
+template <typename F>
+int Engine::stage_block(int n, const int* addr, const int* id, const F& fill) {
+  if (open_stage() != 0) return -1;
+  if (nstaged_ + n > stage_[cur_].cap && grow_staging(nstaged_ + n) != 0) return -1;
+  Stage& sg = stage_[cur_];
+  const int base = nstaged_;
+  sg.addr.resize((size_t)base + n);
+  AddrState* as = addr_.data();
+  std::atomic<bool> again{false}, changed{false};
+  std::atomic<int> top{max_addr_};
+  par_for((size_t)n, [&](size_t b, size_t e) {
+    bool met = false, ch = false;
+    int mx = -1;
+    for (size_t k = b; k < e; ++k) {
+      const int ad = addr[k], was = __atomic_load_n(&as[ad].slot, __ATOMIC_RELAXED);
+      met |= was >= 0;
+      ch |= was == SLOT_NEW || __atomic_load_n(&as[ad].id, __ATOMIC_RELAXED) != id[k];
+      if (was < 0) __atomic_store_n(&as[ad].slot, base + (int)k, __ATOMIC_RELAXED);
+      __atomic_store_n(&as[ad].id, id[k], __ATOMIC_RELAXED);
+      __atomic_fetch_or(&sg.bits[ad >> 5], 1u << (ad & 31), __ATOMIC_RELAXED);
+      sg.addr[(size_t)base + k] = ad;
+      mx = std::max(mx, ad);
+    }
+    if (met) again.store(true, std::memory_order_relaxed);
+    if (ch) changed.store(true, std::memory_order_relaxed);
+    for (int t = top.load(); t < mx && !top.compare_exchange_weak(t, mx);) {}
+  });
+  if (!again.load())
+    par_for((size_t)n, [&](size_t b, size_t e) {
+      bool met = false;
+      for (size_t k = b; k < e; ++k) {
+        met |= as[addr[k]].slot != base + (int)k;  // two updates of one address wrote its slot
+        fill(base + (int)k, (int)k);
+      }
+      if (met) again.store(true, std::memory_order_relaxed);
+    });
+  if (again.load()) {
+    for (int k = 0; k < n; ++k)
+      if (as[addr[k]].slot >= base) as[addr[k]].slot = SLOT_NONE;
+    sg.addr.resize((size_t)base);
+    new_ids_ = true;  // the ids before this block are overwritten
+    return 0;
+  }
+  nstaged_ = base + n;
+  new_ids_ |= changed.load();
+  max_addr_ = top.load();
+  jhost_valid_ = false;
+  if (nstaged_ - flushed_ >= EARLY_FLUSH_ROWS && copy_staged() != 0) return -1;
+  return 1;
+}
+
 // Reference send_j_particles_to_device + copyJInDev (sapporohostclass.cpp:889-923,
-// 1204-1248), fused with the neighbour-counter reset of dev_reset_buffers.
-// upload_updates issues the host->device copy of the staged updates; the
-// scatter kernel is launched separately so callers can bracket device work.
+// 1204-1248).  upload_updates issues the host->device copy of the staged
+// updates for a captured call, whose scatter kernel applies them; every other
+// path hands them to k_prep.
 int Engine::upload_updates(int* nupd) {
   const int n = nstaged_;
   *nupd = n;
   if (n <= 0) return 0;
   if (ensure_store(max_addr_ + 1) != 0) return -1;
   if (copy_staged() != 0) return -1;
-  for (const int a : staged_addr_) slot_of_[a] = -1;
-  staged_addr_.clear();
+  hand_over();
+  return 0;
+}
+
+// The staged rows are the device's from here on; staging goes on in the other
+// stage.
+void Engine::hand_over() {
+  const std::vector<int>& staged = stage_[cur_].addr;
+  par_for(staged.size(), [&](size_t b, size_t e) {
+    for (size_t k = b; k < e; ++k) addr_[staged[k]].slot = SLOT_NONE;
+  });
   nstaged_ = 0;
   flushed_ = 0;
+  new_ids_ = false;
   cur_ ^= 1;
+}
+
+// Staged updates, prediction of [0, pred_j1) and, for a force call, its call
+// block and counter reset (k_prep).  by_call: the caller records the call's
+// completion next, and the stage is free with it.
+int Engine::prep(int pred_j1, int call_bytes, int ni_reset, bool by_call) {
+  const int n = nstaged_;
+  if (n > 0 && ensure_store(max_addr_ + 1) != 0) return -1;
+  Stage& sg = stage_[cur_];
+  PrepArgs a{};
+  a.st = st_;
+  a.rows_d = upd_d_;
+  a.rows_h = sg.dd;
+  a.nd = flushed_;
+  a.nupd = n;
+  if (n > 0 && pred_j1 > 0) {
+    a.bits = sg.bits_d;
+    a.nbits = (int)std::min<size_t>(sg.words * 32, INT_MAX);
+  }
+  a.new_ids = new_ids_ ? 1 : 0;
+  a.ti = t_i_;
+  a.pred_j1 = pred_j1;
+  a.call_h = reinterpret_cast<const int4*>(call_hd_);
+  a.call_d = reinterpret_cast<int4*>(call_d_);
+  a.call_n16 = (call_bytes + 15) / 16;
+  a.ngb_cnt = cnt_d_;
+  a.ni_reset = ni_reset;
+  a.pack_ctr = pack_ctr_d_;
+  const bool ev = timing_;
+  timed_scatter_ = timed_predict_ = false;
+  if (n > 0 && pred_j1 > 0 && new_ids_) {
+    // ids change: the tile id ranges are rebuilt from the updated store
+    PrepArgs u = a;
+    u.pred_j1 = u.nbits = 0;
+    if (ev) HIPCHK(hipEventRecord(ev_s0_, stream_), "event");
+    if (launch_prep(stream_, order_, f64_, u) != 0) return fail("update launch", hipGetLastError());
+    if (ev) HIPCHK(hipEventRecord(ev_s1_, stream_), "event");
+    timed_scatter_ = ev;
+    last_nupd_ = n;
+    a.nupd = a.call_n16 = a.ni_reset = a.nbits = 0;
+  }
+  if (ev) HIPCHK(hipEventRecord(ev_p0_, stream_), "event");
+  if (launch_prep(stream_, order_, f64_, a) != 0) return fail("prep launch", hipGetLastError());
+  if (ev) HIPCHK(hipEventRecord(ev_p1_, stream_), "event");
+  timed_predict_ = ev && pred_j1 > 0;
+  if (n > 0) {
+    if (!by_call) {
+      HIPCHK(hipEventRecord(sg.ev, stream_), "event");
+      ++rec_seq_;
+    }
+    sg.busy = true;
+    sg.by_call = by_call;
+    sg.seq = by_call ? rec_seq_ + 1 : rec_seq_;  // the call's completion is the next event recorded
+    hand_over();
+  }
   return 0;
 }
 
@@ -448,44 +659,7 @@ int Engine::scatter_blocks(int n, int ni_reset) const {
   return nb;
 }
 
-int Engine::scatter_updates(int n, int ni_reset, int pred_j1) {
-  ScatterArgs a{};
-  a.st = st_;
-  a.upd = upd_d_;
-  a.nf = raw_fields(order_);
-  a.ngb_cnt = cnt_d_;
-  a.pack_ctr = pack_ctr_d_;
-  a.cd = desc_d_;
-  a.grid_blocks = scatter_blocks(n, ni_reset);
-  a.pred_j1 = pred_j1;
-  if (a.grid_blocks == 0) return 0;
-  if (launch_scatter(stream_, order_, f64_, a) != 0) return fail("scatter launch", hipGetLastError());
-  return 0;
-}
-
-// Writes the call descriptor (pinned host copy) and queues its upload.  The
-// previous upload has to have read the host copy before it is rewritten.
-int Engine::post_desc(int ni, int nupd, int ni_reset, double eps2) {
-  if (desc_pending_ && desc_seq_ > done_seq_) HIPCHK(hipEventSynchronize(ev_desc_), "descriptor wait");
-  desc_h_->ti = t_i_;
-  desc_h_->eps2 = eps2;
-  desc_h_->ni = ni;
-  desc_h_->nupd = nupd;
-  desc_h_->ni_reset = ni_reset;
-  desc_h_->pad = 0;
-  HIPCHK(hipMemcpyAsync(desc_d_, desc_h_, sizeof(CallDesc), hipMemcpyHostToDevice, stream_), "descriptor upload");
-  HIPCHK(hipEventRecord(ev_desc_, stream_), "event");
-  desc_pending_ = true;
-  desc_seq_ = ++rec_seq_;
-  return 0;
-}
-
-int Engine::flush_updates(int ni_reset, int pred_j1) {
-  int n = 0;
-  if (upload_updates(&n) != 0) return -1;
-  if (post_desc(0, n, ni_reset, 0.0) != 0) return -1;
-  return scatter_updates(n, ni_reset, pred_j1);
-}
+int Engine::flush_updates() { return prep(0, 0, 0, false); }
 
 int Engine::predict_range(int j0, int j1) {
   if (j1 <= j0) return 0;
@@ -608,9 +782,9 @@ int Engine::ensure_icap(int need) {
   HIPCHK(hmalloc(&iid_h_, nI), "pinned i ids");
   HIPCHK(dmalloc(&ibuf_d_, IBUF_FIELDS * nI), "i buffer");
   HIPCHK(dmalloc(&iid_d_, nI), "i ids");
-  HIPCHK(hmap(&res_h_, &res_hd_, nI * out_fields(order_)), "host-mapped results");
+  HIPCHK(hmap(&res_h_, &res_hd_, nI * out_fields(order_), host_coherent()), "host-mapped results");
   res_stride_ = (long)nI;
-  HIPCHK(hmap(&loff_h_, &loff_hd_, nI), "host-mapped list offsets");
+  HIPCHK(hmap(&loff_h_, &loff_hd_, nI, host_coherent()), "host-mapped list offsets");
   HIPCHK(dmalloc(&cnt_d_, nI), "neighbour counts");
   HIPCHK(dmalloc(&idesc_d_, nI), "ensemble i descriptors");
   HIPCHK(hipMemsetAsync(cnt_d_, 0, nI * sizeof(int), stream_), "memset");
@@ -640,7 +814,7 @@ int Engine::ensure_packed(long need) {
   if (stream_) HIPCHK(hipStreamSynchronize(stream_), "packed-list grow sync");
   inflight_ = false;
   hfree(packed_h_);
-  HIPCHK(hmap(&packed_h_, &packed_hd_, (size_t)need), "host-mapped packed lists");
+  HIPCHK(hmap(&packed_h_, &packed_hd_, (size_t)need, host_coherent()), "host-mapped packed lists");
   packed_cap_ = need;
   have_results_ = false;
   ++gen_;
@@ -685,7 +859,7 @@ int Engine::set_clusters(int n, const int* njc) {
     if (off > (1L << 30)) return fail("set_clusters: too many particles");
   }
   nj_max_ = std::max(nj_max_, (int)off);
-  if ((int)slot_of_.size() < nj_max_) slot_of_.resize(nj_max_, -1);
+  if ((int)addr_.size() < nj_max_ && grow_maps() != 0) return -1;
   if (ensure_store((int)off) != 0) return -1;
   cl_total_ = (int)off;
   return 0;
@@ -904,16 +1078,11 @@ int Engine::start_grav_calc_clusters(int ni, const int* cluster, const int* id, 
   if (launch_ens_idesc(stream_, reinterpret_cast<const EnsGroup*>(ens_tab_d_ + o_grp), ng, ni, idesc_d_) != 0)
     return fail("ensemble descriptor launch", hipGetLastError());
 
-  int nupd = 0;
-  if (upload_updates(&nupd) != 0) return -1;
-  if (post_desc(ni, nupd, ngb_on ? ni : 0, 0.0) != 0) return -1;
+  if (desc_pending_ && desc_seq_ > done_seq_) HIPCHK(hipEventSynchronize(ev_desc_), "descriptor wait");
+  desc_pending_ = false;
+  *desc_h_ = CallDesc{t_i_, 0.0, ni, 0, 0, 0};
   if (timing_) HIPCHK(hipEventRecord(ev_d0_, stream_), "event");
-  if (scatter_updates(nupd, ngb_on ? ni : 0, predict_ ? cl_total_ : 0) != 0) return -1;
-  if (predict_) {
-    if (predict_range(0, cl_total_) != 0) return -1;
-  } else {
-    timed_predict_ = false;
-  }
+  if (prep(predict_ ? cl_total_ : 0, (int)sizeof(CallDesc), ngb_on ? ni : 0, true) != 0) return -1;
   predict_ = false;
   if (ensure_partials((size_t)nitems * 64) != 0) return -1;
   EnsArgs ea{};
@@ -992,9 +1161,12 @@ int Engine::start_grav_calc(int nj, int ni, const int* id, const double (*xi)[3]
     if (ensure_packed((long)NPIPES * NGB_CAP) != 0) return -1;
   }
 
-  int nupd = 0;
-  if (upload_updates(&nupd) != 0) return -1;
-  // descriptor, ids and doubles in one copy
+  // Direct calls take the staged rows and the call block (descriptor, ids and
+  // doubles) from pinned memory in k_prep; a captured graph holds its
+  // arguments, so replayed calls upload both with copy commands and read the
+  // call's values from the descriptor.
+  int nupd = graphs_ ? 0 : nstaged_;
+  if (graphs_ && upload_updates(&nupd) != 0) return -1;
   desc_h_->ti = t_i_;
   desc_h_->eps2 = eps2;
   desc_h_->ni = ni;
@@ -1002,10 +1174,12 @@ int Engine::start_grav_calc(int nj, int ni, const int* id, const double (*xi)[3]
   desc_h_->ni_reset = ngb_on ? ni : 0;
   desc_h_->pad = 0;
   const size_t nbytes = (size_t)((char*)(bx + nd) - (char*)call_h_);
-  HIPCHK(hipMemcpyAsync(call_d_, call_h_, nbytes, hipMemcpyHostToDevice, stream_), "call upload");
-  HIPCHK(hipEventRecord(ev_desc_, stream_), "event");
-  desc_pending_ = true;
-  desc_seq_ = ++rec_seq_;
+  if (graphs_) {
+    HIPCHK(hipMemcpyAsync(call_d_, call_h_, nbytes, hipMemcpyHostToDevice, stream_), "call upload");
+    HIPCHK(hipEventRecord(ev_desc_, stream_), "event");
+    desc_pending_ = true;
+    desc_seq_ = ++rec_seq_;
+  }
   const bool predict = predict_;
   predict_ = false;  // reference 698
   const ForceConfig cfg = choose_config(ni, nj, ngb_on);
@@ -1014,15 +1188,15 @@ int Engine::start_grav_calc(int nj, int ni, const int* id, const double (*xi)[3]
   // finalize shape follows the bucket in both cases, so results agree.
   const int grid_ni = graphs_ ? std::min(bucket, NPIPES) : ni;
   if (ensure_partials((size_t)cfg.S * grid_ni) != 0) return -1;
-  const int sblocks = scatter_blocks(nupd, ngb_on ? ni : 0);
-  // device window: everything after the host->device copies
+  // device window: all device work (after the host->device copies of a replayed call)
   if (timing_) HIPCHK(hipEventRecord(ev_d0_, stream_), "event");
   if (graphs_) {
+    const int sblocks = scatter_blocks(nupd, ngb_on ? ni : 0);
     if (launch_call_graph(grid_ni, nj, cfg, ngb_on, predict, sblocks, bucket >= 1024) != 0) return -1;
     timed_predict_ = timed_force_ = false;
   } else {
-    if (enqueue_call(grid_ni, nj, cfg, ngb_on, predict, sblocks, bucket >= 1024) != 0) return -1;
-    if (!predict) timed_predict_ = false;
+    if (prep(predict ? nj : 0, (int)nbytes, ngb_on ? ni : 0, true) != 0) return -1;
+    if (enqueue_force(grid_ni, nj, cfg, ngb_on, bucket >= 1024) != 0) return -1;
     timed_force_ = timing_;
   }
   if (timing_) HIPCHK(hipEventRecord(ev_d1_, stream_), "event");
@@ -1041,31 +1215,30 @@ int Engine::start_grav_calc(int nj, int ni, const int* id, const double (*xi)[3]
   return 0;
 }
 
-// The device work of one force call: [scatter] -> [predict] -> force ->
+// The device work of a captured force call: [scatter] -> [predict] -> force ->
 // finalize.  Every per-call value comes from the descriptor, so the sequence
-// depends only on its arguments here (the key of a captured graph).
+// depends only on its arguments here (the key of the graph).
 int Engine::enqueue_call(int grid_ni, int nj, const ForceConfig& cfg, bool ngb_on, bool predict, int sblocks,
                          bool rows) {
   if (sblocks > 0) {
     ScatterArgs a{};
     a.st = st_;
     a.upd = upd_d_;
-      a.nf = raw_fields(order_);
+    a.nf = raw_fields(order_);
     a.ngb_cnt = cnt_d_;
     a.pack_ctr = pack_ctr_d_;
     a.cd = desc_d_;
     a.grid_blocks = sblocks;
     a.pred_j1 = predict ? nj : 0;
-    const bool ev = timing_ && !capturing_;
-    if (ev) HIPCHK(hipEventRecord(ev_s0_, stream_), "event");
     if (launch_scatter(stream_, order_, f64_, a) != 0) return fail("scatter launch", hipGetLastError());
-    if (ev) HIPCHK(hipEventRecord(ev_s1_, stream_), "event");
-    timed_scatter_ = ev;
-    last_nupd_ = desc_h_->nupd;
-  } else {
-    timed_scatter_ = false;
   }
+  timed_scatter_ = false;
   if (predict && predict_range(0, nj) != 0) return -1;
+  return enqueue_force(grid_ni, nj, cfg, ngb_on, rows);
+}
+
+// Force and finalize kernels of a call.
+int Engine::enqueue_force(int grid_ni, int nj, const ForceConfig& cfg, bool ngb_on, bool rows) {
   ForceArgs fa{};
   fa.rec = st_.rec;
   fa.idr = st_.idr;
@@ -1388,10 +1561,8 @@ int Engine::force_prediction(int nj) {
   if (!open_) return fail("force_prediction: library not open");
   HIPCHK(hipSetDevice(device_), "hipSetDevice");
   if (inflight_ && wait_results() != 0) return -1;
-  if (flush_updates(0, predict_ ? std::max(nj, 0) : 0) != 0) return -1;
-  if (predict_ && nj > 0) {
-    if (predict_range(0, nj) != 0) return -1;
-  }
+  const int pred_j1 = predict_ ? std::max(nj, 0) : 0;
+  if (ensure_store(pred_j1) != 0 || prep(pred_j1, 0, 0, false) != 0) return -1;
   predict_ = false;
   jhost_valid_ = false;
   return 0;
@@ -1402,7 +1573,7 @@ int Engine::fetch_j_host(int need) {
   if (jhost_valid_ && need <= jhost_n_) return 0;
   HIPCHK(hipSetDevice(device_), "hipSetDevice");
   if (inflight_ && wait_results() != 0) return -1;
-  if (flush_updates(0) != 0) return -1;
+  if (flush_updates() != 0) return -1;
   const int n = std::max(need, max_addr_ + 1);
   if (n <= 0) return 0;
   if (ensure_store(n) != 0) return -1;
@@ -1442,7 +1613,7 @@ int Engine::retrieve_predicted_j_particles(int n, const int* addr, double* mass,
   if (n == 0) return 0;
   HIPCHK(hipSetDevice(device_), "hipSetDevice");
   if (inflight_ && wait_results() != 0) return -1;
-  if (flush_updates(0) != 0) return -1;
+  if (flush_updates() != 0) return -1;
   for (int k = 0; k < n; ++k)
     if (addr[k] < 0 || addr[k] > max_addr_) return fail("retrieve_predicted_j_particles: address never set");
   if (gather_cap_ < (size_t)n) {
@@ -1511,7 +1682,7 @@ long long Engine::state_bytes() {
   if (!open_) return fail("state_bytes: library not open");
   HIPCHK(hipSetDevice(device_), "hipSetDevice");
   if (inflight_ && wait_results() != 0) return -1;
-  if (flush_updates(0) != 0) return -1;
+  if (flush_updates() != 0) return -1;
   const size_t n = (size_t)std::max(max_addr_ + 1, cl_total_);
   const size_t nfr = raw_fields(order_);
   size_t b = pad8(sizeof(StateHeader)) + pad8(sizeof(int) * cl_n_.size());
@@ -1566,7 +1737,7 @@ int Engine::load_state(const void* buf, long long bytes) {
   if (h.n < 0 || h.ncl < 0 || h.max_addr >= h.n) return fail("load_state: corrupt header");
   HIPCHK(hipSetDevice(device_), "hipSetDevice");
   if (inflight_ && wait_results() != 0) return -1;
-  if (flush_updates(0) != 0) return -1;  // staged updates are superseded by the dump
+  if (flush_updates() != 0) return -1;  // staged updates are superseded by the dump
   const char* p = static_cast<const char*>(buf) + pad8(sizeof(h));
   const size_t n = h.n;
   const size_t nfr = raw_fields(order_);
@@ -1582,7 +1753,8 @@ int Engine::load_state(const void* buf, long long bytes) {
   if (h.ncl && set_clusters(h.ncl, sizes.data()) != 0) return -1;
   if (cl_total_ > h.n) return fail("load_state: corrupt cluster sizes");
   nj_max_ = std::max({h.nj_max, h.max_addr + 1, cl_total_});  // the source's logical capacity
-  if ((int)slot_of_.size() < nj_max_) slot_of_.resize(nj_max_, -1);
+  if ((int)addr_.size() < nj_max_ && grow_maps() != 0) return -1;
+  std::fill(addr_.begin(), addr_.end(), AddrState{});  // the dump's ids are not looked at here
   if (ensure_store(std::max(h.n, 1)) != 0) return -1;
   // clear the whole store: addresses beyond the dump's were never set there
   const size_t cap = st_.cap;

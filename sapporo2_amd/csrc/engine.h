@@ -4,10 +4,10 @@
 // (lib/include/sapporohostclass.h:121-176, lib/src/sapporohostclass.cpp) with
 // the same call sequence and result semantics, re-designed for one MI355X:
 //   * j-particles live in an FP64 field-major store in HBM; updates are staged
-//     in pinned host memory and sent with one asynchronous copy per flush,
-//     then scattered by a kernel (no per-particle map lookups on the device);
-//   * each force call is scatter -> [predict] -> force -> finalize on one HIP
-//     stream; the finalize writes the result rows and the sorted, packed
+//     in pinned host memory, large ones sent ahead with asynchronous copies, and
+//     applied by a kernel (no per-particle map lookups on the device);
+//   * each force call is prep (updates, prediction, inputs) -> force -> finalize
+//     on one HIP stream; the finalize writes the result rows and the sorted, packed
 //     neighbour lists straight into host-mapped pinned memory, so lasthalf and
 //     read_neighbour_list wait for one completion event and copy nothing.  The
 //     kernels take the call's values (block time, softening, counts) from a
@@ -111,10 +111,10 @@ class Engine {
   int graph_count() const { return (int)graph_cache_.size(); }
   float last_force_ms();          // force kernel time of the last call (timing on)
   float last_predict_ms();        // predictor time of the last call (timing on, 0 if none)
-  // scatter (j-update) kernel time of the last call and its update count (timing on, 0 if none)
+  // time of the last call's update launch and its update count (timing on; 0 if none or fused with the prediction)
   float last_scatter_ms(int* nupd);
   float last_finalize_ms();       // finalize (reduction, list sort, host writes) time of the last call (timing on)
-  float last_device_ms();         // scatter..finalize (lists packed) device time of the last call (timing on)
+  float last_device_ms();         // prep..finalize (lists packed) device time of the last call (timing on)
   sapk::ForceConfig last_config() const { return last_cfg_; }
   int device() const { return device_; }
   int num_cus() const { return cus_; }
@@ -123,20 +123,30 @@ class Engine {
   int synchronize();
 
  private:
+  struct Stage;
   int fail(const char* what, hipError_t e = hipSuccess);
   int ensure_store(int need);
   int ensure_partials(size_t entries);
-  int flush_updates(int ni_reset, int pred_j1 = 0);
+  int flush_updates();
   int upload_updates(int* nupd);
   int copy_staged();
-  int scatter_updates(int n, int ni_reset, int pred_j1 = 0);
+  int wait_stage(Stage& s);
+  int ensure_bits(int need);
+  int grow_maps();
+  int admit(int addr);
+  int open_stage();
+  template <typename F>
+  int stage_block(int n, const int* addr, const int* id, const F& fill);
+  int stage_row(int addr, int id);
+  void hand_over();
+  int prep(int pred_j1, int call_bytes, int ni_reset, bool by_call);
   int predict_range(int j0, int j1);
-  int post_desc(int ni, int nupd, int ni_reset, double eps2);
   bool pack_i(int i0, int i1, const int* id, const double (*xi)[3], const double (*vi)[3], const double (*ai)[3],
               const double* h2, double* bx, double* bv, double* ba, double* bh, int* bid);
   int scatter_blocks(int nupd, int ni_reset) const;
   int enqueue_call(int grid_ni, int nj, const sapk::ForceConfig& cfg, bool ngb_on, bool predict,
                    int sblocks, bool rows);
+  int enqueue_force(int grid_ni, int nj, const sapk::ForceConfig& cfg, bool ngb_on, bool rows);
   int launch_call_graph(int grid_ni, int nj, const sapk::ForceConfig& cfg, bool ngb_on, bool predict,
                         int sblocks, bool rows);
   void drop_graphs();
@@ -163,16 +173,26 @@ class Engine {
   // staged updates (pinned), double-buffered
   struct Stage {
     double* d = nullptr;      // cap rows of nf doubles + one (address, id) int pair
+    double* dd = nullptr;     // its device alias
     int cap = 0;
+    // addresses of its rows, in row order, and as a bit set (host-mapped: host
+    // pointer, device alias, words); both are cleared when the stage is reused
+    std::vector<int> addr;
+    unsigned* bits = nullptr; unsigned* bits_d = nullptr; size_t words = 0;
     hipEvent_t ev = nullptr;  // completion of the copy that last read it
     bool busy = false;
+    bool by_call = false;     // read by the last call's prep kernel: free when that call has completed
     uint64_t seq = 0;         // position of ev among the stream's recorded events
   };
   Stage stage_[2];
   int cur_ = 0, nstaged_ = 0;
   int flushed_ = 0;           // staged rows [0, flushed_) already copied to the device (early flush)
-  std::vector<int> slot_of_;  // address -> staged slot or -1
-  std::vector<int> staged_addr_;  // addresses of the staged rows, in row order
+  // per address: its staged row (SLOT_NONE: not staged, SLOT_NEW: nor was its id
+  // ever staged, or a load replaced it) and the id last staged for it
+  struct AddrState { int slot = SLOT_NEW, id = 0; };
+  static constexpr int SLOT_NONE = -1, SLOT_NEW = -2;
+  std::vector<AddrState> addr_;
+  bool new_ids_ = false;      // some staged row changes its address's id
   double* upd_d_ = nullptr;
   int upd_cap_d_ = 0;
 
@@ -213,6 +233,7 @@ class Engine {
   const int* call_iid_d_ = nullptr;
   sapk::CallDesc* desc_h_ = nullptr;   // the descriptor slot at the start of the call block
   sapk::CallDesc* desc_d_ = nullptr;
+  double* call_hd_ = nullptr;          // device alias of call_h_
   hipEvent_t ev_desc_ = nullptr;
   bool desc_pending_ = false;
   uint64_t desc_seq_ = 0;

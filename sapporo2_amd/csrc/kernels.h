@@ -105,6 +105,31 @@ struct PredictArgs {
   const CallDesc* cd;    // ti
 };
 
+// One launch before a directly launched call's force kernel: applies the staged
+// updates, predicts [0, pred_j1), copies the call block (descriptor, i ids, i
+// doubles) to the device and clears the neighbour counters.  Work-groups take
+// one role each: [0, nb_upd) updates, then nb_copy for the call block, the rest
+// predict.  Updates and call block are read from pinned host memory.
+constexpr int PREP_ROWS = 64;   // update rows per work-group
+struct PrepArgs {
+  StoreView st;
+  const double* rows_d;   // staged rows [0, nd), already on the device
+  const double* rows_h;   // staged rows [nd, nupd), host-mapped (row k at row index k)
+  int nd, nupd;
+  const unsigned* bits;   // host-mapped: bit a (< nbits) set when address a is among the updates
+  int nbits;
+  int new_ids;            // some update changes an address's id: widen its tile's id range
+  double ti;
+  int pred_j1;
+  const int4* call_h;     // call block, host-mapped, and its device copy, in 16-byte units
+  int4* call_d;
+  int call_n16;
+  int* ngb_cnt;           // zeroed for [0, ni_reset), with *pack_ctr
+  int ni_reset;
+  int* pack_ctr;
+  int nb_upd, nb_copy;    // filled by launch_prep
+};
+
 struct ForceArgs {
   const void* rec;       // predicted records
   const int2* idr;       // tile id ranges (StoreView::idr)
@@ -187,6 +212,7 @@ struct GatherArgs { StoreView st; int n; double* out; const int* addr; };
 
 int launch_scatter(hipStream_t s, int order, bool f64, const ScatterArgs& a);
 int launch_predict(hipStream_t s, int order, bool f64, const PredictArgs& a);
+int launch_prep(hipStream_t s, int order, bool f64, const PrepArgs& a);
 int launch_force(hipStream_t s, int order, bool f64, const ForceArgs& a, const ForceConfig& c);
 int launch_finalize(hipStream_t s, int order, bool f64, const FinalizeArgs& a);
 // Ensemble force + finalize (+ list sort) over a work table whose first n64

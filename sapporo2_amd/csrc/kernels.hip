@@ -1,10 +1,13 @@
 // kernels.hip -- gfx950 kernels of the direct-summation engine.
 //
-//   k_scatter     staged j-updates -> FP64 SoA store + predicted records
-//                 (reference dev_copy_particles, kernels.cu:245-301), fused with
-//                 the per-call reset of neighbour counters (dev_reset_buffers,
-//                 kernels.cu:1109-1144).
-//   k_predict     FP64 Horner predictor, HBM-bound (dev_predictor, kernels.cu:307-411).
+//   k_prep        one launch before the force kernel: staged j-updates -> FP64
+//                 SoA store + predicted records (reference dev_copy_particles,
+//                 kernels.cu:245-301), FP64 Horner predictor of the other
+//                 j-particles (dev_predictor, kernels.cu:307-411), the call's
+//                 inputs from pinned host memory, and the reset of the neighbour
+//                 counters (dev_reset_buffers, kernels.cu:1109-1144).
+//   k_scatter, k_predict   the same work as launches of their own, for captured
+//                 graphs (their arguments stay fixed) and the allocation-free call.
 //   k_force       acc / pot / jerk [/ snap] + nearest neighbour + neighbour list
 //                 (dev_evaluate_gravity_*, kernels.cu:552-1041).  One wave owns P
 //                 i-particles held in registers and Q = 64/P j-lanes per
@@ -106,10 +109,10 @@ __global__ __launch_bounds__(256) void k_scatter(ScatterArgs a) {
 // ---------------------------------------------------------------------------
 // FP64 predictor.  The expression is the reference's (kernels.cu:332-383),
 // evaluated without contraction, including the zero terms for FOURTH order.
-template <int ORDER>
-__device__ __forceinline__ void predict_one(const double* __restrict__ R, size_t cap, int j,
-                                            double ti, double p[3], double v[3], double ac[3]) {
-  const double dt = ti - R[RF_T * cap + j];
+// get(f) is the particle's raw field f.
+template <int ORDER, typename G>
+__device__ __forceinline__ void predict_one(const G& get, double ti, double p[3], double v[3], double ac[3]) {
+  const double dt = ti - get(RF_T);
   const double dt2 = (1. / 2.) * dt;
   const double dt3 = (1. / 3.) * dt;
   double dt4 = (1. / 4.) * dt;
@@ -117,12 +120,12 @@ __device__ __forceinline__ void predict_one(const double* __restrict__ R, size_t
   if constexpr (ORDER <= ORDER_H4) { dt4 = 0; dt5 = 0; }
 #pragma unroll
   for (int d = 0; d < 3; ++d) {
-    const double xs = R[(RF_X + d) * cap + j];
-    const double vs = R[(RF_VX + d) * cap + j];
-    const double as = R[(RF_AX + d) * cap + j];
-    const double js = R[(RF_JX + d) * cap + j];
+    const double xs = get(RF_X + d);
+    const double vs = get(RF_VX + d);
+    const double as = get(RF_AX + d);
+    const double js = get(RF_JX + d);
     double ss = 0.0, cs = 0.0;
-    if constexpr (ORDER >= ORDER_H6) { ss = R[(RF_SX + d) * cap + j]; cs = R[(RF_CX + d) * cap + j]; }
+    if constexpr (ORDER >= ORDER_H6) { ss = get(RF_SX + d); cs = get(RF_CX + d); }
     p[d] = xs + dt * (vs + dt2 * (as + dt3 * (js + dt4 * (ss + dt5 * (cs)))));
     v[d] = vs + dt * (as + dt2 * (js + dt3 * (ss + dt4 * (cs))));
     ac[d] = as;
@@ -130,34 +133,108 @@ __device__ __forceinline__ void predict_one(const double* __restrict__ R, size_t
   }
 }
 
+// Exact id range of the wave's tile (a wave holds the JTILE addresses of one
+// tile); addresses past the predicted range are included so that later calls
+// with a larger nj stay covered.
+__device__ __forceinline__ void tile_id_range(const StoreView& st, int j) {
+  const int id = j < st.cap ? st.id[j] : 0;
+  int lo = j < st.cap ? id : INT_MAX, hi = j < st.cap ? id : INT_MIN;
+#pragma unroll
+  for (int m = 1; m < 64; m <<= 1) {
+    lo = min(lo, __shfl_xor(lo, m));
+    hi = max(hi, __shfl_xor(hi, m));
+  }
+  if ((threadIdx.x & 63) == 0 && j < st.cap) st.idr[j / JTILE] = make_int2(lo, hi);
+}
+
+// Write the predicted state of address j: the working-precision record and, in
+// mixed precision, the FP64 state kept for read-back.
+template <int ORDER, bool F64>
+__device__ __forceinline__ void put_pred(const StoreView& st, int j, const double p[3], const double v[3],
+                                         const double ac[3], double m, int id) {
+  const size_t cap = (size_t)st.cap;
+  put_rec<ORDER, F64>(st.rec, j, p[0], p[1], p[2], m, v[0], v[1], v[2], ac[0], ac[1], ac[2], id);
+  if constexpr (!F64) {
+    st.ppos[j] = p[0]; st.ppos[cap + j] = p[1]; st.ppos[2 * cap + j] = p[2];
+    st.pvel[j] = v[0]; st.pvel[cap + j] = v[1]; st.pvel[2 * cap + j] = v[2];
+    if constexpr (ORDER >= ORDER_H6) {
+      st.pacc[j] = ac[0]; st.pacc[cap + j] = ac[1]; st.pacc[2 * cap + j] = ac[2];
+    }
+  }
+}
+
 template <int ORDER, bool F64>
 __global__ __launch_bounds__(256) void k_predict(PredictArgs a) {
   const int j = a.j0 + blockIdx.x * blockDim.x + threadIdx.x;
-  // exact id range of this wave's tile (j0 is a multiple of JTILE = wave size);
-  // addresses past j1 are included so later calls with a larger nj stay covered
-  {
-    const int id = j < a.st.cap ? a.st.id[j] : 0;
-    int lo = j < a.st.cap ? id : INT_MAX, hi = j < a.st.cap ? id : INT_MIN;
-#pragma unroll
-    for (int m = 1; m < 64; m <<= 1) {
-      lo = min(lo, __shfl_xor(lo, m));
-      hi = max(hi, __shfl_xor(hi, m));
-    }
-    if ((threadIdx.x & 63) == 0 && j < a.st.cap) a.st.idr[j / JTILE] = make_int2(lo, hi);
-  }
+  tile_id_range(a.st, j);
   if (j >= a.j1) return;
   const size_t cap = (size_t)a.st.cap;
   double p[3], v[3], ac[3];
-  predict_one<ORDER>(a.st.raw, cap, j, a.cd->ti, p, v, ac);
-  put_rec<ORDER, F64>(a.st.rec, j, p[0], p[1], p[2], a.st.raw[RF_M * cap + j], v[0], v[1], v[2],
-                      ac[0], ac[1], ac[2], a.st.id[j]);
-  if constexpr (!F64) {
-    a.st.ppos[j] = p[0]; a.st.ppos[cap + j] = p[1]; a.st.ppos[2 * cap + j] = p[2];
-    a.st.pvel[j] = v[0]; a.st.pvel[cap + j] = v[1]; a.st.pvel[2 * cap + j] = v[2];
-    if constexpr (ORDER >= ORDER_H6) {
-      a.st.pacc[j] = ac[0]; a.st.pacc[cap + j] = ac[1]; a.st.pacc[2 * cap + j] = ac[2];
+  predict_one<ORDER>([&](int f) { return a.st.raw[f * cap + j]; }, a.cd->ti, p, v, ac);
+  put_pred<ORDER, F64>(a.st, j, p, v, ac, a.st.raw[RF_M * cap + j], a.st.id[j]);
+}
+
+// Everything a call needs before its force kernel, in one launch.  It replaces
+// two copy commands, the scatter and the predictor: their run times (3, 4, 4 and
+// 7 us at N = 131072) were less than the 5-8 us gaps between them.  A call of one
+// i-particle went from 58 to 40 us, one of 333 from 149 to 119 us.  Bound by
+// launch and PCIe latency, not by bandwidth (10.4 us for 28 MB at N = 131072).  The predictor skips the addresses whose
+// bit is set: the work-group that holds such an update writes its stored fields
+// and its predicted record from the staged row, so the roles never write the
+// same address and need no order among them.  The tile id ranges are the
+// predictor's alone: a call whose updates change an id runs the updates in a
+// launch of their own before it (new_ids).
+template <int ORDER, bool F64>
+__global__ __launch_bounds__(256) void k_prep(PrepArgs a) {
+  constexpr int NF = raw_fields(ORDER), NR = NF + 1;
+  __shared__ double buf[PREP_ROWS * NR];
+  const int t = threadIdx.x;
+  const size_t cap = (size_t)a.st.cap;
+  int b = blockIdx.x;
+  if (b < a.nb_upd) {
+    const int k0 = b * PREP_ROWS, n = min(PREP_ROWS, a.nupd - k0);
+    // whole lines over PCIe: the group's rows are one contiguous range
+    for (int e = t; e < n * NR; e += 256) {
+      const size_t o = (size_t)k0 * NR + e;
+      buf[e] = o < (size_t)a.nd * NR ? a.rows_d[o] : a.rows_h[o];
     }
+    __syncthreads();
+    const int r = t & (PREP_ROWS - 1);
+    if (r >= n) return;
+    const double* u = buf + r * NR;
+    const int2 pair = *reinterpret_cast<const int2*>(u + NF);  // address, id
+    const int addr = pair.x;
+    if (addr < 0 || addr >= a.st.cap) return;  // host guarantees range
+    for (int f = t / PREP_ROWS; f < NF; f += 256 / PREP_ROWS) a.st.raw[(size_t)f * cap + addr] = u[f];
+    if (t >= PREP_ROWS) return;
+    if (a.new_ids) {
+      a.st.id[addr] = pair.y;
+      atomicMin(&a.st.idr[addr / JTILE].x, pair.y);
+      atomicMax(&a.st.idr[addr / JTILE].y, pair.y);
+    }
+    // predicted = stored for addresses that are not predicted (kernels.cu:281-298)
+    double p[3] = {u[RF_X], u[RF_Y], u[RF_Z]}, v[3] = {u[RF_VX], u[RF_VY], u[RF_VZ]}, ac[3] = {0, 0, 0};
+    if constexpr (ORDER >= ORDER_H6) { ac[0] = u[RF_AX]; ac[1] = u[RF_AY]; ac[2] = u[RF_AZ]; }
+    if (addr < a.pred_j1) predict_one<ORDER>([&](int f) { return u[f]; }, a.ti, p, v, ac);
+    put_pred<ORDER, F64>(a.st, addr, p, v, ac, u[RF_M], pair.y);
+    return;
   }
+  b -= a.nb_upd;
+  if (b < a.nb_copy) {
+    const int stride = a.nb_copy * 256;
+    for (int k = b * 256 + t; k < a.call_n16; k += stride) a.call_d[k] = a.call_h[k];
+    for (int k = b * 256 + t; k < a.ni_reset; k += stride) a.ngb_cnt[k] = 0;
+    if (b == 0 && t == 0 && a.ni_reset > 0) *a.pack_ctr = 0;
+    return;
+  }
+  b -= a.nb_copy;
+  const int j = b * 256 + t;
+  const bool skip = j < a.nbits && (a.bits[j >> 5] >> (j & 31) & 1u);
+  tile_id_range(a.st, j);
+  if (j >= a.pred_j1 || skip) return;
+  double p[3], v[3], ac[3];
+  predict_one<ORDER>([&](int f) { return a.st.raw[f * cap + j]; }, a.ti, p, v, ac);
+  put_pred<ORDER, F64>(a.st, j, p, v, ac, a.st.raw[RF_M * cap + j], a.st.id[j]);
 }
 
 // ---------------------------------------------------------------------------
@@ -977,6 +1054,20 @@ int launch_predict(hipStream_t s, int order, bool f64, const PredictArgs& a) {
   const int nb = blocks_for(a.j1 - a.j0, 256);
   dispatch_op(order, f64, [&](auto OR, auto FP) {
     hipLaunchKernelGGL((k_predict<decltype(OR)::value, decltype(FP)::value>), dim3(nb), dim3(256), 0, s, a);
+  });
+  return hip_status();
+}
+
+// Copy work-groups: 4 x 16 bytes a thread, at most 64 groups (256 KB in flight
+// covers the PCIe latency at its full rate).
+int launch_prep(hipStream_t s, int order, bool f64, const PrepArgs& args) {
+  PrepArgs a = args;
+  a.nb_upd = blocks_for(a.nupd, PREP_ROWS);
+  a.nb_copy = std::min(64, blocks_for(std::max<long>(a.call_n16, a.ni_reset), 1024));
+  const int nb = a.nb_upd + a.nb_copy + blocks_for(a.pred_j1, 256);
+  if (nb == 0) return 0;
+  dispatch_op(order, f64, [&](auto OR, auto FP) {
+    hipLaunchKernelGGL((k_prep<decltype(OR)::value, decltype(FP)::value>), dim3(nb), dim3(256), 0, s, a);
   });
   return hip_status();
 }
