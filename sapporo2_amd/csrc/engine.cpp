@@ -34,12 +34,21 @@ namespace {
 constexpr int WAVES_PER_SIMD_TARGET = 32;   // several dispatch rounds balance better
 constexpr int MIN_ITERS_PER_LANE = 16;
 constexpr int MIN_J_PER_SPLIT = 512;
-constexpr int FOLD = 64;   // interactions per lane between FP64 folds (kernels.hip KT)
+// Launch shapes of lane shape P = 64 (choose_config)
+constexpr long MIN_CHUNK = 64, MAX_CHUNK = 256, MAX_WAVES = 65536;
+// Mixed launches of at most this many waves (4 per SIMD) take their records
+// ahead: one wave alone waits ~190 ns per pair for scalar loads, 80 with them
+// ahead (64 i x 131072 j in 2048 waves 26 -> 23 us); a full SIMD hides them, and
+// the grouped operands then cost issue slots (16384 i: 1349 -> 1558 us).
+constexpr long AHEAD_WAVES = 4096;
 constexpr int IBUF_FIELDS = 10;  // xi 3, vi 3, ai 3, h2 1
 // Staged j-update rows are copied to the device as soon as this many are
 // pending, while the caller is still staging (the copy overlaps its loop).
 constexpr int EARLY_FLUSH_ROWS = 4096;
 constexpr int BATCH_ROWS = 16384;  // rows a batch stages at a time
+// Rows from which staging uses the host threads: waking them costs ~50 us after
+// a long call, a row ~10 ns on the caller (2500 rows: 70 us with them, 20 without).
+constexpr size_t PAR_ROWS = 6144;
 // Upload block of a single-system call, one host->device copy: the call
 // descriptor, then the i ids, then the i doubles.  The ids region is sized by
 // the power-of-two bucket of ni, so every offset depends on the bucket only
@@ -375,9 +384,11 @@ int Engine::open_stage() {
   if (nstaged_ != 0) return 0;
   Stage& sg = stage_[cur_];
   if (sg.busy && wait_stage(sg) != 0) return -1;
-  par_for(sg.addr.size(), [&](size_t b, size_t e) {
+  auto clear = [&](size_t b, size_t e) {
     for (size_t k = b; k < e; ++k) __atomic_store_n(&sg.bits[sg.addr[k] >> 5], 0u, __ATOMIC_RELAXED);
-  });
+  };
+  if (sg.addr.size() >= PAR_ROWS) par_for(sg.addr.size(), clear);
+  else clear(0, sg.addr.size());
   sg.addr.clear();
   return 0;
 }
@@ -496,7 +507,7 @@ int Engine::set_j_particles(int n, const int* addr, const int* id, const double*
                dtj ? dtj[k] : 0.0, mass[k], a ? a + o : nullptr, jrk ? jrk + o : nullptr, v ? v + o : nullptr, x + o,
                snp ? snp + o : nullptr, crk ? crk + o : nullptr, eps ? eps[k] : 0.0);
     };
-    if (amin >= 0 && e - b >= (int)(2 * HOST_CHUNK)) {
+    if (amin >= 0 && e - b >= (int)PAR_ROWS) {
       const int rc = stage_block(e - b, addr + b, id + b, [&](int r, int k) { row(r, b + k); });
       if (rc < 0) return -1;
       if (rc > 0) continue;
@@ -584,9 +595,11 @@ int Engine::upload_updates(int* nupd) {
 // stage.
 void Engine::hand_over() {
   const std::vector<int>& staged = stage_[cur_].addr;
-  par_for(staged.size(), [&](size_t b, size_t e) {
+  auto release = [&](size_t b, size_t e) {
     for (size_t k = b; k < e; ++k) addr_[staged[k]].slot = SLOT_NONE;
-  });
+  };
+  if (staged.size() >= PAR_ROWS) par_for(staged.size(), release);
+  else release(0, staged.size());
   nstaged_ = 0;
   flushed_ = 0;
   new_ids_ = false;
@@ -746,7 +759,20 @@ ForceConfig Engine::choose_config(int ni, int nj, bool ngb) const {
   const int Q = 64 / P;
   const long G = (ni + P - 1) / P;
   long S;
-  if (jchunk_t > 0) {
+  if (P == 64 && ni > 32) {
+    // One round of waves (8 per SIMD mixed, 5 in FP64) while that leaves a wave
+    // MIN_CHUNK j or more; the fixed cost of a wave (its i-particles, cold
+    // records, epilogue) is then small against its pairs.  More i-groups take
+    // several rounds of MAX_CHUNK j, so that the last round is short, up to
+    // MAX_WAVES, where the partial rows begin to cost more than the balance gains.
+    // Force + finalize in us, N = 131072 unless said, by j per split:
+    //   128 i   32: 35+36  64: 31+22  128: 38+14 | 333 i   64: 59+22 128: 52+15 256: 65+11
+    //   1000 i 128: 111+37 256: 115+23 512: 132+16 | 3000 i 128: 279+39 256: 276+25 784: 317+22
+    //   16384 i 512: 1349+75 1024: 1365+78 2048: 1448+79; N = 2^20 4096: 11050+38 8192: 11271+38
+    const long slots = (long)cus_ * 4 * (f64_ ? 5 : 8);
+    const long jc = std::min<long>(MAX_CHUNK, std::max<long>(MIN_CHUNK, ((long)nj * G + slots - 1) / slots));
+    S = std::min<long>((nj + jc - 1) / jc, std::max<long>(1, MAX_WAVES / G));
+  } else if (jchunk_t > 0) {
     S = (nj + jchunk_t - 1) / jchunk_t;
   } else {
     const long target = (long)cus_ * 4 * WAVES_PER_SIMD_TARGET;
@@ -758,13 +784,18 @@ ForceConfig Engine::choose_config(int ni, int nj, bool ngb) const {
   if (ovr_S_ > 0) S = ovr_S_;
   if (S < 1) S = 1;
   long jchunk = (nj + S - 1) / S;
-  const long tile = (long)Q * FOLD;
-  if (jchunk >= tile) jchunk = (jchunk + tile - 1) / tile * tile;
+  const long unit = (long)Q * FORCE_SUB;
+  if (jchunk >= unit) jchunk = (jchunk + unit - 1) / unit * unit;
   else jchunk = (jchunk + Q - 1) / Q * Q;
   if (jchunk < 1) jchunk = 1;
   S = (nj + jchunk - 1) / jchunk;
-  if (S < 1) S = 1;
-  return ForceConfig{P, (int)S, (int)jchunk, ovr_smajor_, ovr_pipe_};
+  // Empty splits at the end, so that work-groups are whole; and, consecutive work-
+  // groups going to the 8 XCDs in turn, whole eights of them per i-group, so that
+  // a j-range stays in one XCD's L2.
+  const long whole = P == 64 && S >= 256 ? 32 : 4;
+  S = (S + whole - 1) / whole * whole;
+  const int ahead = G * S <= AHEAD_WAVES ? 1 : 0;
+  return ForceConfig{P, (int)S, (int)jchunk, ovr_smajor_, ovr_pipe_, ahead};
 }
 
 // i-particle-sized buffers (ensemble inputs, host-mapped result rows and list
@@ -1124,7 +1155,7 @@ int Engine::start_grav_calc_clusters(int ni, const int* cluster, const int* id, 
   ngb_on_last_ = ngb_on;
   ni_last_ = ni;
   nj_last_ = cl_total_;
-  last_cfg_ = ForceConfig{0, nitems, (int)jch64, 0, 0};
+  last_cfg_ = ForceConfig{0, nitems, (int)jch64, 0, 0, 0};
   jhost_valid_ = false;
   return 0;
 }
@@ -1192,11 +1223,11 @@ int Engine::start_grav_calc(int nj, int ni, const int* id, const double (*xi)[3]
   if (timing_) HIPCHK(hipEventRecord(ev_d0_, stream_), "event");
   if (graphs_) {
     const int sblocks = scatter_blocks(nupd, ngb_on ? ni : 0);
-    if (launch_call_graph(grid_ni, nj, cfg, ngb_on, predict, sblocks, bucket >= 1024) != 0) return -1;
+    if (launch_call_graph(grid_ni, nj, cfg, ngb_on, predict, sblocks, finalize_threads(bucket)) != 0) return -1;
     timed_predict_ = timed_force_ = false;
   } else {
     if (prep(predict ? nj : 0, (int)nbytes, ngb_on ? ni : 0, true) != 0) return -1;
-    if (enqueue_force(grid_ni, nj, cfg, ngb_on, bucket >= 1024) != 0) return -1;
+    if (enqueue_force(grid_ni, nj, cfg, ngb_on, finalize_threads(bucket)) != 0) return -1;
     timed_force_ = timing_;
   }
   if (timing_) HIPCHK(hipEventRecord(ev_d1_, stream_), "event");
@@ -1219,7 +1250,7 @@ int Engine::start_grav_calc(int nj, int ni, const int* id, const double (*xi)[3]
 // finalize.  Every per-call value comes from the descriptor, so the sequence
 // depends only on its arguments here (the key of the graph).
 int Engine::enqueue_call(int grid_ni, int nj, const ForceConfig& cfg, bool ngb_on, bool predict, int sblocks,
-                         bool rows) {
+                         int fin_u) {
   if (sblocks > 0) {
     ScatterArgs a{};
     a.st = st_;
@@ -1234,11 +1265,11 @@ int Engine::enqueue_call(int grid_ni, int nj, const ForceConfig& cfg, bool ngb_o
   }
   timed_scatter_ = false;
   if (predict && predict_range(0, nj) != 0) return -1;
-  return enqueue_force(grid_ni, nj, cfg, ngb_on, rows);
+  return enqueue_force(grid_ni, nj, cfg, ngb_on, fin_u);
 }
 
 // Force and finalize kernels of a call.
-int Engine::enqueue_force(int grid_ni, int nj, const ForceConfig& cfg, bool ngb_on, bool rows) {
+int Engine::enqueue_force(int grid_ni, int nj, const ForceConfig& cfg, bool ngb_on, int fin_u) {
   ForceArgs fa{};
   fa.rec = st_.rec;
   fa.idr = st_.idr;
@@ -1259,7 +1290,7 @@ int Engine::enqueue_force(int grid_ni, int nj, const ForceConfig& cfg, bool ngb_
   if (ev) HIPCHK(hipEventRecord(ev_f1_, stream_), "event");
   FinalizeArgs fz = finalize_args(grid_ni, ngb_on);
   fz.S = partial_rows(cfg);
-  fz.rows = rows ? 1 : 0;
+  fz.U = fin_u;
   if (launch_finalize(stream_, order_, f64_, fz) != 0) return fail("finalize launch", hipGetLastError());
   return 0;
 }
@@ -1333,7 +1364,7 @@ int Engine::grav_calc_scratch(void* scratch, size_t bytes, int nj, int ni, const
   fz.S = partial_rows(cfg);
   fz.cd = cd;
   fz.grid_ni = ni;
-  fz.rows = bucket >= 1024 ? 1 : 0;
+  fz.U = finalize_threads(bucket);
   fz.rec = st_.rec;
   fz.out = out_d;
   fz.ostride = ni;
@@ -1348,9 +1379,9 @@ constexpr size_t MAX_GRAPHS = 64;
 // needed (least recently used graphs are dropped beyond MAX_GRAPHS; graphs
 // whose buffers were reallocated are dropped when next seen).
 int Engine::launch_call_graph(int grid_ni, int nj, const ForceConfig& cfg, bool ngb_on, bool predict, int sblocks,
-                              bool rows) {
-  const GraphKey key{grid_ni, nj, cfg.P, cfg.S, cfg.jchunk, cfg.smajor, cfg.pipe, ngb_on ? 1 : 0,
-                     predict ? 1 : 0, sblocks * 2 + (rows ? 1 : 0), gen_};
+                              int fin_u) {
+  const GraphKey key{grid_ni, nj, cfg.P, cfg.S, cfg.jchunk, cfg.smajor, cfg.pipe, cfg.ahead, ngb_on ? 1 : 0,
+                     predict ? 1 : 0, sblocks, fin_u, gen_};
   for (auto& e : graph_cache_) {
     if (e.key == key) {
       e.used = ++tick_;
@@ -1381,7 +1412,7 @@ int Engine::launch_call_graph(int grid_ni, int nj, const ForceConfig& cfg, bool 
   hipGraph_t g = nullptr;
   HIPCHK(hipStreamBeginCapture(stream_, hipStreamCaptureModeRelaxed), "graph capture");
   capturing_ = true;
-  const int rc = enqueue_call(grid_ni, nj, cfg, ngb_on, predict, sblocks, rows);
+  const int rc = enqueue_call(grid_ni, nj, cfg, ngb_on, predict, sblocks, fin_u);
   capturing_ = false;
   const hipError_t ec = hipStreamEndCapture(stream_, &g);
   if (rc != 0 || ec != hipSuccess || !g) {

@@ -145,10 +145,10 @@ class Engine {
               const double* h2, double* bx, double* bv, double* ba, double* bh, int* bid);
   int scatter_blocks(int nupd, int ni_reset) const;
   int enqueue_call(int grid_ni, int nj, const sapk::ForceConfig& cfg, bool ngb_on, bool predict,
-                   int sblocks, bool rows);
-  int enqueue_force(int grid_ni, int nj, const sapk::ForceConfig& cfg, bool ngb_on, bool rows);
+                   int sblocks, int fin_u);
+  int enqueue_force(int grid_ni, int nj, const sapk::ForceConfig& cfg, bool ngb_on, int fin_u);
   int launch_call_graph(int grid_ni, int nj, const sapk::ForceConfig& cfg, bool ngb_on, bool predict,
-                        int sblocks, bool rows);
+                        int sblocks, int fin_u);
   void drop_graphs();
   int wait_results();
   int ensure_lists(int need);
@@ -222,7 +222,7 @@ class Engine {
   bool timed_predict_ = false, timed_force_ = false;
   bool capturing_ = false;
   int ni_last_ = 0, nj_last_ = 0;
-  sapk::ForceConfig last_cfg_{64, 1, 1, 0, 0};
+  sapk::ForceConfig last_cfg_{64, 1, 1, 0, 0, 0};
   bool timing_ = false;
   int ovr_P_ = 0, ovr_S_ = 0, ovr_smajor_ = 0, ovr_pipe_ = 0;
 
@@ -244,11 +244,11 @@ class Engine {
   uint64_t gen_ = 1;          // bumped whenever a buffer a captured graph uses is reallocated
   uint64_t tick_ = 0;
   struct GraphKey {
-    int grid_ni, nj, P, S, jchunk, smajor, pipe, ngb_on, predict, sblocks;
+    int grid_ni, nj, P, S, jchunk, smajor, pipe, ahead, ngb_on, predict, sblocks, fin_u;
     uint64_t gen;
     bool operator==(const GraphKey& o) const {
       return grid_ni == o.grid_ni && nj == o.nj && P == o.P && S == o.S && jchunk == o.jchunk &&
-             smajor == o.smajor && pipe == o.pipe && ngb_on == o.ngb_on && predict == o.predict &&
+             smajor == o.smajor && pipe == o.pipe && ahead == o.ahead && fin_u == o.fin_u && ngb_on == o.ngb_on && predict == o.predict &&
              sblocks == o.sblocks && gen == o.gen;
     }
   };

@@ -148,13 +148,25 @@ struct ForceArgs {
 
 // Launch geometry of one force call: each wave owns P i-particles and Q = 64/P
 // j-lanes per i-particle over one of S contiguous j-ranges of jchunk.
-// smajor: wave-to-split mapping; pipe: neighbour-id stores deferred by one group.
-struct ForceConfig { int P; int S; int jchunk; int smajor; int pipe; };
+// smajor: wave-to-split mapping; pipe: neighbour-id stores deferred by one group;
+// ahead (P = 64): records loaded ahead of the pairs.
+struct ForceConfig { int P; int S; int jchunk; int smajor; int pipe; int ahead; };
+
+// Iterations of a lane that the pair loop takes at a time; a j-split is a whole
+// number of them (SUB * Q j), except for what the last split has left.
+constexpr int FORCE_SUB = 16;
 
 // Partial-sum rows a force launch writes per i-particle.  With S a multiple of
 // 4 and split-minor wave order the 4 waves of a work-group are 4 consecutive
 // splits of one i-group; they combine their sums in LDS and write one row.
 inline int partial_rows(const ForceConfig& c) { return (c.S % 4 == 0 && !c.smajor) ? c.S / 4 : c.S; }
+
+// Threads per i-particle of the finalize for a power-of-two bucket of ni (the
+// shape decides the order of the sums, so direct, replayed and allocation-free
+// calls of one ni take the same).  A launch of ~16384 threads or more keeps the
+// row reads in flight: with 4 threads each, 1000 i-particles of 128 rows took
+// 23 us.
+constexpr int finalize_threads(int bucket) { return bucket > 4096 ? 4 : bucket > 512 ? 16 : 64; }
 
 // Results and neighbour lists go straight to host-mapped pinned memory (no
 // copy command): field-major result rows out[f * ostride + i], and each sorted
@@ -172,7 +184,7 @@ struct FinalizeArgs {
   int S;
   const CallDesc* cd;    // ni
   int grid_ni;           // launch size (host), >= cd->ni
-  int rows;              // shape: 1 thread per i-particle (else a work-group per i-particle)
+  int U;                 // threads per i-particle (finalize_threads)
   const void* rec;       // to look up the neighbour's id
   int* ngb_cnt; int* ngb_list;
   double* out;           // host-mapped: out_fields x ostride doubles, field-major

@@ -296,8 +296,7 @@ template <int ORDER> constexpr int nf() { return ORDER >= ORDER_H6 ? NF6 : NF4; 
 // nnaddr hold the distance and the address j of the nearest so far.
 template <int ORDER, bool NGB, bool CHECK, bool BLOCKMIN, typename R, typename Rec>
 __device__ __forceinline__ bool pair(const Rec& r, const int j, const bool ok, const IState<ORDER, R>& s,
-                                     const R eps2, R (&t)[nf<ORDER>()], R& dsmin, int& nnaddr,
-                                     int* __restrict__ ngb_cnt, int* __restrict__ ngb_list) {
+                                     const R eps2, R (&t)[nf<ORDER>()], R& dsmin, int& nnaddr) {
   R dx, dy, dz;
   const R ds2 = pair_ds2<R>(r, s, dx, dy, dz);
   // bitwise & keeps the predicates branch-free (no exec-masked regions)
@@ -357,12 +356,40 @@ __device__ __forceinline__ bool pair(const Rec& r, const int j, const bool ok, c
   return NGB & use & (s.h2 > ds2);
 }
 
-// Append id to the i-particle's list; rare (~32 per 1e5 pairs), so a global
-// atomic takes the slot; the count stays exact past NGB_CAP.
-__device__ __forceinline__ void ngb_append(int* __restrict__ ngb_cnt, int* __restrict__ ngb_list, int i, int id) {
-  const int k = atomicAdd(&ngb_cnt[i], 1);
-  if (k < NGB_CAP) ngb_list[(size_t)i * NGB_CAP + k] = id;
-}
+// Append to the i-particle's list; rare (~32 per 1e5 pairs), so a global atomic
+// takes the slots.  The count stays exact past NGB_CAP; a lane that has met a
+// full list only counts (over >= 0) and adds its count at the end, so that an
+// i-particle with most of the system inside its radius does not serialise the
+// launch on one counter (777 i x 30011 j with one such particle: 284 us of
+// which the pairs are 90).
+struct NgbList {
+  int* __restrict__ cnt;
+  int* __restrict__ list;
+  int i;
+  int over;  // -1: the list may have room
+  __device__ __forceinline__ void add(int id) {
+    if (over >= 0) { ++over; return; }
+    const int k = atomicAdd(&cnt[i], 1);
+    if (k < NGB_CAP) list[(size_t)i * NGB_CAP + k] = id;
+    else over = 0;
+  }
+  // the pairs u of a group with nb[u], ids through id(u): their slots in one atomic
+  template <typename F> __device__ __forceinline__ void add4(const bool (&nb)[4], const F& id) {
+    const int c = (int)nb[0] + (int)nb[1] + (int)nb[2] + (int)nb[3];
+    if (c == 0) return;
+    if (over >= 0) { over += c; return; }
+    int k = atomicAdd(&cnt[i], c);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      if (nb[u] && k < NGB_CAP) list[(size_t)i * NGB_CAP + k] = id(u);
+      k += nb[u] ? 1 : 0;
+    }
+    if (k >= NGB_CAP) over = 0;
+  }
+  __device__ __forceinline__ void finish() {
+    if (over > 0) atomicAdd(&cnt[i], over);
+  }
+};
 
 // Neighbour slots reserved by one group whose id stores are still pending.
 struct PendingNgb {
@@ -395,8 +422,7 @@ __device__ __forceinline__ void settle(R (&t)[nf<ORDER>()]) {
 // positions live across it, which costs a wave of occupancy.
 template <int ORDER, bool NGB, bool CHECK, int Q, bool PIPE, typename R, typename Rec>
 __device__ __forceinline__ void pair4(const Rec* __restrict__ rec, const int j0, const IState<ORDER, R>& s,
-                                      const R eps2, R (&t)[nf<ORDER>()], R& smin, int* __restrict__ ngb_cnt,
-                                      int* __restrict__ ngb_list, PendingNgb& pend) {
+                                      const R eps2, R (&t)[nf<ORDER>()], R& smin, NgbList& ngb, PendingNgb& pend) {
   R d[4];
   int idj[4];
   int unused = 0;
@@ -405,7 +431,7 @@ __device__ __forceinline__ void pair4(const Rec* __restrict__ rec, const int j0,
     const int j = j0 + u * Q;
     const Rec& r = rec[j];
     idj[u] = r.id;
-    pair<ORDER, NGB, CHECK, true>(r, j, true, s, eps2, t, d[u], unused, ngb_cnt, ngb_list);
+    pair<ORDER, NGB, CHECK, true>(r, j, true, s, eps2, t, d[u], unused);
   }
   // the group's nearest distance: it lowers the sub-block minimum, and h2 > it
   // is the test whether any of the four pairs is a neighbour
@@ -417,12 +443,12 @@ __device__ __forceinline__ void pair4(const Rec* __restrict__ rec, const int j0,
   if constexpr (!NGB) __builtin_amdgcn_sched_barrier(0);
   const bool any = NGB && __ballot(s.h2 > g) != 0;
   if constexpr (NGB && PIPE) {
-    ngb_flush(pend, ngb_list, s.i);
+    ngb_flush(pend, ngb.list, s.i);
     if (any) {
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
         const bool nb = s.h2 > d[u];
-        if (nb) pend.k[u] = atomicAdd(&ngb_cnt[s.i], 1);
+        if (nb) pend.k[u] = atomicAdd(&ngb.cnt[s.i], 1);
         pend.id[u] = idj[u];
         pend.m[u] = nb;
       }
@@ -430,19 +456,91 @@ __device__ __forceinline__ void pair4(const Rec* __restrict__ rec, const int j0,
   } else if constexpr (NGB) {
     if (any) {
 #pragma unroll
-      for (int u = 0; u < 4; ++u)
-        if (s.h2 > d[u]) ngb_append(ngb_cnt, ngb_list, s.i, idj[u]);
+      for (int u = 0; u < 4; ++u) asm volatile("" : "+v"(d[u]));
+      const bool nb[4] = {s.h2 > d[0], s.h2 > d[1], s.h2 > d[2], s.h2 > d[3]};
+      ngb.add4(nb, [&](int u) { return rec[j0 + u * Q].id; });
     }
   }
 }
 
 constexpr int KT = 64;  // interactions per lane between FP64 folds
+constexpr int SUB = FORCE_SUB;
+static_assert(KT % SUB == 0 && SUB % 4 == 0, "fold");
+
+// J-records on their way through the scalar cache (lane shape P = 64): JU
+// consecutive records held in SGPRs, as one or two wide scalar loads.
+typedef int v8i __attribute__((ext_vector_type(8)));
+typedef int v16i __attribute__((ext_vector_type(16)));
+template <typename Rec> struct JUnit {
+  static constexpr int JU = sizeof(Rec) == 48 ? 2 : 1;
+  static constexpr bool TAIL = sizeof(Rec) * JU == 96;
+  v16i h;
+  v8i t;
+  __device__ __forceinline__ void load(const Rec* __restrict__ p) {
+    h = *reinterpret_cast<const v16i*>(p);
+    if constexpr (TAIL) t = *reinterpret_cast<const v8i*>(reinterpret_cast<const char*>(p) + 64);
+  }
+  // The loads have arrived (scalar loads return out of order: a wait is for
+  // all of them, so this comes before the next unit's loads are issued).
+  __device__ __forceinline__ void arrive() {
+    asm volatile("" : "+s"(h));
+    if constexpr (TAIL) asm volatile("" : "+s"(t));
+  }
+  __device__ __forceinline__ Rec get(int u) const {
+    struct { v16i h; v8i t; } b{h, t};
+    Rec r;
+    __builtin_memcpy(&r, reinterpret_cast<const char*>(&b) + u * sizeof(Rec), sizeof(Rec));
+    return r;
+  }
+};
+
+// Four consecutive j of a wave whose lanes share the j-record (Q = 1): the
+// arithmetic of pair4, with the records of the next pairs loaded while the
+// present ones are computed.  a holds the first unit of the group on entry and
+// the first unit of the next group (at jnext) on return.
+template <int ORDER, bool NGB, bool CHECK, typename R, typename Rec>
+__device__ __forceinline__ void group4(const Rec* __restrict__ rec, const int j0, const int jnext, JUnit<Rec>& a,
+                                       const IState<ORDER, R>& s, const R eps2, R (&t)[nf<ORDER>()], R& smin,
+                                       NgbList& ngb) {
+  constexpr int JU = JUnit<Rec>::JU;
+  R d[4];
+  int unused = 0;
+  JUnit<Rec> b;
+#pragma unroll
+  for (int u = 0; u < 4; u += 2 * JU) {
+    a.arrive();
+    __builtin_amdgcn_sched_barrier(0);
+    b.load(rec + j0 + u + JU);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int k = 0; k < JU; ++k)
+      pair<ORDER, NGB, CHECK, true>(a.get(k), 0, true, s, eps2, t, d[u + k], unused);
+    b.arrive();
+    __builtin_amdgcn_sched_barrier(0);
+    a.load(rec + (u + 2 * JU < 4 ? j0 + u + 2 * JU : jnext));
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int k = 0; k < JU; ++k)
+      pair<ORDER, NGB, CHECK, true>(b.get(k), 0, true, s, eps2, t, d[u + JU + k], unused);
+  }
+  const R g = minR<R>(minR<R>(minR<R>(d[0], d[1]), d[2]), d[3]);
+  smin = minR<R>(smin, g);
+  if constexpr (NGB) {
+    settle<ORDER>(t);
+    if (__ballot(s.h2 > g) != 0) {
+      const bool nb[4] = {s.h2 > d[0], s.h2 > d[1], s.h2 > d[2], s.h2 > d[3]};
+      ngb.add4(nb, [&](int u) { return rec[j0 + u].id; });
+    }
+  }
+}
 
 // The work of one wave: i-particles [i0, i0 + icount) (icount <= P) against
 // j in [jb, je), Q = 64/P j-lanes per i-particle.  On return the lanes with
 // writer set hold the wave-reduced FP64 sums T, nearest-neighbour (ds2,
 // address) and their i-slot.
-template <int ORDER, bool F64, int P, bool NGB, bool PIPE = false>
+// AHEAD (P = 64): the records of the next pairs are loaded while the present
+// ones are computed.
+template <int ORDER, bool F64, int P, bool NGB, bool PIPE = false, bool AHEAD = false>
 __device__ __forceinline__ void wave_force(
     const typename RecOf<ORDER, F64>::T* __restrict__ rec, const int2* __restrict__ idr,
     const double* __restrict__ ipos, const double* __restrict__ ivel, const double* __restrict__ iacc,
@@ -473,6 +571,7 @@ __device__ __forceinline__ void wave_force(
 
 #pragma unroll
   for (int f = 0; f < NF; ++f) T[f] = 0.0;
+  NgbList ngb{ngb_cnt, ngb_list, il, -1};
   R dsmin = R(INFINITY);
   // nearest pair so far: -1 none; >= 0 the first address of the sub-block of
   // 16 pairs (whole tiles) that holds it; <= -2 the exact address a, as -2 - a
@@ -483,62 +582,63 @@ __device__ __forceinline__ void wave_force(
   for (int u = 0; u < 4; ++u) { pend.m[u] = false; pend.k[u] = 0; pend.id[u] = 0; }
 
   const int nk = (je > jb) ? (je - jb + Q - 1) / Q : 0;  // iterations of the lane with jsub 0
+  const int nw = (je > jb) ? (je - jb) / Q : 0;          // iterations that every lane has
   // FP32 pair terms are summed per fold of KT and folded into FP64 T; in FP64
   // the pair terms go straight into t, which becomes T at the end
   R t[NF];
 #pragma unroll
   for (int f = 0; f < NF; ++f) t[f] = R(0);
+  JUnit<Rec> ja;
+  const int jend = jb + nw / SUB * SUB;  // AHEAD: end of the whole sub-blocks, loads stay below it
+  if constexpr (AHEAD) ja.load(rec + (nw >= SUB ? jb : 0));
   for (int k0 = 0; k0 < nk; k0 += KT) {
     if constexpr (!F64) {
 #pragma unroll
       for (int f = 0; f < NF; ++f) t[f] = R(0);
     }
     const int kn = min(KT, nk - k0);
+    // whole sub-blocks of SUB iterations; what is left of the range's end goes pair by pair
+    const int kw = min(KT, nw - k0) / SUB * SUB;
     const int jt = jb + k0 * Q + jsub;
-    if (kn == KT && jb + (k0 + KT) * Q <= je) {
-      // P = 64: one JTILE-aligned tile per fold; skip the self test when no
-      // lane's id can occur in the tile
+    if (kw > 0) {
+      // P = 64: the fold's j lie in at most two tiles; skip the self test when
+      // no lane's id can occur in them
       bool check = true;
       if constexpr (Q == 1) {
-        if ((jt & (JTILE - 1)) == 0) {
-          const int2 r = idr[jt / JTILE];
-          check = __ballot(st.id >= r.x && st.id <= r.y) != 0;
-        }
+        const int2 r0 = idr[jt / JTILE], r1 = idr[(jt + kw - 1) / JTILE];
+        check = __ballot(st.id >= min(r0.x, r1.x) && st.id <= max(r0.y, r1.y)) != 0;
       }
       // Nearest neighbour: each pair only lowers the minimum of its sub-block of
       // 16 pairs (one v_min); a sub-block that beats the lane's nearest so far
       // records its first address, resolved to the pair after the loop.
-      if (check) {
-        for (int k = 0; k < KT; k += 16) {
+      auto sweep = [&](auto chk) {
+        for (int k = 0; k < kw; k += SUB) {
           R sm = R(INFINITY);
 #pragma unroll
-          for (int q = 0; q < 16; q += 4)
-            pair4<ORDER, NGB, true, Q, PIPE>(rec, jt + (k + q) * Q, st, eps2, t, sm, ngb_cnt, ngb_list, pend);
+          for (int q = 0; q < SUB; q += 4) {
+            const int j = jt + (k + q) * Q;
+            if constexpr (AHEAD)
+              group4<ORDER, NGB, decltype(chk)::value>(rec, j, j + 4 < jend ? j + 4 : jb, ja, st, eps2, t, sm, ngb);
+            else
+              pair4<ORDER, NGB, decltype(chk)::value, Q, PIPE>(rec, j, st, eps2, t, sm, ngb, pend);
+          }
           const bool better = sm < dsmin;
           dsmin = better ? sm : dsmin;
           nnblk = better ? jt + k * Q : nnblk;
         }
-      } else {
-        for (int k = 0; k < KT; k += 16) {
-          R sm = R(INFINITY);
-#pragma unroll
-          for (int q = 0; q < 16; q += 4)
-            pair4<ORDER, NGB, false, Q, PIPE>(rec, jt + (k + q) * Q, st, eps2, t, sm, ngb_cnt, ngb_list, pend);
-          const bool better = sm < dsmin;
-          dsmin = better ? sm : dsmin;
-          nnblk = better ? jt + k * Q : nnblk;
-        }
-      }
-    } else {
-      if constexpr (NGB && PIPE) ngb_flush(pend, ngb_list, st.i);
+      };
+      if (check) sweep(std::true_type{});
+      else sweep(std::false_type{});
+    }
+    if (kw < kn) {
+      if constexpr (NGB && PIPE) ngb_flush(pend, ngb.list, st.i);
       const R before = dsmin;
       int cand = 0;
-      for (int k = 0; k < kn; ++k) {
+      for (int k = max(kw, 0); k < kn; ++k) {
         const int j = jt + k * Q;
         const bool ok = j < je;
         const Rec& r = rec[ok ? j : jb];
-        if (pair<ORDER, NGB, true, false>(r, j, ok, st, eps2, t, dsmin, cand, ngb_cnt, ngb_list))
-          ngb_append(ngb_cnt, ngb_list, st.i, r.id);
+        if (pair<ORDER, NGB, true, false>(r, j, ok, st, eps2, t, dsmin, cand)) ngb.add(r.id);
       }
       if (dsmin < before) nnblk = -2 - cand;  // a later pair, strictly nearer: its address is exact
     }
@@ -557,7 +657,7 @@ __device__ __forceinline__ void wave_force(
   nnaddr = nnblk <= -2 ? -2 - nnblk : INT_MAX;
   if (nnblk >= 0) {
     bool found = false;
-    for (int u = 0; u < 16; ++u) {
+    for (int u = 0; u < SUB; ++u) {
       const int j = nnblk + u * Q;
       const Rec& r = rec[j];
       R dx, dy, dz;
@@ -568,7 +668,8 @@ __device__ __forceinline__ void wave_force(
     }
   }
 
-  if constexpr (NGB && PIPE) ngb_flush(pend, ngb_list, st.i);
+  if constexpr (NGB && PIPE) ngb_flush(pend, ngb.list, st.i);
+  if constexpr (NGB) ngb.finish();
   dsd = (double)dsmin;
   if constexpr (Q > 1) {
 #pragma unroll
@@ -585,7 +686,7 @@ __device__ __forceinline__ void wave_force(
   writer = ivalid && jsub == 0;
 }
 
-template <int ORDER, bool F64, int P, bool NGB, bool PIPE>
+template <int ORDER, bool F64, int P, bool NGB, bool PIPE, bool AHEAD>
 __global__ __launch_bounds__(256) void k_force(
     const typename RecOf<ORDER, F64>::T* __restrict__ rec, const int2* __restrict__ idr, const int nj,
     const double* __restrict__ ibuf, const int* __restrict__ iid, const CallDesc* __restrict__ cd,
@@ -603,7 +704,7 @@ __global__ __launch_bounds__(256) void k_force(
   const double* ih2 = ibuf + (ORDER >= ORDER_H6 ? 9 : 6) * (size_t)ni;
   // wave-uniform by construction; readfirstlane lets the compiler keep the
   // j-loop bookkeeping and (for P = 64) the j-record loads in SGPRs
-  const int wave = __builtin_amdgcn_readfirstlane(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6));
+  const int wave = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
   const int G = (ni + P - 1) / P;
   if (wave >= G * S) return;  // whole wave (a whole block when S % 4 == 0)
   // smajor: consecutive waves (a block's 4) share one j-range and so its
@@ -616,7 +717,7 @@ __global__ __launch_bounds__(256) void k_force(
   double dsd;
   int nnaddr, islot;
   bool writer;
-  wave_force<ORDER, F64, P, NGB, PIPE>(rec, idr, ipos, ivel, iacc, ih2, iid, g * P, min(P, ni - g * P), jb, je, eps2d,
+  wave_force<ORDER, F64, P, NGB, PIPE, AHEAD>(rec, idr, ipos, ivel, iacc, ih2, iid, g * P, min(P, ni - g * P), jb, je, eps2d,
                                  ngb_cnt, ngb_list, T, dsd, nnaddr, islot, writer);
   if (blockred) {
     // The block's waves are splits 4q..4q+3 of one i-group (S % 4 == 0, so
@@ -774,24 +875,16 @@ __global__ __launch_bounds__(256) void k_finalize_ens(FinalizeArgs f, EnsArgs a)
 }
 
 // ---------------------------------------------------------------------------
-// Finalize.  Fixed-order sums of the S partial rows of each i-particle, the
+// Finalize.  Fixed-order sums of the partial rows of each i-particle, the
 // nearest neighbour as the (ds2, address) minimum, the result row, and the
-// ascending sort of the neighbour list.  Two shapes:
-//   k_finalize_rows  one thread per i-particle (partials read coalesced over i),
-//                    followed by k_sort_lists (one wave per list);
-//   k_finalize_block one work-group per i-particle, threads striding over the
-//                    splits (few i-particles, many splits).
-// Result row of i-particle i, field-major (consecutive i of a wave write
-// consecutive doubles of each field: whole lines over PCIe).
+// ascending sort of the neighbour list.
+// Nearest neighbour and count of i-particle i.
 template <int ORDER, bool F64>
-__device__ __forceinline__ void write_row(const FinalizeArgs& a, int i, const double* T, double ds, int ad,
-                                          int cnt) {
+__device__ __forceinline__ void write_nn(const FinalizeArgs& a, int i, double ds, int ad, int cnt) {
   using Rec = typename RecOf<ORDER, F64>::T;
   constexpr int NF = nf<ORDER>();
   double* o = a.out + i;
   const size_t st = (size_t)a.ostride;
-#pragma unroll
-  for (int f = 0; f < NF; ++f) o[f * st] = T[f];
   const bool has = ad != INT_MAX;
   // the device returns ds2 rounded to float (kernels.cu:999-1002)
   o[NF * st] = has ? (double)(float)ds : INFINITY;
@@ -799,59 +892,125 @@ __device__ __forceinline__ void write_row(const FinalizeArgs& a, int i, const do
   o[(NF + 2) * st] = (double)cnt;
 }
 
-// Rank sort of c ids staged in s[0..c) by one wave, written to dst.
-__device__ __forceinline__ void wave_rank_sort(const int* s, int c, int lane, int* dst) {
-  for (int k = lane; k < c; k += 64) {
-    const int v = s[k];
-    int rank = 0;
-    for (int q = 0; q < c; ++q) {
-      const int u = s[q];
-      rank += (u < v) || (u == v && q < k);
-    }
-    dst[rank] = v;
-  }
+// Result row of i-particle i, field-major (consecutive i of a wave write
+// consecutive doubles of each field: whole lines over PCIe).
+template <int ORDER, bool F64>
+__device__ __forceinline__ void write_row(const FinalizeArgs& a, int i, const double* T, double ds, int ad,
+                                          int cnt) {
+  constexpr int NF = nf<ORDER>();
+  double* o = a.out + i;
+  const size_t st = (size_t)a.ostride;
+#pragma unroll
+  for (int f = 0; f < NF; ++f) o[f * st] = T[f];
+  write_nn<ORDER, F64>(a, i, ds, ad, cnt);
 }
 
-// Four consecutive lanes per i-particle: lane u sums rows u, u + 4, ... in
-// order, then the four sums combine as (S0 + S1) + (S2 + S3) (IEEE addition
-// commutes exactly, so every lane of the four holds the same value).
-template <int ORDER, bool F64>
-__device__ __forceinline__ void finalize_rows_block(const FinalizeArgs& a, int b) {
-  constexpr int NF = nf<ORDER>();
+// Rank sort of c ids staged in s[0..c) by one wave, written to dst.  s is 16-byte
+// aligned and padded to a multiple of four: a lane ranks its (up to four) ids
+// against four at a time, one LDS read for all of them (a full list of 256: 30 us
+// with one read per comparison).
+__device__ __forceinline__ void wave_rank_sort(const int* s, int c, int lane, int* dst) {
+  constexpr int M = NGB_CAP / 64;
+  int v[M], rank[M];
+#pragma unroll
+  for (int m = 0; m < M; ++m) {
+    v[m] = lane + 64 * m < c ? s[lane + 64 * m] : 0;
+    rank[m] = 0;
+  }
+  for (int q = 0; q < c; q += 4) {
+    const int4 w = *reinterpret_cast<const int4*>(s + q);
+    const int u[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+    for (int m = 0; m < M; ++m) {
+      if (64 * m >= c) break;  // uniform
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        rank[m] += q + e < c && (u[e] < v[m] || (u[e] == v[m] && q + e < lane + 64 * m)) ? 1 : 0;
+    }
+  }
+#pragma unroll
+  for (int m = 0; m < M; ++m)
+    if (lane + 64 * m < c) dst[rank[m]] = v[m];
+}
+
+// U threads per i-particle, 256 / U consecutive i-particles per work-group (a
+// row is read whole-line): thread u sums rows u, u + U, ... in order, the U sums
+// are added through LDS in a fixed order.  Bound by the latency of the row reads
+// and of the PCIe writes; U grows as ni falls so that few i-particles still have
+// many reads in flight (333 i-particles of 782 rows: 32 us with one work-group
+// per i-particle reading across rows).
+template <int ORDER, bool F64, int U>
+__device__ __forceinline__ void finalize_block(const FinalizeArgs& a, int b) {
+  constexpr int NF = nf<ORDER>(), I = 256 / U;
+  __shared__ double red[NF][256];
+  __shared__ double red_d[256];
+  __shared__ int red_a[256];
   const int ni = a.cd->ni;
-  const int t = b * 256 + threadIdx.x;
-  const int i = t >> 2, u = t & 3;
-  if (i >= ni) return;  // the four lanes of an i-particle leave together
+  const int t = threadIdx.x;
+  const int ii = t % I, u = t / I;
+  const int i = b * I + ii;
+  if (b * I >= ni) return;  // whole work-group (the grid may cover more i-particles)
   double T[NF];
 #pragma unroll
   for (int f = 0; f < NF; ++f) T[f] = 0.0;
   double ds = INFINITY;
   int ad = INT_MAX;
-  for (int s = u; s < a.S; s += 4) {
+  if (i < ni) {
+#pragma unroll 2
+    for (int s = u; s < a.S; s += U) {
 #pragma unroll
-    for (int f = 0; f < NF; ++f) T[f] += a.part[((size_t)f * a.S + s) * ni + i];
-    const double d = a.part_ds2[(size_t)s * ni + i];
-    const int ad2 = a.part_addr[(size_t)s * ni + i];
-    const bool take = (d < ds) || (d == ds && ad2 < ad);
-    ds = take ? d : ds;
-    ad = take ? ad2 : ad;
+      for (int f = 0; f < NF; ++f) T[f] += a.part[((size_t)f * a.S + s) * ni + i];
+      const double d = a.part_ds2[(size_t)s * ni + i];
+      const int ad2 = a.part_addr[(size_t)s * ni + i];
+      const bool take = (d < ds) || (d == ds && ad2 < ad);
+      ds = take ? d : ds;
+      ad = take ? ad2 : ad;
+    }
   }
 #pragma unroll
-  for (int m = 1; m < 4; m <<= 1) {
+  for (int f = 0; f < NF; ++f) red[f][t] = T[f];
+  red_d[t] = ds;
+  red_a[t] = ad;
+  __syncthreads();
+  // output o: field o / I of i-particle o % I, and last the nearest neighbour and
+  // count; L lanes each take every L-th of its U values
+  constexpr int L = U == 64 ? 4 : 1, OUT = (NF + 1) * I;
+  static_assert(L == 1 || L * OUT <= 256, "one pass");
+  for (int o = t / L; o < OUT; o += 256 / L) {
+    const int f = o / I, k = o % I, io = b * I + k, l = t % L;
+    if (f < NF) {
+      constexpr int C = U / L < 4 ? U / L : 4;  // chains
+      double v[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-    for (int f = 0; f < NF; ++f) T[f] += __shfl_xor(T[f], m);
-    const double od = __shfl_xor(ds, m);
-    const int oa = __shfl_xor(ad, m);
-    const bool take = (od < ds) || (od == ds && oa < ad);
-    ds = take ? od : ds;
-    ad = take ? oa : ad;
+      for (int q = 0; q < U / L; q += C)
+#pragma unroll
+        for (int c = 0; c < C; ++c) v[c] += red[f][((q + c) * L + l) * I + k];
+      double r = (v[0] + v[1]) + (v[2] + v[3]);
+#pragma unroll
+      for (int m = 1; m < L; m <<= 1) r += __shfl_xor(r, m);
+      if (l == 0 && io < ni) a.out[(size_t)f * a.ostride + io] = r;
+    } else {
+      double bd = red_d[l * I + k];
+      int ba = red_a[l * I + k];
+#pragma unroll
+      for (int q = 1; q < U / L; ++q) {
+        const double od = red_d[(q * L + l) * I + k];
+        const int oa = red_a[(q * L + l) * I + k];
+        const bool take = (od < bd) || (od == bd && oa < ba);
+        bd = take ? od : bd;
+        ba = take ? oa : ba;
+      }
+#pragma unroll
+      for (int m = 1; m < L; m <<= 1) {
+        const double od = __shfl_xor(bd, m);
+        const int oa = __shfl_xor(ba, m);
+        const bool take = (od < bd) || (od == bd && oa < ba);
+        bd = take ? od : bd;
+        ba = take ? oa : ba;
+      }
+      if (l == 0 && io < ni) write_nn<ORDER, F64>(a, io, bd, ba, a.ngb_on ? a.ngb_cnt[io] : 0);
+    }
   }
-  if (u == 0) write_row<ORDER, F64>(a, i, T, ds, ad, a.ngb_on ? a.ngb_cnt[i] : 0);
-}
-
-template <int ORDER, bool F64>
-__global__ __launch_bounds__(256) void k_finalize_rows(FinalizeArgs a) {
-  finalize_rows_block<ORDER, F64>(a, blockIdx.x);
 }
 
 // Host offset of i-particle i's list in a single-system call: its region's
@@ -885,7 +1044,7 @@ __device__ __forceinline__ void store_list(const FinalizeArgs& a, int i, const i
 // four lists of a work-group taking their offsets with one atomic on the
 // call's counter.
 __device__ __forceinline__ void sort_lists_block(const FinalizeArgs& a, int b) {
-  __shared__ int lst[4][NGB_CAP];
+  __shared__ __align__(16) int lst[4][NGB_CAP];
   __shared__ int srt[4][NGB_CAP];
   __shared__ int cnts[4];
   __shared__ int base;
@@ -917,81 +1076,10 @@ __global__ __launch_bounds__(256) void k_sort_lists(FinalizeArgs a) { sort_lists
 // Finalize and list sort in one launch (independent work: the sort only
 // reorders the lists, the finalize reads counts): the first nfin work-groups
 // finalize, the others sort; both roles are uniform per work-group.
-template <int ORDER, bool F64>
-__global__ __launch_bounds__(256) void k_finalize_rows_sort(FinalizeArgs a, int nfin) {
-  if ((int)blockIdx.x < nfin) finalize_rows_block<ORDER, F64>(a, blockIdx.x);
+template <int ORDER, bool F64, int U>
+__global__ __launch_bounds__(256) void k_finalize(FinalizeArgs a, int nfin) {
+  if ((int)blockIdx.x < nfin) finalize_block<ORDER, F64, U>(a, blockIdx.x);
   else sort_lists_block(a, blockIdx.x - nfin);
-}
-
-// One 256-thread block per i-particle: thread t sums the splits s = t, t+256, ...
-// in order, then a fixed-order tree over the 256 threads in LDS (deterministic).
-template <int ORDER, bool F64>
-__global__ __launch_bounds__(256) void k_finalize_block(FinalizeArgs a) {
-  constexpr int NF = nf<ORDER>();
-  __shared__ double shT[NF][256];
-  __shared__ double shD[256];
-  __shared__ int shA[256];
-  __shared__ int lst[NGB_CAP];
-  __shared__ int srt[NGB_CAP];
-  __shared__ int base;
-  const int t = threadIdx.x;
-  const int i = blockIdx.x;
-  const int ni = a.cd->ni;
-  if (i >= ni) return;  // whole block (the grid may cover more i-particles)
-  double T[NF];
-#pragma unroll
-  for (int f = 0; f < NF; ++f) T[f] = 0.0;
-  double ds = INFINITY;
-  int ad = INT_MAX;
-  for (int s = t; s < a.S; s += 256) {
-#pragma unroll
-    for (int f = 0; f < NF; ++f) T[f] += a.part[((size_t)f * a.S + s) * ni + i];
-    const double d = a.part_ds2[(size_t)s * ni + i];
-    const int ad2 = a.part_addr[(size_t)s * ni + i];
-    const bool take = (d < ds) || (d == ds && ad2 < ad);
-    ds = take ? d : ds;
-    ad = take ? ad2 : ad;
-  }
-#pragma unroll
-  for (int f = 0; f < NF; ++f) shT[f][t] = T[f];
-  shD[t] = ds;
-  shA[t] = ad;
-  __syncthreads();
-  for (int h = 128; h > 0; h >>= 1) {
-    if (t < h) {
-#pragma unroll
-      for (int f = 0; f < NF; ++f) shT[f][t] += shT[f][t + h];
-      const double od = shD[t + h];
-      const int oa = shA[t + h];
-      if ((od < shD[t]) || (od == shD[t] && oa < shA[t])) { shD[t] = od; shA[t] = oa; }
-    }
-    __syncthreads();
-  }
-  const int cnt = a.ngb_on ? a.ngb_cnt[i] : 0;
-  const int c = min(cnt, NGB_CAP);
-  if (t == 0) {
-    double R[NF];
-#pragma unroll
-    for (int f = 0; f < NF; ++f) R[f] = shT[f][0];
-    write_row<ORDER, F64>(a, i, R, shD[0], shA[0], cnt);
-    if (a.ngb_on && !a.inorder) {
-      base = c > 0 ? atomicAdd(a.pack_ctr, c) : 0;
-      a.list_off[i] = base;
-    }
-  }
-  if (a.ngb_on && a.inorder && t < 64) {  // uniform over the block; a whole wave
-    const int o = region_offset(a.ngb_cnt, i, t);
-    if (t == 0) {
-      base = o;
-      a.list_off[i] = o;
-    }
-  }
-  if (c == 0) return;  // uniform over the block
-  for (int k = t; k < c; k += 256) lst[k] = a.ngb_list[(size_t)i * NGB_CAP + k];
-  __syncthreads();
-  if (t < 64) wave_rank_sort(lst, c, t, srt);
-  __syncthreads();
-  store_list(a, i, srt, c, base, t, 256);
 }
 
 // ---------------------------------------------------------------------------
@@ -1076,21 +1164,28 @@ bool force_p_supported(int P) {
   return P == 64 || P == 32 || P == 16 || P == 8 || P == 4 || P == 2 || P == 1;
 }
 
-template <int OR, bool FP, int P>
-static void launch_force_p(hipStream_t s, const ForceArgs& a, const ForceConfig& c) {
-  using Rec = typename RecOf<OR, FP>::T;
+template <int OR, bool FP, int P, bool PIPE, bool AHEAD>
+static void launch_force_w(hipStream_t s, const ForceArgs& a, const ForceConfig& c) {
   const long G = (a.grid_ni + P - 1) / P;
-  const int nb = blocks_for(G * c.S, 4);
-  const Rec* rec = reinterpret_cast<const Rec*>(a.rec);
+  const dim3 nb(blocks_for(G * c.S, 4)), bs(256);
+  const auto* rec = reinterpret_cast<const typename RecOf<OR, FP>::T*>(a.rec);
 #define SAPK_FORCE_ARGS rec, a.idr, a.nj, a.ibuf, a.iid, a.cd, a.part, a.part_ds2, \
                         a.part_addr, a.ngb_cnt, a.ngb_list, c.S, c.jchunk, c.smajor, partial_rows(c) != c.S ? 1 : 0
-  if (a.ngb_on && c.pipe)
-    hipLaunchKernelGGL((k_force<OR, FP, P, true, true>), dim3(nb), dim3(256), 0, s, SAPK_FORCE_ARGS);
-  else if (a.ngb_on)
-    hipLaunchKernelGGL((k_force<OR, FP, P, true, false>), dim3(nb), dim3(256), 0, s, SAPK_FORCE_ARGS);
-  else
-    hipLaunchKernelGGL((k_force<OR, FP, P, false, false>), dim3(nb), dim3(256), 0, s, SAPK_FORCE_ARGS);
+  if (a.ngb_on) hipLaunchKernelGGL((k_force<OR, FP, P, true, PIPE, AHEAD>), nb, bs, 0, s, SAPK_FORCE_ARGS);
+  else hipLaunchKernelGGL((k_force<OR, FP, P, false, false, AHEAD>), nb, bs, 0, s, SAPK_FORCE_ARGS);
 #undef SAPK_FORCE_ARGS
+}
+
+// Lists with deferred id stores (c.pipe) have kernels of their own.  P = 64 takes
+// records ahead in FP64 always, in mixed precision where the launch shape says
+// so (choose_config).
+template <int OR, bool FP, int P>
+static void launch_force_p(hipStream_t s, const ForceArgs& a, const ForceConfig& c) {
+  if (c.pipe) return launch_force_w<OR, FP, P, true, false>(s, a, c);
+  if constexpr (P == 64) {
+    if (FP || c.ahead) return launch_force_w<OR, FP, P, false, true>(s, a, c);
+  }
+  if constexpr (P != 64 || !FP) launch_force_w<OR, FP, P, false, false>(s, a, c);
 }
 
 template <int OR, bool FP>
@@ -1118,19 +1213,15 @@ int launch_force(hipStream_t s, int order, bool f64, const ForceArgs& a, const F
 
 int launch_finalize(hipStream_t s, int order, bool f64, const FinalizeArgs& a) {
   if (a.grid_ni <= 0) return 0;
-  // rows: coalesced over i, best when many i-particles share few splits
   dispatch_op(order, f64, [&](auto OR, auto FP) {
     constexpr int O = decltype(OR)::value;
     constexpr bool F = decltype(FP)::value;
-    if (a.rows) {
-      const int nfin = blocks_for(4L * a.grid_ni, 256);
-      if (a.ngb_on)
-        hipLaunchKernelGGL((k_finalize_rows_sort<O, F>), dim3(nfin + blocks_for(a.grid_ni, 4)), dim3(256), 0, s, a,
-                           nfin);
-      else
-        hipLaunchKernelGGL((k_finalize_rows<O, F>), dim3(nfin), dim3(256), 0, s, a);
-    } else {
-      hipLaunchKernelGGL((k_finalize_block<O, F>), dim3(a.grid_ni), dim3(256), 0, s, a);
+    const int nsort = a.ngb_on ? blocks_for(a.grid_ni, 4) : 0;
+    const int nfin = blocks_for((long)a.U * a.grid_ni, 256);
+    switch (a.U) {
+      case 64: hipLaunchKernelGGL((k_finalize<O, F, 64>), dim3(nfin + nsort), dim3(256), 0, s, a, nfin); break;
+      case 16: hipLaunchKernelGGL((k_finalize<O, F, 16>), dim3(nfin + nsort), dim3(256), 0, s, a, nfin); break;
+      default: hipLaunchKernelGGL((k_finalize<O, F, 4>), dim3(nfin + nsort), dim3(256), 0, s, a, nfin); break;
     }
   });
   return hip_status();
