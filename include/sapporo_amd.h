@@ -136,9 +136,9 @@ float sapamd_last_finalize_ms(sapamd_engine *e);
  * finalize kernel */
 float sapamd_last_device_ms(sapamd_engine *e);
 int sapamd_last_config(sapamd_engine *e, int *P, int *S, int *jchunk);
-/* Launch-shape table (sapporo2_amd/autotune.py output; loaded at open from
- * $SAPPORO2_AMD_TUNE or tune/<arch>.txt beside the library).  Returns the
- * number of entries read (0: heuristic shapes). */
+/* Launch-shape table (sapporo2_amd/autotune.py output) instead of the built-in
+ * rule; loaded at open from $SAPPORO2_AMD_TUNE when that is set.  Returns the
+ * number of entries read (0: the built-in rule). */
 int sapamd_load_tuning(sapamd_engine *e, const char *path);
 int sapamd_tuning_entries(sapamd_engine *e);
 int sapamd_num_cus(sapamd_engine *e);

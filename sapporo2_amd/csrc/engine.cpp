@@ -2,7 +2,6 @@
 #include "engine.h"
 #include "hostpool.h"
 
-#include <dlfcn.h>
 #include <immintrin.h>
 
 #include <algorithm>
@@ -35,6 +34,7 @@ constexpr int WAVES_PER_SIMD_TARGET = 32;   // several dispatch rounds balance b
 constexpr int MIN_ITERS_PER_LANE = 16;
 constexpr int MIN_J_PER_SPLIT = 512;
 // Launch shapes of lane shape P = 64 (choose_config)
+constexpr int SMALL_ROWS = 512;
 constexpr long MIN_CHUNK = 64, MAX_CHUNK = 256, MAX_WAVES = 65536;
 // Mixed launches of at most this many waves (4 per SIMD) take their records
 // ahead: one wave alone waits ~190 ns per pair for scalar loads, 80 with them
@@ -133,22 +133,8 @@ int Engine::open(int device, int order, int precision) {
   hipDeviceProp_t prop;
   HIPCHK(hipGetDeviceProperties(&prop, device_), "hipGetDeviceProperties");
   cus_ = prop.multiProcessorCount > 0 ? prop.multiProcessorCount : 256;
-  arch_ = prop.gcnArchName;
-  arch_ = arch_.substr(0, arch_.find(':'));
-  {
-    // tuned launch shapes: $SAPPORO2_AMD_TUNE, else tune/<arch>.txt beside the library
-    std::string path;
-    if (const char* env = getenv("SAPPORO2_AMD_TUNE")) {
-      path = env;
-    } else {
-      Dl_info info;
-      if (dladdr(reinterpret_cast<void*>(&sapk::launch_force), &info) && info.dli_fname) {
-        path = info.dli_fname;
-        path = path.substr(0, path.rfind('/') + 1) + "tune/" + arch_ + ".txt";
-      }
-    }
-    if (!path.empty()) load_tuning(path.c_str());
-  }
+  // a launch-shape table instead of the built-in rule, on request
+  if (const char* env = getenv("SAPPORO2_AMD_TUNE")) load_tuning(env);
   HIPCHK(hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking), "hipStreamCreate");
   HIPCHK(hipEventCreateWithFlags(&ev_done_, hipEventDisableTiming), "hipEventCreate");
   HIPCHK(hipEventCreate(&ev_d0_), "hipEventCreate");
@@ -162,6 +148,9 @@ int Engine::open(int device, int order, int precision) {
   for (auto& s : stage_) HIPCHK(hipEventCreateWithFlags(&s.ev, hipEventDisableTiming), "hipEventCreate");
   HIPCHK(hipEventCreateWithFlags(&ev_desc_, hipEventDisableTiming), "hipEventCreate");
   HIPCHK(dmalloc(&pack_ctr_d_, 1), "pack counter");
+  HIPCHK(dmalloc(&cnt_small_d_, 2 * SMALL_NI), "small-call counters");
+  HIPCHK(hipMemsetAsync(cnt_small_d_, 0, 2 * SMALL_NI * sizeof(int), stream_), "memset");
+  small_flip_ = false;
   HIPCHK(hmap(&call_h_, &call_hd_, CALL_DOUBLES, true), "pinned call block");
   HIPCHK(dmalloc(&call_d_, CALL_DOUBLES), "call block");
   desc_h_ = reinterpret_cast<CallDesc*>(call_h_);
@@ -216,6 +205,7 @@ int Engine::close() {
   hfree(loff_h_); loff_hd_ = nullptr;
   hfree(packed_h_); packed_hd_ = nullptr; packed_cap_ = 0;
   dfree(pack_ctr_d_);
+  dfree(cnt_small_d_);
   dfree(cnt_d_); dfree(list_d_); list_cap_ = 0;
   slot_lists_h_.clear();
   dfree(gather_d_); gather_cap_ = 0;
@@ -649,17 +639,25 @@ int Engine::prep(int pred_j1, int call_bytes, int ni_reset, bool by_call) {
   if (launch_prep(stream_, order_, f64_, a) != 0) return fail("prep launch", hipGetLastError());
   if (ev) HIPCHK(hipEventRecord(ev_p1_, stream_), "event");
   timed_predict_ = ev && pred_j1 > 0;
-  if (n > 0) {
-    if (!by_call) {
-      HIPCHK(hipEventRecord(sg.ev, stream_), "event");
-      ++rec_seq_;
-    }
+  if (n > 0 && by_call) {
+    stage_to_call();
+  } else if (n > 0) {
+    HIPCHK(hipEventRecord(sg.ev, stream_), "event");
     sg.busy = true;
-    sg.by_call = by_call;
-    sg.seq = by_call ? rec_seq_ + 1 : rec_seq_;  // the call's completion is the next event recorded
+    sg.by_call = false;
+    sg.seq = ++rec_seq_;
     hand_over();
   }
   return 0;
+}
+
+// The current stage is read by the call being launched: it is free when that has
+// completed (its completion is numbered next).
+void Engine::stage_to_call() {
+  Stage& sg = stage_[cur_];
+  sg.busy = sg.by_call = true;
+  sg.seq = rec_seq_ + 1;
+  hand_over();
 }
 
 // Work-groups of the scatter launch: grid-stride over the descriptor's counts,
@@ -731,10 +729,12 @@ static int ceil_log2(long v) {
   return l;
 }
 
-// Launch shape: the tuned table's entry for (order, precision, neighbour lists,
-// active-count bucket, nearest nj) when present; otherwise P i-particles per
-// wave (64 unless fewer are active) and S j-splits for ~WAVES_PER_SIMD_TARGET
-// waves per SIMD with at least MIN_J_PER_SPLIT j per split.
+// Launch shape: an explicitly loaded table's entry for (order, precision,
+// neighbour lists, active-count bucket, nearest nj); otherwise, by the active
+// count, the small-call kernel or lane shape P = 64 with the splits below.
+// Overrides and the optional launch modes keep the general shapes: P i-particles
+// per wave (64 unless fewer are active), j-splits for ~WAVES_PER_SIMD_TARGET
+// waves per SIMD with at least MIN_J_PER_SPLIT j each.
 ForceConfig Engine::choose_config(int ni, int nj, bool ngb) const {
   int P = 64;
   if (ni < 64) {
@@ -742,7 +742,8 @@ ForceConfig Engine::choose_config(int ni, int nj, bool ngb) const {
     while (P < ni) P <<= 1;
   }
   long jchunk_t = 0;
-  if (!tune_.empty() && ovr_P_ <= 0 && ovr_S_ <= 0) {
+  const bool plain = ovr_P_ <= 0 && ovr_S_ <= 0;
+  if (!tune_.empty() && plain) {
     const int li = ceil_log2(ni), lj = ceil_log2(nj);
     const int prec = f64_ ? PREC_DOUBLE : PREC_DS;
     const TuneEntry* best = nullptr;
@@ -755,11 +756,19 @@ ForceConfig Engine::choose_config(int ni, int nj, bool ngb) const {
       jchunk_t = 1L << best->jlog;
     }
   }
+  if (plain && jchunk_t == 0 && !ovr_smajor_ && !ovr_pipe_) {
+    if (ni <= SMALL_NI) {
+      // At most SMALL_ROWS work-groups, each one row for the finalize to read.
+      const int ntiles = (nj + 255) / 256, tiles = (ntiles + SMALL_ROWS - 1) / SMALL_ROWS;
+      return ForceConfig{P, (ntiles + tiles - 1) / tiles, tiles * 256, 0, 0, 0, 1};
+    }
+    P = 64;
+  }
   if (ovr_P_ > 0 && force_p_supported(ovr_P_)) P = ovr_P_;
   const int Q = 64 / P;
   const long G = (ni + P - 1) / P;
   long S;
-  if (P == 64 && ni > 32) {
+  if (P == 64 && plain && jchunk_t == 0) {
     // One round of waves (8 per SIMD mixed, 5 in FP64) while that leaves a wave
     // MIN_CHUNK j or more; the fixed cost of a wave (its i-particles, cold
     // records, epilogue) is then small against its pairs.  More i-groups take
@@ -795,7 +804,7 @@ ForceConfig Engine::choose_config(int ni, int nj, bool ngb) const {
   const long whole = P == 64 && S >= 256 ? 32 : 4;
   S = (S + whole - 1) / whole * whole;
   const int ahead = G * S <= AHEAD_WAVES ? 1 : 0;
-  return ForceConfig{P, (int)S, (int)jchunk, ovr_smajor_, ovr_pipe_, ahead};
+  return ForceConfig{P, (int)S, (int)jchunk, ovr_smajor_, ovr_pipe_, ahead, 0};
 }
 
 // i-particle-sized buffers (ensemble inputs, host-mapped result rows and list
@@ -1155,7 +1164,7 @@ int Engine::start_grav_calc_clusters(int ni, const int* cluster, const int* id, 
   ngb_on_last_ = ngb_on;
   ni_last_ = ni;
   nj_last_ = cl_total_;
-  last_cfg_ = ForceConfig{0, nitems, (int)jch64, 0, 0, 0};
+  last_cfg_ = ForceConfig{0, nitems, (int)jch64, 0, 0, 0, 0};
   jhost_valid_ = false;
   return 0;
 }
@@ -1226,8 +1235,12 @@ int Engine::start_grav_calc(int nj, int ni, const int* id, const double (*xi)[3]
     if (launch_call_graph(grid_ni, nj, cfg, ngb_on, predict, sblocks, finalize_threads(bucket)) != 0) return -1;
     timed_predict_ = timed_force_ = false;
   } else {
-    if (prep(predict ? nj : 0, (int)nbytes, ngb_on ? ni : 0, true) != 0) return -1;
-    if (enqueue_force(grid_ni, nj, cfg, ngb_on, finalize_threads(bucket)) != 0) return -1;
+    if (cfg.small && predict && !new_ids_ && nstaged_ <= SMALL_UPD && flushed_ == 0 && max_addr_ < nj) {
+      if (call_small(nj, cfg, ngb_on, bucket) != 0) return -1;
+    } else {
+      if (prep(predict ? nj : 0, (int)nbytes, ngb_on ? ni : 0, true) != 0) return -1;
+      if (enqueue_force(grid_ni, nj, cfg, ngb_on, finalize_threads(bucket)) != 0) return -1;
+    }
     timed_force_ = timing_;
   }
   if (timing_) HIPCHK(hipEventRecord(ev_d1_, stream_), "event");
@@ -1243,6 +1256,43 @@ int Engine::start_grav_calc(int nj, int ni, const int* id, const double (*xi)[3]
   nj_last_ = nj;
   last_cfg_ = cfg;
   jhost_valid_ = false;
+  return 0;
+}
+
+// A call of at most SMALL_NI i-particles in two launches: updates, prediction and
+// forces, then the finalize.  Inputs are read from pinned memory; the neighbour
+// counters alternate between two buffers, each cleared while the other is in use.
+int Engine::call_small(int nj, const ForceConfig& cfg, bool ngb_on, int bucket) {
+  const int ni = desc_h_->ni;
+  int* cnt = cnt_small_d_ + (small_flip_ ? SMALL_NI : 0);
+  const Stage& sg = stage_[cur_];
+  const ptrdiff_t alias = reinterpret_cast<char*>(call_hd_) - reinterpret_cast<char*>(call_d_);
+  SmallArgs a{};
+  a.f = force_args(ni, nj, ngb_on);
+  a.f.ibuf = reinterpret_cast<const double*>(reinterpret_cast<const char*>(call_ibuf_d_) + alias);
+  a.f.iid = reinterpret_cast<const int*>(reinterpret_cast<const char*>(call_iid_d_) + alias);
+  a.f.cd = reinterpret_cast<const CallDesc*>(call_hd_);
+  a.f.ngb_cnt = cnt;
+  a.tiles = cfg.jchunk / 256;
+  a.st = st_;
+  a.rows_h = sg.dd;
+  a.bits = sg.bits_d;
+  a.nbits = nstaged_ > 0 ? (int)std::min<size_t>(sg.words * 32, INT_MAX) : 0;
+  a.nupd = nstaged_;
+  a.ti = t_i_;
+  a.cnt_clear = cnt_small_d_ + (small_flip_ ? 0 : SMALL_NI);
+  small_flip_ = !small_flip_;
+  timed_scatter_ = timed_predict_ = false;
+  if (timing_) HIPCHK(hipEventRecord(ev_f0_, stream_), "event");
+  if (launch_force_small(stream_, order_, f64_, a, cfg, true) != 0) return fail("force launch", hipGetLastError());
+  if (timing_) HIPCHK(hipEventRecord(ev_f1_, stream_), "event");
+  FinalizeArgs fz = finalize_args(ni, ngb_on);
+  fz.cd = a.f.cd;
+  fz.ngb_cnt = cnt;
+  fz.S = partial_rows(cfg);
+  fz.U = finalize_threads(bucket);
+  if (launch_finalize(stream_, order_, f64_, fz) != 0) return fail("finalize launch", hipGetLastError());
+  if (nstaged_ > 0) stage_to_call();
   return 0;
 }
 
@@ -1268,8 +1318,7 @@ int Engine::enqueue_call(int grid_ni, int nj, const ForceConfig& cfg, bool ngb_o
   return enqueue_force(grid_ni, nj, cfg, ngb_on, fin_u);
 }
 
-// Force and finalize kernels of a call.
-int Engine::enqueue_force(int grid_ni, int nj, const ForceConfig& cfg, bool ngb_on, int fin_u) {
+ForceArgs Engine::force_args(int grid_ni, int nj, bool ngb_on) const {
   ForceArgs fa{};
   fa.rec = st_.rec;
   fa.idr = st_.idr;
@@ -1284,6 +1333,12 @@ int Engine::enqueue_force(int grid_ni, int nj, const ForceConfig& cfg, bool ngb_
   fa.ngb_cnt = cnt_d_;
   fa.ngb_list = list_d_;
   fa.ngb_on = ngb_on ? 1 : 0;
+  return fa;
+}
+
+// Force and finalize kernels of a call.
+int Engine::enqueue_force(int grid_ni, int nj, const ForceConfig& cfg, bool ngb_on, int fin_u) {
+  const ForceArgs fa = force_args(grid_ni, nj, ngb_on);
   const bool ev = timing_ && !capturing_;
   if (ev) HIPCHK(hipEventRecord(ev_f0_, stream_), "event");
   if (launch_force(stream_, order_, f64_, fa, cfg) != 0) return fail("force launch", hipGetLastError());
@@ -1380,7 +1435,7 @@ constexpr size_t MAX_GRAPHS = 64;
 // whose buffers were reallocated are dropped when next seen).
 int Engine::launch_call_graph(int grid_ni, int nj, const ForceConfig& cfg, bool ngb_on, bool predict, int sblocks,
                               int fin_u) {
-  const GraphKey key{grid_ni, nj, cfg.P, cfg.S, cfg.jchunk, cfg.smajor, cfg.pipe, cfg.ahead, ngb_on ? 1 : 0,
+  const GraphKey key{grid_ni, nj, cfg.P, cfg.S, cfg.jchunk, cfg.smajor, cfg.pipe, cfg.ahead + 2 * cfg.small, ngb_on ? 1 : 0,
                      predict ? 1 : 0, sblocks, fin_u, gen_};
   for (auto& e : graph_cache_) {
     if (e.key == key) {

@@ -146,6 +146,9 @@ class Engine {
   int scatter_blocks(int nupd, int ni_reset) const;
   int enqueue_call(int grid_ni, int nj, const sapk::ForceConfig& cfg, bool ngb_on, bool predict,
                    int sblocks, int fin_u);
+  sapk::ForceArgs force_args(int grid_ni, int nj, bool ngb_on) const;
+  int call_small(int nj, const sapk::ForceConfig& cfg, bool ngb_on, int bucket);
+  void stage_to_call();
   int enqueue_force(int grid_ni, int nj, const sapk::ForceConfig& cfg, bool ngb_on, int fin_u);
   int launch_call_graph(int grid_ni, int nj, const sapk::ForceConfig& cfg, bool ngb_on, bool predict,
                         int sblocks, int fin_u);
@@ -210,6 +213,7 @@ class Engine {
   int* loff_h_ = nullptr; int* loff_hd_ = nullptr;
   int* packed_h_ = nullptr; int* packed_hd_ = nullptr; long packed_cap_ = 0;
   int* pack_ctr_d_ = nullptr;
+  int* cnt_small_d_ = nullptr; bool small_flip_ = false;  // neighbour counters of small calls, two buffers
   int* cnt_d_ = nullptr; int* list_d_ = nullptr; int list_cap_ = 0;
   std::vector<int> slot_lists_h_;   // device list slots read back when the packed lists did not fit
   bool lists_in_slots_ = false;     // lists read back from the device slots (packed overflow)
@@ -222,7 +226,7 @@ class Engine {
   bool timed_predict_ = false, timed_force_ = false;
   bool capturing_ = false;
   int ni_last_ = 0, nj_last_ = 0;
-  sapk::ForceConfig last_cfg_{64, 1, 1, 0, 0, 0};
+  sapk::ForceConfig last_cfg_{64, 1, 1, 0, 0, 0, 0};
   bool timing_ = false;
   int ovr_P_ = 0, ovr_S_ = 0, ovr_smajor_ = 0, ovr_pipe_ = 0;
 
@@ -267,7 +271,7 @@ class Engine {
 
   struct TuneEntry { int order, prec, ngb, li, lj, P, jlog; };
   std::vector<TuneEntry> tune_;
-  std::string tune_path_, arch_;
+  std::string tune_path_;
 
   // read-back cache of the j-store (predicted and raw state)
   bool jhost_valid_ = false;

@@ -146,11 +146,27 @@ struct ForceArgs {
   int ngb_on;            // neighbour search enabled (some h2 > 0)
 };
 
+// k_force_small: at most SMALL_NI i-particles; with the prediction in the same
+// launch (pred), also the staged updates, at most SMALL_UPD, all at addresses
+// below f.nj and none changing an id.  f.cd, f.ibuf and f.iid may be host-mapped.
+constexpr int SMALL_NI = 32, SMALL_UPD = 256;
+struct SmallArgs {
+  ForceArgs f;
+  int tiles;              // tiles of 256 j per work-group
+  StoreView st;           // pred from here on
+  const double* rows_h;   // staged rows, host-mapped
+  const unsigned* bits;   // their addresses as a bit set of nbits, host-mapped
+  int nbits, nupd;
+  double ti;
+  int* cnt_clear;         // SMALL_NI counters cleared for the next call of this kind
+};
+
 // Launch geometry of one force call: each wave owns P i-particles and Q = 64/P
 // j-lanes per i-particle over one of S contiguous j-ranges of jchunk.
 // smajor: wave-to-split mapping; pipe: neighbour-id stores deferred by one group;
-// ahead (P = 64): records loaded ahead of the pairs.
-struct ForceConfig { int P; int S; int jchunk; int smajor; int pipe; int ahead; };
+// ahead (P = 64): records loaded ahead of the pairs.  small: k_force_small, S
+// work-groups of jchunk j (whole tiles of 256), one partial row each.
+struct ForceConfig { int P; int S; int jchunk; int smajor; int pipe; int ahead; int small; };
 
 // Iterations of a lane that the pair loop takes at a time; a j-split is a whole
 // number of them (SUB * Q j), except for what the last split has left.
@@ -159,14 +175,14 @@ constexpr int FORCE_SUB = 16;
 // Partial-sum rows a force launch writes per i-particle.  With S a multiple of
 // 4 and split-minor wave order the 4 waves of a work-group are 4 consecutive
 // splits of one i-group; they combine their sums in LDS and write one row.
-inline int partial_rows(const ForceConfig& c) { return (c.S % 4 == 0 && !c.smajor) ? c.S / 4 : c.S; }
+inline int partial_rows(const ForceConfig& c) { return (c.S % 4 == 0 && !c.smajor && !c.small) ? c.S / 4 : c.S; }
 
 // Threads per i-particle of the finalize for a power-of-two bucket of ni (the
 // shape decides the order of the sums, so direct, replayed and allocation-free
 // calls of one ni take the same).  A launch of ~16384 threads or more keeps the
 // row reads in flight: with 4 threads each, 1000 i-particles of 128 rows took
 // 23 us.
-constexpr int finalize_threads(int bucket) { return bucket > 4096 ? 4 : bucket > 512 ? 16 : 64; }
+constexpr int finalize_threads(int bucket) { return bucket > 4096 ? 4 : bucket > 512 ? 16 : bucket > 32 ? 64 : 256; }
 
 // Results and neighbour lists go straight to host-mapped pinned memory (no
 // copy command): field-major result rows out[f * ostride + i], and each sorted
@@ -226,6 +242,7 @@ int launch_scatter(hipStream_t s, int order, bool f64, const ScatterArgs& a);
 int launch_predict(hipStream_t s, int order, bool f64, const PredictArgs& a);
 int launch_prep(hipStream_t s, int order, bool f64, const PrepArgs& a);
 int launch_force(hipStream_t s, int order, bool f64, const ForceArgs& a, const ForceConfig& c);
+int launch_force_small(hipStream_t s, int order, bool f64, const SmallArgs& a, const ForceConfig& c, bool pred);
 int launch_finalize(hipStream_t s, int order, bool f64, const FinalizeArgs& a);
 // Ensemble force + finalize (+ list sort) over a work table whose first n64
 // items have lane shape P = 64; one single-wave work-group per item.  Without

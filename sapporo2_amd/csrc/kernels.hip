@@ -53,11 +53,11 @@ __device__ __forceinline__ DSF to_ds(double x) {
 __device__ __forceinline__ void put_pos(double& dst, double x) { dst = x; }
 __device__ __forceinline__ void put_pos(DSF& dst, double x) { dst = to_ds(x); }
 
-// Write the working-precision record of particle j from FP64 values.
+// Working-precision record from FP64 values.
 template <int ORDER, bool F64>
-__device__ __forceinline__ void put_rec(void* base, int j, double x, double y, double z, double m,
-                                        double vx, double vy, double vz, double ax, double ay,
-                                        double az, int id) {
+__device__ __forceinline__ typename RecOf<ORDER, F64>::T make_rec(double x, double y, double z, double m, double vx,
+                                                                  double vy, double vz, double ax, double ay,
+                                                                  double az, int id) {
   using Rec = typename RecOf<ORDER, F64>::T;
   using R = typename std::conditional<F64, double, float>::type;
   Rec r{};
@@ -65,7 +65,25 @@ __device__ __forceinline__ void put_rec(void* base, int j, double x, double y, d
   r.m = (R)m; r.vx = (R)vx; r.vy = (R)vy; r.vz = (R)vz;
   if constexpr (ORDER >= ORDER_H6) { r.ax = (R)ax; r.ay = (R)ay; r.az = (R)az; }
   r.id = id;
-  reinterpret_cast<Rec*>(base)[j] = r;
+  return r;
+}
+
+// Write the predicted state of address j: the working-precision record and, in
+// mixed precision, the FP64 state kept for read-back.  Returns the record.
+template <int ORDER, bool F64>
+__device__ __forceinline__ typename RecOf<ORDER, F64>::T put_pred(const StoreView& st, int j, const double p[3], const double v[3],
+                                         const double ac[3], double m, int id) {
+  const size_t cap = (size_t)st.cap;
+  const auto r = make_rec<ORDER, F64>(p[0], p[1], p[2], m, v[0], v[1], v[2], ac[0], ac[1], ac[2], id);
+  reinterpret_cast<typename RecOf<ORDER, F64>::T*>(st.rec)[j] = r;
+  if constexpr (!F64) {
+    st.ppos[j] = p[0]; st.ppos[cap + j] = p[1]; st.ppos[2 * cap + j] = p[2];
+    st.pvel[j] = v[0]; st.pvel[cap + j] = v[1]; st.pvel[2 * cap + j] = v[2];
+    if constexpr (ORDER >= ORDER_H6) {
+      st.pacc[j] = ac[0]; st.pacc[cap + j] = ac[1]; st.pacc[2 * cap + j] = ac[2];
+    }
+  }
+  return r;
 }
 
 // ---------------------------------------------------------------------------
@@ -92,17 +110,10 @@ __global__ __launch_bounds__(256) void k_scatter(ScatterArgs a) {
     // predicted = raw for updated particles (kernels.cu:281-298), unless the
     // predictor that follows rewrites this address anyway
     if (addr < a.pred_j1) continue;
-    double ax = 0, ay = 0, az = 0;
-    if constexpr (ORDER >= ORDER_H6) { ax = u[RF_AX]; ay = u[RF_AY]; az = u[RF_AZ]; }
-    put_rec<ORDER, F64>(a.st.rec, addr, u[RF_X], u[RF_Y], u[RF_Z], u[RF_M], u[RF_VX], u[RF_VY],
-                        u[RF_VZ], ax, ay, az, id);
-    if constexpr (!F64) {
-      a.st.ppos[addr] = u[RF_X]; a.st.ppos[cap + addr] = u[RF_Y]; a.st.ppos[2 * cap + addr] = u[RF_Z];
-      a.st.pvel[addr] = u[RF_VX]; a.st.pvel[cap + addr] = u[RF_VY]; a.st.pvel[2 * cap + addr] = u[RF_VZ];
-      if constexpr (ORDER >= ORDER_H6) {
-        a.st.pacc[addr] = ax; a.st.pacc[cap + addr] = ay; a.st.pacc[2 * cap + addr] = az;
-      }
-    }
+    const double p[3] = {u[RF_X], u[RF_Y], u[RF_Z]}, v[3] = {u[RF_VX], u[RF_VY], u[RF_VZ]};
+    double ac[3] = {0, 0, 0};
+    if constexpr (ORDER >= ORDER_H6) { ac[0] = u[RF_AX]; ac[1] = u[RF_AY]; ac[2] = u[RF_AZ]; }
+    put_pred<ORDER, F64>(a.st, addr, p, v, ac, u[RF_M], id);
   }
 }
 
@@ -145,22 +156,6 @@ __device__ __forceinline__ void tile_id_range(const StoreView& st, int j) {
     hi = max(hi, __shfl_xor(hi, m));
   }
   if ((threadIdx.x & 63) == 0 && j < st.cap) st.idr[j / JTILE] = make_int2(lo, hi);
-}
-
-// Write the predicted state of address j: the working-precision record and, in
-// mixed precision, the FP64 state kept for read-back.
-template <int ORDER, bool F64>
-__device__ __forceinline__ void put_pred(const StoreView& st, int j, const double p[3], const double v[3],
-                                         const double ac[3], double m, int id) {
-  const size_t cap = (size_t)st.cap;
-  put_rec<ORDER, F64>(st.rec, j, p[0], p[1], p[2], m, v[0], v[1], v[2], ac[0], ac[1], ac[2], id);
-  if constexpr (!F64) {
-    st.ppos[j] = p[0]; st.ppos[cap + j] = p[1]; st.ppos[2 * cap + j] = p[2];
-    st.pvel[j] = v[0]; st.pvel[cap + j] = v[1]; st.pvel[2 * cap + j] = v[2];
-    if constexpr (ORDER >= ORDER_H6) {
-      st.pacc[j] = ac[0]; st.pacc[cap + j] = ac[1]; st.pacc[2 * cap + j] = ac[2];
-    }
-  }
 }
 
 template <int ORDER, bool F64>
@@ -271,6 +266,23 @@ struct IState {
   R vx, vy, vz, ax, ay, az, h2;
   int id, i;
 };
+
+template <int ORDER, typename R, bool NGB>
+__device__ __forceinline__ IState<ORDER, R> load_i(const double* __restrict__ ipos, const double* __restrict__ ivel,
+                                                   const double* __restrict__ iacc, const double* __restrict__ ih2,
+                                                   const int* __restrict__ iid, int il, bool valid) {
+  IState<ORDER, R> st;
+  get_pos(st.x, ipos[3 * il]); get_pos(st.y, ipos[3 * il + 1]); get_pos(st.z, ipos[3 * il + 2]);
+  st.vx = (R)ivel[3 * il]; st.vy = (R)ivel[3 * il + 1]; st.vz = (R)ivel[3 * il + 2];
+  st.ax = st.ay = st.az = R(0);
+  if constexpr (ORDER >= ORDER_H6) {
+    st.ax = (R)iacc[3 * il]; st.ay = (R)iacc[3 * il + 1]; st.az = (R)iacc[3 * il + 2];
+  }
+  st.h2 = (NGB && valid) ? (R)ih2[il] : R(-1);
+  st.id = iid[il];
+  st.i = il;
+  return st;
+}
 
 template <typename R> __device__ __forceinline__ R minR(R a, R b);
 template <> __device__ __forceinline__ float minR<float>(float a, float b) { return __builtin_fminf(a, b); }
@@ -557,16 +569,7 @@ __device__ __forceinline__ void wave_force(
   const bool ivalid = islot < icount;
   const int il = i0 + (ivalid ? islot : 0);
 
-  IState<ORDER, R> st;
-  get_pos(st.x, ipos[3 * il]); get_pos(st.y, ipos[3 * il + 1]); get_pos(st.z, ipos[3 * il + 2]);
-  st.vx = (R)ivel[3 * il]; st.vy = (R)ivel[3 * il + 1]; st.vz = (R)ivel[3 * il + 2];
-  st.ax = st.ay = st.az = R(0);
-  if constexpr (ORDER >= ORDER_H6) {
-    st.ax = (R)iacc[3 * il]; st.ay = (R)iacc[3 * il + 1]; st.az = (R)iacc[3 * il + 2];
-  }
-  st.h2 = (NGB && ivalid) ? (R)ih2[il] : R(-1);
-  st.id = iid[il];
-  st.i = il;
+  const IState<ORDER, R> st = load_i<ORDER, R, NGB>(ipos, ivel, iacc, ih2, iid, il, ivalid);
   const R eps2 = (R)eps2d;
 
 #pragma unroll
@@ -772,6 +775,136 @@ __global__ __launch_bounds__(256) void k_force(
   }
 }
 
+// Force kernel of at most SMALL_NI i-particles: a work-group takes tiles of 256
+// j, one thread each, into LDS; then each of its waves sums its 64 j of a tile
+// for the i-particles, P = the power of two above ni of them on the lanes and
+// Q = 64 / P j at a time.  One partial row per work-group.  PRED: the thread's j
+// is predicted here (and updated first if it is among the staged rows), so that
+// a call is this launch and the finalize; otherwise its record is read.  The
+// tiles and the order of the sums are the same in both, and do not depend on the
+// updates.  Bound by launch, PCIe and memory latency: the pairs of 24 x 131072
+// take 2 us at the full rate.
+template <int ORDER, bool F64, bool NGB, bool PRED>
+__global__ __launch_bounds__(256) void k_force_small(SmallArgs a) {
+  using R = typename std::conditional<F64, double, float>::type;
+  using Rec = typename RecOf<ORDER, F64>::T;
+  constexpr int NF = nf<ORDER>(), NR = raw_fields(ORDER) + 1;
+  __shared__ __align__(16) Rec tile[256];
+  __shared__ double red[4][NF][SMALL_NI];
+  __shared__ double red_d[4][SMALL_NI];
+  __shared__ int red_a[4][SMALL_NI];
+  __shared__ int row_of[256];
+  const int t = threadIdx.x, w = t >> 6, lane = t & 63, b = blockIdx.x;
+  const int ni = min(a.f.cd->ni, SMALL_NI), nj = a.f.nj;
+  const R eps2 = (R)a.f.cd->eps2;
+  const int lp = ni > 1 ? 32 - __clz(ni - 1) : 0, P = 1 << lp;
+  const int islot = lane & (P - 1), jsub = lane >> lp;
+  const double* ib = a.f.ibuf;
+  const IState<ORDER, R> st =
+      load_i<ORDER, R, NGB>(ib, ib + 3 * ni, ib + 6 * ni, ib + (ORDER >= ORDER_H6 ? 9 : 6) * ni, a.f.iid,
+                            islot < ni ? islot : 0, islot < ni);
+  NgbList ngb{a.f.ngb_cnt, a.f.ngb_list, st.i, -1};
+  double T[NF];
+#pragma unroll
+  for (int f = 0; f < NF; ++f) T[f] = 0.0;
+  R dsmin = R(INFINITY);
+  int nnaddr = INT_MAX;
+  if constexpr (PRED) {
+    // the other buffer of counters, for the next call of this kind
+    if (b == 0 && t < SMALL_NI) a.cnt_clear[t] = 0;
+  }
+  const int ntiles = (nj + 255) / 256;
+  const int t1 = min(ntiles, (b + 1) * a.tiles);
+  for (int tl = b * a.tiles; tl < t1; ++tl) {
+    const int j = tl * 256 + t;
+    if constexpr (PRED) {
+      Rec r{};
+      const bool upd = j < a.nbits && (a.bits[j >> 5] >> (j & 31) & 1u);
+      if (__syncthreads_or(upd)) {  // also: every wave is done with the last tile
+        if (t < a.nupd) {
+          const int q = reinterpret_cast<const int2*>(a.rows_h + (size_t)t * NR + NR - 1)->x - tl * 256;
+          if (q >= 0 && q < 256) row_of[q] = t;
+        }
+        __syncthreads();
+      }
+      tile_id_range(a.st, j);
+      if (j < nj) {
+        const size_t cap = (size_t)a.st.cap;
+        double p[3], v[3], ac[3], m;
+        if (upd) {
+          const double* u = a.rows_h + (size_t)row_of[t] * NR;
+          double raw[NR - 1];
+#pragma unroll
+          for (int f = 0; f < NR - 1; ++f) raw[f] = u[f];
+#pragma unroll
+          for (int f = 0; f < NR - 1; ++f) a.st.raw[(size_t)f * cap + j] = raw[f];
+          predict_one<ORDER>([&](int f) { return raw[f]; }, a.ti, p, v, ac);
+          m = raw[RF_M];
+        } else {
+          predict_one<ORDER>([&](int f) { return a.st.raw[f * cap + j]; }, a.ti, p, v, ac);
+          m = a.st.raw[RF_M * cap + j];
+        }
+        r = put_pred<ORDER, F64>(a.st, j, p, v, ac, m, a.st.id[j]);
+      }
+      tile[t] = r;  // past nj a massless record at the origin
+    } else {
+      __syncthreads();
+      if (j < nj) tile[t] = reinterpret_cast<const Rec*>(a.f.rec)[j];
+      else tile[t] = Rec{};
+    }
+    __syncthreads();
+    R s[NF];
+#pragma unroll
+    for (int f = 0; f < NF; ++f) s[f] = R(0);
+#pragma unroll 2
+    for (int k = 0; k < P; ++k) {
+      const int q = w * 64 + jsub + (k << (6 - lp));
+      const int jq = tl * 256 + q;
+      const Rec& rj = tile[q];
+      if (pair<ORDER, NGB, true, false>(rj, jq, jq < nj, st, eps2, s, dsmin, nnaddr)) ngb.add(rj.id);
+    }
+#pragma unroll
+    for (int f = 0; f < NF; ++f) T[f] += (double)s[f];
+  }
+  if constexpr (NGB) ngb.finish();
+  double dsd = (double)dsmin;
+  for (int m = P; m < 64; m <<= 1) {
+#pragma unroll
+    for (int f = 0; f < NF; ++f) T[f] += __shfl_xor(T[f], m);
+    const double od = __shfl_xor(dsd, m);
+    const int oa = __shfl_xor(nnaddr, m);
+    const bool take = (od < dsd) || (od == dsd && oa < nnaddr);
+    dsd = take ? od : dsd;
+    nnaddr = take ? oa : nnaddr;
+  }
+  if (jsub == 0) {
+#pragma unroll
+    for (int f = 0; f < NF; ++f) red[w][f][islot] = T[f];
+    red_d[w][islot] = dsd;
+    red_a[w][islot] = nnaddr;
+  }
+  __syncthreads();
+  const int rows = gridDim.x;
+  for (int o = t; o < (NF + 1) * SMALL_NI; o += 256) {
+    const int f = o / SMALL_NI, i = o % SMALL_NI;
+    if (i >= ni) continue;
+    if (f < NF) {
+      a.f.part[((size_t)f * rows + b) * ni + i] = (red[0][f][i] + red[1][f][i]) + (red[2][f][i] + red[3][f][i]);
+    } else {
+      double bd = red_d[0][i];
+      int ba = red_a[0][i];
+#pragma unroll
+      for (int q = 1; q < 4; ++q) {
+        const bool take = (red_d[q][i] < bd) || (red_d[q][i] == bd && red_a[q][i] < ba);
+        bd = take ? red_d[q][i] : bd;
+        ba = take ? red_a[q][i] : ba;
+      }
+      a.f.part_ds2[(size_t)b * ni + i] = bd;
+      a.f.part_addr[(size_t)b * ni + i] = ba;
+    }
+  }
+}
+
 template <int ORDER, bool F64>
 __device__ __forceinline__ void write_row(const FinalizeArgs& a, int i, const double* T, double ds, int ad,
                                           int cnt);
@@ -974,7 +1107,7 @@ __device__ __forceinline__ void finalize_block(const FinalizeArgs& a, int b) {
   __syncthreads();
   // output o: field o / I of i-particle o % I, and last the nearest neighbour and
   // count; L lanes each take every L-th of its U values
-  constexpr int L = U == 64 ? 4 : 1, OUT = (NF + 1) * I;
+  constexpr int L = U == 256 ? 16 : U == 64 ? 4 : 1, OUT = (NF + 1) * I;
   static_assert(L == 1 || L * OUT <= 256, "one pass");
   for (int o = t / L; o < OUT; o += 256 / L) {
     const int f = o / I, k = o % I, io = b * I + k, l = t % L;
@@ -1203,8 +1336,29 @@ static int launch_force_t(hipStream_t s, const ForceArgs& a, const ForceConfig& 
   return hip_status();
 }
 
+int launch_force_small(hipStream_t s, int order, bool f64, const SmallArgs& a, const ForceConfig& c, bool pred) {
+  if (a.f.grid_ni <= 0 || a.f.nj <= 0) return 0;
+  if (a.f.grid_ni > SMALL_NI || a.nupd > SMALL_UPD || a.tiles <= 0 || (long)c.S * a.tiles * 256 < a.f.nj) return -3;
+  dispatch_op(order, f64, [&](auto OR, auto FP) {
+    constexpr int O = decltype(OR)::value;
+    constexpr bool F = decltype(FP)::value;
+    const dim3 nb(c.S), bs(256);
+    if (pred && a.f.ngb_on) hipLaunchKernelGGL((k_force_small<O, F, true, true>), nb, bs, 0, s, a);
+    else if (pred) hipLaunchKernelGGL((k_force_small<O, F, false, true>), nb, bs, 0, s, a);
+    else if (a.f.ngb_on) hipLaunchKernelGGL((k_force_small<O, F, true, false>), nb, bs, 0, s, a);
+    else hipLaunchKernelGGL((k_force_small<O, F, false, false>), nb, bs, 0, s, a);
+  });
+  return hip_status();
+}
+
 int launch_force(hipStream_t s, int order, bool f64, const ForceArgs& a, const ForceConfig& c) {
   if (a.grid_ni <= 0 || a.nj <= 0) return 0;
+  if (c.small) {
+    SmallArgs sm{};
+    sm.f = a;
+    sm.tiles = c.jchunk / 256;
+    return launch_force_small(s, order, f64, sm, c, false);
+  }
   if (c.S <= 0 || c.jchunk <= 0 || (long)c.S * c.jchunk < a.nj) return -3;
   int rc = 0;
   dispatch_op(order, f64, [&](auto OR, auto FP) { rc = launch_force_t<decltype(OR)::value, decltype(FP)::value>(s, a, c); });
@@ -1219,6 +1373,7 @@ int launch_finalize(hipStream_t s, int order, bool f64, const FinalizeArgs& a) {
     const int nsort = a.ngb_on ? blocks_for(a.grid_ni, 4) : 0;
     const int nfin = blocks_for((long)a.U * a.grid_ni, 256);
     switch (a.U) {
+      case 256: hipLaunchKernelGGL((k_finalize<O, F, 256>), dim3(nfin + nsort), dim3(256), 0, s, a, nfin); break;
       case 64: hipLaunchKernelGGL((k_finalize<O, F, 64>), dim3(nfin + nsort), dim3(256), 0, s, a, nfin); break;
       case 16: hipLaunchKernelGGL((k_finalize<O, F, 16>), dim3(nfin + nsort), dim3(256), 0, s, a, nfin); break;
       default: hipLaunchKernelGGL((k_finalize<O, F, 4>), dim3(nfin + nsort), dim3(256), 0, s, a, nfin); break;

@@ -16,14 +16,16 @@ from _util import load_engine, plummer_system, random_derivs
 pytestmark = pytest.mark.gpu
 
 # (updates, addresses repeated within the batch, addresses staged just before it, ids changed)
-ROUNDS = [(1, 0, 0, 0), (63, 0, 0, 0), (64, 1, 0, 0), (65, 0, 2, 1), (2047, 0, 0, 0), (2048, 0, 0, 0),
-          (2100, 0, 0, 3), (2500, 40, 0, 0), (2500, 0, 40, 0), (4099, 0, 0, 0)]
+ROUNDS = [(1, 0, 0, 0), (63, 0, 0, 0), (64, 1, 0, 0), (65, 0, 2, 1), (255, 0, 0, 0), (256, 3, 0, 0), (257, 0, 0, 0),
+          (1, 0, 0, 1), (256, 0, 9, 0), (0, 0, 0, 0), (2047, 0, 0, 0), (2048, 0, 0, 0),
+          (2100, 0, 0, 3), (2500, 40, 0, 0), (2500, 0, 40, 0), (4099, 0, 0, 0), (6500, 30, 0, 0),
+          (7000, 0, 0, 5), (6200, 0, 20, 0)]
 
 
 @pytest.mark.parametrize("order", [sa.FOURTH, sa.SIXTH])
 @pytest.mark.parametrize("prec", [sa.DOUBLESINGLE, sa.DOUBLE])
 def test_update_routes_agree(order, prec):
-    n = 6001
+    n = 7001
     m, x, v, ids, h2 = plummer_system(n, seed=71)
     ids = ids.copy()
     acc, jrk, snp, crk = random_derivs(n, 72, 0.3)
@@ -55,13 +57,14 @@ def test_update_routes_agree(order, prec):
                               opt(crk, batch), tj=tj[batch])
             for q in u:
                 b.set_j_particle(q, ids[q], tj[q], 0.0, m[q], acc[q], jrk[q], v[q], x[q], opt(snp, q), opt(crk, q))
-            predict = r % 4 != 3
+            predict = r % 5 != 3
             ti = 1.0 / 512 * (1 + r % 3)
             for e in (a, b):
                 e.set_time(ti) if predict else e.set_no_time()
-            nj = n - 200 if r % 3 == 2 else n        # some updates lie beyond the predicted range
+            nj = n - 200 if r % 4 == 2 else n        # some updates lie beyond the predicted range
             b.force_prediction(nj)
-            sel = np.sort(rng.choice(n, 150, replace=False))
+            # small calls apply up to 256 updates in their force launch
+            sel = np.sort(rng.choice(n, (150, 3, 32)[r % 3], replace=False))
             ai = acc[sel] if order >= sa.SIXTH else None
             res = []
             for e in (a, b):
