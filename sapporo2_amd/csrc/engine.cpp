@@ -35,6 +35,11 @@ constexpr int MIN_ITERS_PER_LANE = 16;
 constexpr int MIN_J_PER_SPLIT = 512;
 // Launch shapes of lane shape P = 64 (choose_config)
 constexpr int SMALL_ROWS = 512;
+// Calls up to these counts complete by the finalize's word, larger ones by an
+// event: every work-group then waits for its output to reach the host, which the
+// many short ones that sort lists pay for (3000 i with lists: finalize 23 -> 52 us;
+// 333 i equal; 2500 i without lists: call 383 -> 350 us).
+constexpr int DONE_WORD_NI = 4096, DONE_WORD_NGB = 128;
 constexpr long MIN_CHUNK = 64, MAX_CHUNK = 256, MAX_WAVES = 65536;
 // Mixed launches of at most this many waves (4 per SIMD) take their records
 // ahead: one wave alone waits ~190 ns per pair for scalar loads, 80 with them
@@ -148,6 +153,12 @@ int Engine::open(int device, int order, int precision) {
   for (auto& s : stage_) HIPCHK(hipEventCreateWithFlags(&s.ev, hipEventDisableTiming), "hipEventCreate");
   HIPCHK(hipEventCreateWithFlags(&ev_desc_, hipEventDisableTiming), "hipEventCreate");
   HIPCHK(dmalloc(&pack_ctr_d_, 1), "pack counter");
+  coherent_ = host_coherent();
+  HIPCHK(hmap(&done_h_, &done_hd_, 16, true), "completion word");
+  *done_h_ = 0;
+  call_seq_ = 0;
+  HIPCHK(dmalloc(&done_ctr_d_, 1), "completion counter");
+  HIPCHK(hipMemsetAsync(done_ctr_d_, 0, sizeof(int), stream_), "memset");
   HIPCHK(dmalloc(&cnt_small_d_, 2 * SMALL_NI), "small-call counters");
   HIPCHK(hipMemsetAsync(cnt_small_d_, 0, 2 * SMALL_NI * sizeof(int), stream_), "memset");
   small_flip_ = false;
@@ -206,10 +217,12 @@ int Engine::close() {
   hfree(packed_h_); packed_hd_ = nullptr; packed_cap_ = 0;
   dfree(pack_ctr_d_);
   dfree(cnt_small_d_);
+  hfree(done_h_); done_hd_ = nullptr;
+  dfree(done_ctr_d_);
   dfree(cnt_d_); dfree(list_d_); list_cap_ = 0;
   slot_lists_h_.clear();
   dfree(gather_d_); gather_cap_ = 0;
-  dfree(gaddr_d_); gaddr_cap_ = 0;
+  hfree(gather_h_); hfree(gaddr_h_); gather_hd_ = nullptr; gaddr_hd_ = nullptr; gather_hcap_ = 0;
   dfree(idesc_d_); dfree(ens_eps_d_); ens_eps_cap_ = 0;
   hfree(ens_tab_h_); dfree(ens_tab_d_); ens_tab_cap_ = 0;
   icap_ = 0; cl_off_.clear(); cl_n_.clear(); cl_total_ = 0;
@@ -822,9 +835,9 @@ int Engine::ensure_icap(int need) {
   HIPCHK(hmalloc(&iid_h_, nI), "pinned i ids");
   HIPCHK(dmalloc(&ibuf_d_, IBUF_FIELDS * nI), "i buffer");
   HIPCHK(dmalloc(&iid_d_, nI), "i ids");
-  HIPCHK(hmap(&res_h_, &res_hd_, nI * out_fields(order_), host_coherent()), "host-mapped results");
+  HIPCHK(hmap(&res_h_, &res_hd_, nI * out_fields(order_), coherent_), "host-mapped results");
   res_stride_ = (long)nI;
-  HIPCHK(hmap(&loff_h_, &loff_hd_, nI, host_coherent()), "host-mapped list offsets");
+  HIPCHK(hmap(&loff_h_, &loff_hd_, nI, coherent_), "host-mapped list offsets");
   HIPCHK(dmalloc(&cnt_d_, nI), "neighbour counts");
   HIPCHK(dmalloc(&idesc_d_, nI), "ensemble i descriptors");
   HIPCHK(hipMemsetAsync(cnt_d_, 0, nI * sizeof(int), stream_), "memset");
@@ -854,7 +867,7 @@ int Engine::ensure_packed(long need) {
   if (stream_) HIPCHK(hipStreamSynchronize(stream_), "packed-list grow sync");
   inflight_ = false;
   hfree(packed_h_);
-  HIPCHK(hmap(&packed_h_, &packed_hd_, (size_t)need, host_coherent()), "host-mapped packed lists");
+  HIPCHK(hmap(&packed_h_, &packed_hd_, (size_t)need, coherent_), "host-mapped packed lists");
   packed_cap_ = need;
   have_results_ = false;
   ++gen_;
@@ -867,6 +880,9 @@ FinalizeArgs Engine::finalize_args(int grid_ni, bool ngb_on) const {
   fz.part_ds2 = pds2_d_;
   fz.part_addr = paddr_d_;
   fz.cd = desc_d_;
+  fz.ni = desc_h_->ni;
+  fz.seq = desc_h_->seq;
+  if (done_word_) { fz.done = done_hd_; fz.done_ctr = done_ctr_d_; }
   fz.grid_ni = grid_ni;
   fz.rec = st_.rec;
   fz.ngb_cnt = cnt_d_;
@@ -1121,6 +1137,7 @@ int Engine::start_grav_calc_clusters(int ni, const int* cluster, const int* id, 
   if (desc_pending_ && desc_seq_ > done_seq_) HIPCHK(hipEventSynchronize(ev_desc_), "descriptor wait");
   desc_pending_ = false;
   *desc_h_ = CallDesc{t_i_, 0.0, ni, 0, 0, 0};
+  done_word_ = false;
   if (timing_) HIPCHK(hipEventRecord(ev_d0_, stream_), "event");
   if (prep(predict_ ? cl_total_ : 0, (int)sizeof(CallDesc), ngb_on ? ni : 0, true) != 0) return -1;
   predict_ = false;
@@ -1212,7 +1229,8 @@ int Engine::start_grav_calc(int nj, int ni, const int* id, const double (*xi)[3]
   desc_h_->ni = ni;
   desc_h_->nupd = nupd;
   desc_h_->ni_reset = ngb_on ? ni : 0;
-  desc_h_->pad = 0;
+  done_word_ = coherent_ && ni <= (ngb_on ? DONE_WORD_NGB : DONE_WORD_NI);
+  desc_h_->seq = next_seq();
   const size_t nbytes = (size_t)((char*)(bx + nd) - (char*)call_h_);
   if (graphs_) {
     HIPCHK(hipMemcpyAsync(call_d_, call_h_, nbytes, hipMemcpyHostToDevice, stream_), "call upload");
@@ -1244,7 +1262,7 @@ int Engine::start_grav_calc(int nj, int ni, const int* id, const double (*xi)[3]
     timed_force_ = timing_;
   }
   if (timing_) HIPCHK(hipEventRecord(ev_d1_, stream_), "event");
-  HIPCHK(hipEventRecord(ev_done_, stream_), "event");
+  if (!done_word_) HIPCHK(hipEventRecord(ev_done_, stream_), "event");
   done_rec_seq_ = ++rec_seq_;
   inflight_ = true;
   have_results_ = true;
@@ -1271,7 +1289,9 @@ int Engine::call_small(int nj, const ForceConfig& cfg, bool ngb_on, int bucket) 
   a.f = force_args(ni, nj, ngb_on);
   a.f.ibuf = reinterpret_cast<const double*>(reinterpret_cast<const char*>(call_ibuf_d_) + alias);
   a.f.iid = reinterpret_cast<const int*>(reinterpret_cast<const char*>(call_iid_d_) + alias);
-  a.f.cd = reinterpret_cast<const CallDesc*>(call_hd_);
+  a.f.cd = nullptr;
+  a.ni = ni;
+  a.eps2 = desc_h_->eps2;
   a.f.ngb_cnt = cnt;
   a.tiles = cfg.jchunk / 256;
   a.st = st_;
@@ -1280,6 +1300,7 @@ int Engine::call_small(int nj, const ForceConfig& cfg, bool ngb_on, int bucket) 
   a.nbits = nstaged_ > 0 ? (int)std::min<size_t>(sg.words * 32, INT_MAX) : 0;
   a.nupd = nstaged_;
   a.ti = t_i_;
+  for (int k = 0; k < std::min(nstaged_, SMALL_ARG); ++k) a.addr[k] = sg.addr[k];
   a.cnt_clear = cnt_small_d_ + (small_flip_ ? 0 : SMALL_NI);
   small_flip_ = !small_flip_;
   timed_scatter_ = timed_predict_ = false;
@@ -1287,7 +1308,7 @@ int Engine::call_small(int nj, const ForceConfig& cfg, bool ngb_on, int bucket) 
   if (launch_force_small(stream_, order_, f64_, a, cfg, true) != 0) return fail("force launch", hipGetLastError());
   if (timing_) HIPCHK(hipEventRecord(ev_f1_, stream_), "event");
   FinalizeArgs fz = finalize_args(ni, ngb_on);
-  fz.cd = a.f.cd;
+  fz.cd = nullptr;
   fz.ngb_cnt = cnt;
   fz.S = partial_rows(cfg);
   fz.U = finalize_threads(bucket);
@@ -1490,19 +1511,37 @@ void Engine::drop_graphs() {
   graph_cache_.clear();
 }
 
-// Waits for the last call's completion event by polling it (the caller is
+// Waits for the last call's completion word or event by polling it (the caller is
 // blocked anyway; polling wakes within a microsecond or two, where a blocking
-// wait costs tens).  Everything recorded before that event is then complete.
+// wait costs tens).  Everything queued before the call's finalize is then complete.
 int Engine::wait_results() {
   if (!inflight_) return 0;
-  hipError_t e;
-  while ((e = hipEventQuery(ev_done_)) == hipErrorNotReady) {
-    for (int k = 0; k < 32; ++k) _mm_pause();
+  hipError_t e = hipSuccess;
+  if (done_word_) {
+    if (wait_word() != 0) return -1;
+  } else {
+    while ((e = hipEventQuery(ev_done_)) == hipErrorNotReady) {
+      for (int k = 0; k < 32; ++k) _mm_pause();
+    }
   }
   if (e != hipSuccess) return fail("result wait", e);
   HIPCHK(hipGetLastError(), "device error");
   inflight_ = false;
   done_seq_ = done_rec_seq_;
+  return 0;
+}
+
+// Polls the completion word of the launch numbered call_seq_.
+int Engine::wait_word() {
+  auto done = [&] { return __atomic_load_n(done_h_, __ATOMIC_ACQUIRE) == call_seq_; };
+  for (unsigned k = 1; !done(); ++k) {
+    _mm_pause();
+    if (k % 8192 != 0) continue;
+    // now and then: has the stream failed, or ended without the word?
+    const hipError_t e = hipStreamQuery(stream_);
+    if (e == hipErrorNotReady || (e == hipSuccess && done())) continue;
+    return fail("wait: the device work ended without its completion word", e);
+  }
   return 0;
 }
 
@@ -1702,34 +1741,42 @@ int Engine::retrieve_predicted_j_particles(int n, const int* addr, double* mass,
   if (flush_updates() != 0) return -1;
   for (int k = 0; k < n; ++k)
     if (addr[k] < 0 || addr[k] > max_addr_) return fail("retrieve_predicted_j_particles: address never set");
-  if (gather_cap_ < (size_t)n) {
-    dfree(gather_d_);
-    HIPCHK(dmalloc(&gather_d_, (size_t)n * 10), "gather buffer");
-    gather_cap_ = n;
+  // addresses and rows go through pinned memory that the kernel reads and writes
+  if (gather_hcap_ < (size_t)n) {
+    hfree(gather_h_);
+    hfree(gaddr_h_);
+    gather_hcap_ = 0;
+    const size_t nc = std::max<size_t>(n, 1024);
+    HIPCHK(hmap(&gather_h_, &gather_hd_, nc * 10, true), "pinned gather rows");
+    HIPCHK(hmap(&gaddr_h_, &gaddr_hd_, nc, true), "pinned gather addresses");
+    gather_hcap_ = nc;
   }
-  if (gaddr_cap_ < (size_t)n) {
-    dfree(gaddr_d_);
-    HIPCHK(dmalloc(&gaddr_d_, (size_t)n), "gather addresses");
-    gaddr_cap_ = n;
-  }
-  HIPCHK(hipMemcpyAsync(gaddr_d_, addr, sizeof(int) * (size_t)n, hipMemcpyHostToDevice, stream_), "address upload");
+  memcpy(gaddr_h_, addr, sizeof(int) * (size_t)n);
   GatherArgs g{};
   g.st = st_;
   g.n = n;
-  g.out = gather_d_;
-  g.addr = gaddr_d_;
+  g.out = gather_hd_;
+  g.addr = gaddr_hd_;
+  g.done = done_hd_;
+  g.done_ctr = done_ctr_d_;
+  g.seq = next_seq();
   if (launch_gather_pred(stream_, order_, f64_, g) != 0) return fail("gather launch", hipGetLastError());
-  gather_h_.resize((size_t)n * 10);
-  HIPCHK(hipMemcpyAsync(gather_h_.data(), gather_d_, sizeof(double) * (size_t)n * 10, hipMemcpyDeviceToHost,
-                        stream_), "gather download");
-  HIPCHK(hipStreamSynchronize(stream_), "read-back sync");
-  for (int k = 0; k < n; ++k) {
-    const double* p = gather_h_.data() + (size_t)k * 10;
-    if (pos) { pos[k][0] = p[0]; pos[k][1] = p[1]; pos[k][2] = p[2]; }
-    if (mass) mass[k] = p[3];
-    if (vel) { vel[k][0] = p[4]; vel[k][1] = p[5]; vel[k][2] = p[6]; }
-    if (acc) { acc[k][0] = p[7]; acc[k][1] = p[8]; acc[k][2] = p[9]; }
-  }
+  if (wait_word() != 0) return -1;
+  HIPCHK(hipGetLastError(), "device error");
+  const double* p = gather_h_;
+  auto rows = [&](size_t b, size_t e) {
+    auto vec = [&](double (*dst)[3], int f) {
+      if (!dst) return;
+      const double *q0 = p + (size_t)f * n, *q1 = q0 + n, *q2 = q1 + n;
+      for (size_t k = b; k < e; ++k) { dst[k][0] = q0[k]; dst[k][1] = q1[k]; dst[k][2] = q2[k]; }
+    };
+    vec(pos, 0);
+    if (mass) memcpy(mass + b, p + 3 * (size_t)n + b, sizeof(double) * (e - b));
+    vec(vel, 4);
+    vec(acc, 7);
+  };
+  if ((size_t)n >= PAR_ROWS) par_for((size_t)n, rows);
+  else rows(0, (size_t)n);
   return 0;
 }
 
@@ -1739,12 +1786,12 @@ int Engine::retrieve_predicted_j_particle(int addr, double* mass, double* id, do
   if (addr < 0) return fail("retrieve_predicted_j_particle: negative address");
   if (fetch_j_host(addr + 1) != 0) return -1;
   if (addr >= jhost_n_) return fail("retrieve_predicted_j_particle: address never set");
-  const double* p = jpred_h_.data() + (size_t)addr * 10;
-  if (pos) { pos[0] = p[0]; pos[1] = p[1]; pos[2] = p[2]; }
-  if (mass) *mass = p[3];
-  if (vel) { vel[0] = p[4]; vel[1] = p[5]; vel[2] = p[6]; }
+  auto p = [&](int f) { return jpred_h_[(size_t)f * jhost_n_ + addr]; };
+  if (pos) { pos[0] = p(0); pos[1] = p(1); pos[2] = p(2); }
+  if (mass) *mass = p(3);
+  if (vel) { vel[0] = p(4); vel[1] = p(5); vel[2] = p(6); }
   if (eps2) *eps2 = jraw_h_[(size_t)RF_EPS * jhost_n_ + addr];
-  if (acc && order_ >= ORDER_H6) { acc[0] = p[7]; acc[1] = p[8]; acc[2] = p[9]; }
+  if (acc && order_ >= ORDER_H6) { acc[0] = p(7); acc[1] = p(8); acc[2] = p(9); }
   if (id) *id = (double)jid_h_[addr];
   return 0;
 }
@@ -1884,17 +1931,17 @@ int Engine::retrieve_j_particle_state(int addr, double* mass, double* id, double
   if (addr >= jhost_n_) return fail("retrieve_j_particle_state: address never set");
   const size_t n = jhost_n_;
   auto raw = [&](int f) { return jraw_h_[(size_t)f * n + addr]; };
-  const double* p = jpred_h_.data() + (size_t)addr * 10;
+  auto p = [&](int f) { return jpred_h_[(size_t)f * jhost_n_ + addr]; };
   if (mass) *mass = raw(RF_M);
   if (pos) for (int d = 0; d < 3; ++d) pos[d] = raw(RF_X + d);
-  if (ppos) for (int d = 0; d < 3; ++d) ppos[d] = p[d];
-  if (pvel) for (int d = 0; d < 3; ++d) pvel[d] = p[4 + d];
+  if (ppos) for (int d = 0; d < 3; ++d) ppos[d] = p(d);
+  if (pvel) for (int d = 0; d < 3; ++d) pvel[d] = p(4 + d);
   if (eps2) *eps2 = raw(RF_EPS);
   if (vel) for (int d = 0; d < 3; ++d) vel[d] = raw(RF_VX + d);
   if (acc) for (int d = 0; d < 3; ++d) acc[d] = raw(RF_AX + d);
   if (jrk) for (int d = 0; d < 3; ++d) jrk[d] = raw(RF_JX + d);
   if (id) *id = (double)jid_h_[addr];
-  if (pacc && order_ >= ORDER_H6) for (int d = 0; d < 3; ++d) pacc[d] = p[7 + d];
+  if (pacc && order_ >= ORDER_H6) for (int d = 0; d < 3; ++d) pacc[d] = p(7 + d);
   return 0;
 }
 

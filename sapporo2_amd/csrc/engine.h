@@ -17,6 +17,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <climits>
 #include <cstdint>
 #include <string>
 #include <vector>
@@ -154,6 +155,8 @@ class Engine {
                         int sblocks, int fin_u);
   void drop_graphs();
   int wait_results();
+  int wait_word();
+  int next_seq() { return call_seq_ = call_seq_ == INT_MAX ? 1 : call_seq_ + 1; }
   int ensure_lists(int need);
   int ensure_packed(long need);
   sapk::FinalizeArgs finalize_args(int grid_ni, bool ngb_on) const;
@@ -218,6 +221,11 @@ class Engine {
   std::vector<int> slot_lists_h_;   // device list slots read back when the packed lists did not fit
   bool lists_in_slots_ = false;     // lists read back from the device slots (packed overflow)
   bool lists_packed_ = false;       // last call's host lists are atomically packed (ensembles), else in i order
+  // completion of a call: a host-mapped word that its finalize sets to call_seq_
+  // (done_word_), or ev_done_
+  bool coherent_ = true, done_word_ = false;
+  int* done_h_ = nullptr; int* done_hd_ = nullptr; int* done_ctr_d_ = nullptr;
+  int call_seq_ = 0;
   hipEvent_t ev_done_ = nullptr, ev_d0_ = nullptr, ev_d1_ = nullptr, ev_f0_ = nullptr, ev_f1_ = nullptr, ev_p0_ = nullptr, ev_p1_ = nullptr;
   hipEvent_t ev_s0_ = nullptr, ev_s1_ = nullptr;
   bool timed_scatter_ = false;
@@ -279,8 +287,9 @@ class Engine {
   std::vector<double> jpred_h_, jraw_h_;
   std::vector<int> jid_h_;
   double* gather_d_ = nullptr; size_t gather_cap_ = 0;
-  int* gaddr_d_ = nullptr; size_t gaddr_cap_ = 0;
-  std::vector<double> gather_h_;
+  // read-back of listed addresses: pinned rows and addresses, with device aliases
+  double* gather_h_ = nullptr; double* gather_hd_ = nullptr;
+  int* gaddr_h_ = nullptr; int* gaddr_hd_ = nullptr; size_t gather_hcap_ = 0;
 };
 
 }  // namespace sap

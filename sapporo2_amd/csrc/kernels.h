@@ -81,7 +81,7 @@ struct CallDesc {
   int ni;                // active i-particles of the call
   int nupd;              // staged j-updates to scatter
   int ni_reset;          // neighbour counters to clear before the call
-  int pad;
+  int seq;               // number of the call (completion word)
 };
 
 // Scatter staged updates into the store and reset the per-i neighbour
@@ -148,17 +148,23 @@ struct ForceArgs {
 
 // k_force_small: at most SMALL_NI i-particles; with the prediction in the same
 // launch (pred), also the staged updates, at most SMALL_UPD, all at addresses
-// below f.nj and none changing an id.  f.cd, f.ibuf and f.iid may be host-mapped.
-constexpr int SMALL_NI = 32, SMALL_UPD = 256;
+// below f.nj and none changing an id; f.ibuf and f.iid are then host-mapped and
+// ni and eps2 come by value (f.cd would be one more read over PCIe before them).
+// A few addresses (SMALL_ARG) come as arguments, more through the bit set and the
+// rows' own (address, id) pairs, two more reads over PCIe before the rows.
+constexpr int SMALL_NI = 32, SMALL_UPD = 256, SMALL_ARG = 16;
 struct SmallArgs {
   ForceArgs f;
   int tiles;              // tiles of 256 j per work-group
-  StoreView st;           // pred from here on
+  int ni;                 // pred from here on
+  double eps2;
+  StoreView st;
   const double* rows_h;   // staged rows, host-mapped
   const unsigned* bits;   // their addresses as a bit set of nbits, host-mapped
   int nbits, nupd;
   double ti;
   int* cnt_clear;         // SMALL_NI counters cleared for the next call of this kind
+  int addr[SMALL_ARG];    // the rows' addresses when nupd <= SMALL_ARG
 };
 
 // Launch geometry of one force call: each wave owns P i-particles and Q = 64/P
@@ -198,7 +204,10 @@ constexpr int LIST_REGION = 256;
 struct FinalizeArgs {
   const double* part; const double* part_ds2; const int* part_addr;
   int S;
-  const CallDesc* cd;    // ni
+  const CallDesc* cd;    // ni, and seq for done; null: ni and seq below
+  int ni; int seq;
+  int* done;             // host-mapped completion word: set to seq when all output is written (null: none)
+  int* done_ctr;         // device: work-groups finished, 0 between launches
   int grid_ni;           // launch size (host), >= cd->ni
   int U;                 // threads per i-particle (finalize_threads)
   const void* rec;       // to look up the neighbour's id
@@ -233,10 +242,13 @@ struct EnsArgs {
   int* ngb_cnt; int* ngb_list; int ngb_on;
 };
 
-// Gathers the FP64 predicted state (pos, mass, vel, [acc]) into a dense AoS
-// buffer for read-back, 10 doubles per row: of all j in [0, n) (addr null) or
-// of the n listed addresses.
-struct GatherArgs { StoreView st; int n; double* out; const int* addr; };
+// Gathers the FP64 predicted state (pos, mass, vel, [acc]) for read-back, 10 x n
+// doubles, field-major: of all j in [0, n) (addr null) or of the n listed
+// addresses.  out and addr may be host-mapped; done as in FinalizeArgs.
+struct GatherArgs {
+  StoreView st; int n; double* out; const int* addr;
+  int* done; int* done_ctr; int seq;
+};
 
 int launch_scatter(hipStream_t s, int order, bool f64, const ScatterArgs& a);
 int launch_predict(hipStream_t s, int order, bool f64, const PredictArgs& a);

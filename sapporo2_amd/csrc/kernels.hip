@@ -795,15 +795,21 @@ __global__ __launch_bounds__(256) void k_force_small(SmallArgs a) {
   __shared__ int red_a[4][SMALL_NI];
   __shared__ int row_of[256];
   const int t = threadIdx.x, w = t >> 6, lane = t & 63, b = blockIdx.x;
-  const int ni = min(a.f.cd->ni, SMALL_NI), nj = a.f.nj;
-  const R eps2 = (R)a.f.cd->eps2;
+  const int ni = PRED ? a.ni : min(a.f.cd->ni, SMALL_NI), nj = a.f.nj;
+  const R eps2 = (R)(PRED ? a.eps2 : a.f.cd->eps2);
   const int lp = ni > 1 ? 32 - __clz(ni - 1) : 0, P = 1 << lp;
   const int islot = lane & (P - 1), jsub = lane >> lp;
-  const double* ib = a.f.ibuf;
-  const IState<ORDER, R> st =
-      load_i<ORDER, R, NGB>(ib, ib + 3 * ni, ib + 6 * ni, ib + (ORDER >= ORDER_H6 ? 9 : 6) * ni, a.f.iid,
-                            islot < ni ? islot : 0, islot < ni);
-  NgbList ngb{a.f.ngb_cnt, a.f.ngb_list, st.i, -1};
+  // the i-particle's doubles are loaded first and converted when the first tile
+  // is there: over PCIe they take as long as the tile
+  constexpr int NI = ORDER >= ORDER_H6 ? 9 : 6;
+  const int il = islot < ni ? islot : 0;
+  double iv[NI], ih = -1.0;
+#pragma unroll
+  for (int f = 0; f < NI; ++f) iv[f] = a.f.ibuf[(size_t)(f / 3) * 3 * ni + 3 * il + f % 3];
+  if (NGB && islot < ni) ih = a.f.ibuf[(size_t)NI * ni + il];
+  const int iid = a.f.iid[il];
+  IState<ORDER, R> st;
+  NgbList ngb{a.f.ngb_cnt, a.f.ngb_list, il, -1};
   double T[NF];
 #pragma unroll
   for (int f = 0; f < NF; ++f) T[f] = 0.0;
@@ -819,32 +825,43 @@ __global__ __launch_bounds__(256) void k_force_small(SmallArgs a) {
     const int j = tl * 256 + t;
     if constexpr (PRED) {
       Rec r{};
-      const bool upd = j < a.nbits && (a.bits[j >> 5] >> (j & 31) & 1u);
-      if (__syncthreads_or(upd)) {  // also: every wave is done with the last tile
-        if (t < a.nupd) {
-          const int q = reinterpret_cast<const int2*>(a.rows_h + (size_t)t * NR + NR - 1)->x - tl * 256;
-          if (q >= 0 && q < 256) row_of[q] = t;
+      // stored fields: loads that do not wait for the update bits
+      const size_t cap = (size_t)a.st.cap;
+      double raw[NR - 1];
+      if (j < nj) {
+#pragma unroll
+        for (int f = 0; f < NR - 1; ++f)
+          if (f != RF_DT && f != RF_EPS) raw[f] = a.st.raw[(size_t)f * cap + j];
+      }
+      int row = -1;  // staged row of this j
+      if (a.nupd <= SMALL_ARG) {
+#pragma unroll
+        for (int u = 0; u < SMALL_ARG; ++u)
+          if (u < a.nupd && a.addr[u] == j) row = u;
+        __syncthreads();  // every wave is done with the last tile
+      } else {
+        const bool upd = j < a.nbits && (a.bits[j >> 5] >> (j & 31) & 1u);
+        if (__syncthreads_or(upd)) {
+          if (t < a.nupd) {
+            const int q = reinterpret_cast<const int2*>(a.rows_h + (size_t)t * NR + NR - 1)->x - tl * 256;
+            if (q >= 0 && q < 256) row_of[q] = t;
+          }
+          __syncthreads();
+          if (upd) row = row_of[t];
         }
-        __syncthreads();
       }
       tile_id_range(a.st, j);
       if (j < nj) {
-        const size_t cap = (size_t)a.st.cap;
-        double p[3], v[3], ac[3], m;
-        if (upd) {
-          const double* u = a.rows_h + (size_t)row_of[t] * NR;
-          double raw[NR - 1];
+        if (row >= 0) {
+          const double* u = a.rows_h + (size_t)row * NR;
 #pragma unroll
           for (int f = 0; f < NR - 1; ++f) raw[f] = u[f];
 #pragma unroll
           for (int f = 0; f < NR - 1; ++f) a.st.raw[(size_t)f * cap + j] = raw[f];
-          predict_one<ORDER>([&](int f) { return raw[f]; }, a.ti, p, v, ac);
-          m = raw[RF_M];
-        } else {
-          predict_one<ORDER>([&](int f) { return a.st.raw[f * cap + j]; }, a.ti, p, v, ac);
-          m = a.st.raw[RF_M * cap + j];
         }
-        r = put_pred<ORDER, F64>(a.st, j, p, v, ac, m, a.st.id[j]);
+        double p[3], v[3], ac[3];
+        predict_one<ORDER>([&](int f) { return raw[f]; }, a.ti, p, v, ac);
+        r = put_pred<ORDER, F64>(a.st, j, p, v, ac, raw[RF_M], a.st.id[j]);
       }
       tile[t] = r;  // past nj a massless record at the origin
     } else {
@@ -853,13 +870,44 @@ __global__ __launch_bounds__(256) void k_force_small(SmallArgs a) {
       else tile[t] = Rec{};
     }
     __syncthreads();
+    if (tl == b * a.tiles) {
+      get_pos(st.x, iv[0]); get_pos(st.y, iv[1]); get_pos(st.z, iv[2]);
+      st.vx = (R)iv[3]; st.vy = (R)iv[4]; st.vz = (R)iv[5];
+      st.ax = st.ay = st.az = R(0);
+      if constexpr (ORDER >= ORDER_H6) { st.ax = (R)iv[6]; st.ay = (R)iv[7]; st.az = (R)iv[8]; }
+      st.h2 = (R)ih;
+      st.id = iid;
+      st.i = il;
+    }
     R s[NF];
 #pragma unroll
     for (int f = 0; f < NF; ++f) s[f] = R(0);
-#pragma unroll 2
-    for (int k = 0; k < P; ++k) {
-      const int q = w * 64 + jsub + (k << (6 - lp));
-      const int jq = tl * 256 + q;
+    // four j at a time (their LDS reads are in flight together), P < 4 one by one
+    int k = 0;
+    for (; k + 4 <= P; k += 4) {
+      R d[4];
+      int id[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int q = w * 64 + jsub + ((k + u) << (6 - lp)), jq = tl * 256 + q;
+        const Rec rj = tile[q];
+        id[u] = rj.id;
+        int unused = 0;
+        pair<ORDER, NGB, true, true>(rj, jq, jq < nj, st, eps2, s, d[u], unused);
+        const bool better = d[u] < dsmin;
+        dsmin = better ? d[u] : dsmin;
+        nnaddr = better ? jq : nnaddr;
+      }
+      if constexpr (NGB) {
+        settle<ORDER>(s);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) asm volatile("" : "+v"(d[u]));
+        const bool nb[4] = {st.h2 > d[0], st.h2 > d[1], st.h2 > d[2], st.h2 > d[3]};
+        ngb.add4(nb, [&](int u) { return id[u]; });
+      }
+    }
+    for (; k < P; ++k) {
+      const int q = w * 64 + jsub + (k << (6 - lp)), jq = tl * 256 + q;
       const Rec& rj = tile[q];
       if (pair<ORDER, NGB, true, false>(rj, jq, jq < nj, st, eps2, s, dsmin, nnaddr)) ngb.add(rj.id);
     }
@@ -1011,6 +1059,33 @@ __global__ __launch_bounds__(256) void k_finalize_ens(FinalizeArgs f, EnsArgs a)
 // Finalize.  Fixed-order sums of the partial rows of each i-particle, the
 // nearest neighbour as the (ds2, address) minimum, the result row, and the
 // ascending sort of the neighbour list.
+// Output in host memory: with a completion word, a store that is at the host when
+// the wave has waited for it (the word's protocol needs no cache write-back then,
+// which took 20 us over the work-groups of 333 i-particles).
+template <typename V> __device__ __forceinline__ void put_host(const int* done, V* p, V v) {
+  if (done) __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  else *p = v;
+}
+
+// The last work-group to finish tells the host: it polls a word in its own memory
+// instead of an event, whose record costs the host 4 us and the device a marker
+// behind the kernel (a chain of three empty kernels: 18 us with an event, 12 with
+// the word).  Every wave waits for its own output (put_host) before its work-
+// group counts.
+__device__ __forceinline__ void finish_word(int* done, int* ctr, int seq) {
+  __builtin_amdgcn_s_waitcnt(0);  // all counters
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const int k = __hip_atomic_fetch_add(ctr, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (k == (int)gridDim.x - 1) {
+      *ctr = 0;
+      __hip_atomic_store(done, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+  }
+}
+
+__device__ __forceinline__ int call_ni(const FinalizeArgs& a) { return a.cd ? a.cd->ni : a.ni; }
+
 // Nearest neighbour and count of i-particle i.
 template <int ORDER, bool F64>
 __device__ __forceinline__ void write_nn(const FinalizeArgs& a, int i, double ds, int ad, int cnt) {
@@ -1020,9 +1095,9 @@ __device__ __forceinline__ void write_nn(const FinalizeArgs& a, int i, double ds
   const size_t st = (size_t)a.ostride;
   const bool has = ad != INT_MAX;
   // the device returns ds2 rounded to float (kernels.cu:999-1002)
-  o[NF * st] = has ? (double)(float)ds : INFINITY;
-  o[(NF + 1) * st] = has ? (double)reinterpret_cast<const Rec*>(a.rec)[ad].id : -1.0;
-  o[(NF + 2) * st] = (double)cnt;
+  put_host(a.done, o + NF * st, has ? (double)(float)ds : (double)INFINITY);
+  put_host(a.done, o + (NF + 1) * st, has ? (double)reinterpret_cast<const Rec*>(a.rec)[ad].id : -1.0);
+  put_host(a.done, o + (NF + 2) * st, (double)cnt);
 }
 
 // Result row of i-particle i, field-major (consecutive i of a wave write
@@ -1078,7 +1153,7 @@ __device__ __forceinline__ void finalize_block(const FinalizeArgs& a, int b) {
   __shared__ double red[NF][256];
   __shared__ double red_d[256];
   __shared__ int red_a[256];
-  const int ni = a.cd->ni;
+  const int ni = call_ni(a);
   const int t = threadIdx.x;
   const int ii = t % I, u = t / I;
   const int i = b * I + ii;
@@ -1121,7 +1196,7 @@ __device__ __forceinline__ void finalize_block(const FinalizeArgs& a, int b) {
       double r = (v[0] + v[1]) + (v[2] + v[3]);
 #pragma unroll
       for (int m = 1; m < L; m <<= 1) r += __shfl_xor(r, m);
-      if (l == 0 && io < ni) a.out[(size_t)f * a.ostride + io] = r;
+      if (l == 0 && io < ni) put_host(a.done, a.out + (size_t)f * a.ostride + io, r);
     } else {
       double bd = red_d[l * I + k];
       int ba = red_a[l * I + k];
@@ -1168,7 +1243,7 @@ __device__ __forceinline__ void store_list(const FinalizeArgs& a, int i, const i
   for (int k = t; k < c; k += nt) {
     const int v = s[k];
     a.ngb_list[(size_t)i * NGB_CAP + k] = v;
-    if (host) a.packed[off + k] = v;
+    if (host) put_host(a.done, a.packed + off + k, v);
   }
 }
 
@@ -1184,7 +1259,7 @@ __device__ __forceinline__ void sort_lists_block(const FinalizeArgs& a, int b) {
   const int lane = threadIdx.x & 63;
   const int w = threadIdx.x >> 6;
   const int i = b * 4 + w;
-  const bool valid = i < a.cd->ni;
+  const bool valid = i < call_ni(a);
   const int c = valid ? min(a.ngb_cnt[i], NGB_CAP) : 0;
   for (int k = lane; k < c; k += 64) lst[w][k] = a.ngb_list[(size_t)i * NGB_CAP + k];
   if (lane == 0) cnts[w] = c;
@@ -1200,7 +1275,7 @@ __device__ __forceinline__ void sort_lists_block(const FinalizeArgs& a, int b) {
     off = base;
     for (int u = 0; u < w; ++u) off += cnts[u];
   }
-  if (valid && lane == 0) a.list_off[i] = off;
+  if (valid && lane == 0) put_host(a.done, a.list_off + i, off);
   store_list(a, i, srt[w], c, off, lane, 64);
 }
 
@@ -1213,33 +1288,38 @@ template <int ORDER, bool F64, int U>
 __global__ __launch_bounds__(256) void k_finalize(FinalizeArgs a, int nfin) {
   if ((int)blockIdx.x < nfin) finalize_block<ORDER, F64, U>(a, blockIdx.x);
   else sort_lists_block(a, blockIdx.x - nfin);
+  if (a.done) finish_word(a.done, a.done_ctr, a.cd ? a.cd->seq : a.seq);
 }
 
 // ---------------------------------------------------------------------------
-// Predicted-state gather for read-back: per j, 10 doubles
-// (x, y, z, m, vx, vy, vz, ax, ay, az) in FP64, plus the id in the m slot's
-// companion array handled by the host.
+// Predicted-state gather for read-back: 10 doubles per j (x, y, z, m, vx, vy, vz,
+// ax, ay, az) in FP64, field-major, so that a wave's stores are whole lines also
+// where out is host memory (then with a completion word: with copy commands for
+// the addresses and the rows, 2500 addresses took 90 us, the kernel 6).
 template <int ORDER, bool F64>
 __global__ __launch_bounds__(256) void k_gather_pred(GatherArgs a) {
   using Rec = typename RecOf<ORDER, F64>::T;
   const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= a.n) return;
-  const int j = a.addr ? a.addr[k] : k;
-  const Rec r = reinterpret_cast<const Rec*>(a.st.rec)[j];
-  const size_t cap = (size_t)a.st.cap;
-  double* o = a.out + (size_t)k * 10;
-  o[3] = a.st.raw[RF_M * cap + j];
-  if constexpr (F64) {
-    o[0] = r.x; o[1] = r.y; o[2] = r.z;
-    o[4] = r.vx; o[5] = r.vy; o[6] = r.vz;
-    if constexpr (ORDER >= ORDER_H6) { o[7] = r.ax; o[8] = r.ay; o[9] = r.az; }
-    else { o[7] = o[8] = o[9] = 0.0; }
-  } else {
-    o[0] = a.st.ppos[j]; o[1] = a.st.ppos[cap + j]; o[2] = a.st.ppos[2 * cap + j];
-    o[4] = a.st.pvel[j]; o[5] = a.st.pvel[cap + j]; o[6] = a.st.pvel[2 * cap + j];
-    if constexpr (ORDER >= ORDER_H6) { o[7] = a.st.pacc[j]; o[8] = a.st.pacc[cap + j]; o[9] = a.st.pacc[2 * cap + j]; }
-    else { o[7] = o[8] = o[9] = 0.0; }
+  if (k < a.n) {
+    const int j = a.addr ? a.addr[k] : k;
+    const Rec r = reinterpret_cast<const Rec*>(a.st.rec)[j];
+    const size_t cap = (size_t)a.st.cap;
+    double v[10];
+    v[3] = a.st.raw[RF_M * cap + j];
+    v[7] = v[8] = v[9] = 0.0;
+    if constexpr (F64) {
+      v[0] = r.x; v[1] = r.y; v[2] = r.z;
+      v[4] = r.vx; v[5] = r.vy; v[6] = r.vz;
+      if constexpr (ORDER >= ORDER_H6) { v[7] = r.ax; v[8] = r.ay; v[9] = r.az; }
+    } else {
+      v[0] = a.st.ppos[j]; v[1] = a.st.ppos[cap + j]; v[2] = a.st.ppos[2 * cap + j];
+      v[4] = a.st.pvel[j]; v[5] = a.st.pvel[cap + j]; v[6] = a.st.pvel[2 * cap + j];
+      if constexpr (ORDER >= ORDER_H6) { v[7] = a.st.pacc[j]; v[8] = a.st.pacc[cap + j]; v[9] = a.st.pacc[2 * cap + j]; }
+    }
+#pragma unroll
+    for (int f = 0; f < 10; ++f) put_host(a.done, a.out + (size_t)f * a.n + k, v[f]);
   }
+  if (a.done) finish_word(a.done, a.done_ctr, a.seq);
 }
 
 __global__ void k_write_desc(CallDesc* cd, CallDesc v) { *cd = v; }
