@@ -152,7 +152,7 @@ struct ForceArgs {
 // ni and eps2 come by value (f.cd would be one more read over PCIe before them).
 // A few addresses (SMALL_ARG) come as arguments, more through the bit set and the
 // rows' own (address, id) pairs, two more reads over PCIe before the rows.
-constexpr int SMALL_NI = 32, SMALL_UPD = 256, SMALL_ARG = 16;
+constexpr int SMALL_NI = 64, SMALL_UPD = 256, SMALL_ARG = 16;
 struct SmallArgs {
   ForceArgs f;
   int tiles;              // tiles of 256 j per work-group
@@ -188,7 +188,7 @@ inline int partial_rows(const ForceConfig& c) { return (c.S % 4 == 0 && !c.smajo
 // calls of one ni take the same).  A launch of ~16384 threads or more keeps the
 // row reads in flight: with 4 threads each, 1000 i-particles of 128 rows took
 // 23 us.
-constexpr int finalize_threads(int bucket) { return bucket > 4096 ? 4 : bucket > 512 ? 16 : bucket > 32 ? 64 : 256; }
+constexpr int finalize_threads(int bucket) { return bucket > 4096 ? 4 : bucket > 512 ? 16 : bucket > 64 ? 64 : 256; }
 
 // Results and neighbour lists go straight to host-mapped pinned memory (no
 // copy command): field-major result rows out[f * ostride + i], and each sorted

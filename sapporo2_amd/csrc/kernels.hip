@@ -338,23 +338,25 @@ __device__ __forceinline__ bool pair(const Rec& r, const int j, const bool ok, c
     const R day = r.ay - s.ay;
     const R daz = r.az - s.az;
     const R v2 = fmaR<R>(dvz, dvz, fmaR<R>(dvy, dvy, dvx * dvx));
-    const R ra = fmaR<R>(dz, daz, fmaR<R>(dy, day, dx * dax));
+    const R v2ra = fmaR<R>(dz, daz, fmaR<R>(dy, day, fmaR<R>(dx, dax, v2)));
     const R alpha = rv * invr2;
-    const R beta = fmaR<R>(v2 + ra, invr2, alpha * alpha);
+    const R beta = fmaR<R>(v2ra, invr2, alpha * alpha);
     const R m3a = alpha * R(-3);
-    // jerk_ij = m/r^3 (dv - 3 alpha dr)
-    const R jx = mr3 * fmaR<R>(m3a, dx, dvx);
-    const R jy = mr3 * fmaR<R>(m3a, dy, dvy);
-    const R jz = mr3 * fmaR<R>(m3a, dz, dvz);
-    // snap_ij = m/r^3 (da - 3 beta dr) - 6 alpha jerk_ij
+    // jerk_ij = m/r^3 w, w = dv - 3 alpha dr
+    const R wx = fmaR<R>(m3a, dx, dvx);
+    const R wy = fmaR<R>(m3a, dy, dvy);
+    const R wz = fmaR<R>(m3a, dz, dvz);
+    t[4] = fmaR<R>(mr3, wx, t[4]);
+    t[5] = fmaR<R>(mr3, wy, t[5]);
+    t[6] = fmaR<R>(mr3, wz, t[6]);
+    // snap_ij = m/r^3 (da - 3 beta dr) - 6 alpha jerk_ij; the products are formed
+    // inside the sums (58.75 operations a pair, 61.75 with jerk_ij and v^2 + dr.da
+    // as values of their own)
     const R m3b = beta * R(-3);
-    const R m6a = alpha * R(-6);
-    t[7] = fmaR<R>(m6a, jx, fmaR<R>(mr3, fmaR<R>(m3b, dx, dax), t[7]));
-    t[8] = fmaR<R>(m6a, jy, fmaR<R>(mr3, fmaR<R>(m3b, dy, day), t[8]));
-    t[9] = fmaR<R>(m6a, jz, fmaR<R>(mr3, fmaR<R>(m3b, dz, daz), t[9]));
-    t[4] = t[4] + jx;
-    t[5] = t[5] + jy;
-    t[6] = t[6] + jz;
+    const R m6 = (alpha * mr3) * R(-6);
+    t[7] = fmaR<R>(m6, wx, fmaR<R>(mr3, fmaR<R>(m3b, dx, dax), t[7]));
+    t[8] = fmaR<R>(m6, wy, fmaR<R>(mr3, fmaR<R>(m3b, dy, day), t[8]));
+    t[9] = fmaR<R>(m6, wz, fmaR<R>(mr3, fmaR<R>(m3b, dz, daz), t[9]));
   }
   // nearest neighbour: strict <, first address wins inside a lane (kernels.cu:539-546)
   if constexpr (BLOCKMIN) {
@@ -1113,32 +1115,36 @@ __device__ __forceinline__ void write_row(const FinalizeArgs& a, int i, const do
   write_nn<ORDER, F64>(a, i, ds, ad, cnt);
 }
 
-// Rank sort of c ids staged in s[0..c) by one wave, written to dst.  s is 16-byte
-// aligned and padded to a multiple of four: a lane ranks its (up to four) ids
-// against four at a time, one LDS read for all of them (a full list of 256: 30 us
-// with one read per comparison).
-__device__ __forceinline__ void wave_rank_sort(const int* s, int c, int lane, int* dst) {
+// Key of list entry k: orders by id, equal ids by k.
+__device__ __forceinline__ unsigned long long list_key(int id, int k) {
+  return ((unsigned long long)((unsigned)id ^ 0x80000000u) << 32) | (unsigned)k;
+}
+
+// Rank sort of c ids by one wave, written to dst: s[0..c) holds their keys, padded
+// to a multiple of four with ~0.  A lane ranks its (up to four) ids against four
+// at a time, one compare and one add each; a full list of 256 took 30 us with
+// one LDS read and an index test per comparison.
+__device__ __forceinline__ void wave_rank_sort(const unsigned long long* s, int c, int lane, int* dst) {
   constexpr int M = NGB_CAP / 64;
-  int v[M], rank[M];
+  unsigned long long v[M];
+  int rank[M];
 #pragma unroll
   for (int m = 0; m < M; ++m) {
-    v[m] = lane + 64 * m < c ? s[lane + 64 * m] : 0;
+    v[m] = lane + 64 * m < c ? s[lane + 64 * m] : 0ull;
     rank[m] = 0;
   }
   for (int q = 0; q < c; q += 4) {
-    const int4 w = *reinterpret_cast<const int4*>(s + q);
-    const int u[4] = {w.x, w.y, w.z, w.w};
+    const unsigned long long u[4] = {s[q], s[q + 1], s[q + 2], s[q + 3]};
 #pragma unroll
     for (int m = 0; m < M; ++m) {
       if (64 * m >= c) break;  // uniform
 #pragma unroll
-      for (int e = 0; e < 4; ++e)
-        rank[m] += q + e < c && (u[e] < v[m] || (u[e] == v[m] && q + e < lane + 64 * m)) ? 1 : 0;
+      for (int e = 0; e < 4; ++e) rank[m] += u[e] < v[m] ? 1 : 0;
     }
   }
 #pragma unroll
   for (int m = 0; m < M; ++m)
-    if (lane + 64 * m < c) dst[rank[m]] = v[m];
+    if (lane + 64 * m < c) dst[rank[m]] = (int)((unsigned)(v[m] >> 32) ^ 0x80000000u);
 }
 
 // U threads per i-particle, 256 / U consecutive i-particles per work-group (a
@@ -1252,7 +1258,7 @@ __device__ __forceinline__ void store_list(const FinalizeArgs& a, int i, const i
 // four lists of a work-group taking their offsets with one atomic on the
 // call's counter.
 __device__ __forceinline__ void sort_lists_block(const FinalizeArgs& a, int b) {
-  __shared__ __align__(16) int lst[4][NGB_CAP];
+  __shared__ __align__(16) unsigned long long lst[4][NGB_CAP];
   __shared__ int srt[4][NGB_CAP];
   __shared__ int cnts[4];
   __shared__ int base;
@@ -1261,7 +1267,8 @@ __device__ __forceinline__ void sort_lists_block(const FinalizeArgs& a, int b) {
   const int i = b * 4 + w;
   const bool valid = i < call_ni(a);
   const int c = valid ? min(a.ngb_cnt[i], NGB_CAP) : 0;
-  for (int k = lane; k < c; k += 64) lst[w][k] = a.ngb_list[(size_t)i * NGB_CAP + k];
+  for (int k = lane; k < (c + 3) / 4 * 4; k += 64)
+    lst[w][k] = k < c ? list_key(a.ngb_list[(size_t)i * NGB_CAP + k], k) : ~0ull;
   if (lane == 0) cnts[w] = c;
   __syncthreads();
   if (threadIdx.x == 0 && !a.inorder) {

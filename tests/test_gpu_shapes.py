@@ -43,7 +43,7 @@ def test_counts_at_shape_edges(order, prec):
         load_engine(eng, m, x, v, ids, np.zeros((n, 3)), np.zeros((n, 3)),
                     *([np.zeros((n, 3))] * 2 if order >= sa.SIXTH else [None, None]))
         eng.set_time(0.0)
-        for ni, nj in [(1, 1), (1, 255), (2, 256), (3, 257), (5, 4097), (8, 1000), (17, 9000), (31, 2047), (32, 8991), (33, 1), (33, 15), (40, 16), (64, 17), (65, 63), (65, 80), (128, 1000), (129, 4097), (512, 8991),
+        for ni, nj in [(1, 1), (1, 255), (2, 256), (3, 257), (5, 4097), (8, 1000), (17, 9000), (31, 2047), (32, 8991), (63, 5000), (33, 1), (33, 15), (40, 16), (64, 17), (65, 63), (65, 80), (128, 1000), (129, 4097), (512, 8991),
                        (513, 9000), (1025, 2047), (4097, 3000)]:
             sel = np.sort(rng.choice(n, ni, replace=False))
             _check(eng, order, prec, sys_, sel, nj, ni % 2 == 1, f"shapes order={order} prec={prec} ni={ni} nj={nj}")
