@@ -33,6 +33,9 @@ namespace {
 constexpr int WAVES_PER_SIMD_TARGET = 32;   // several dispatch rounds balance better
 constexpr int MIN_ITERS_PER_LANE = 16;
 constexpr int MIN_J_PER_SPLIT = 512;
+// Ensembles: smallest split, and the active count from which a cluster takes lane
+// shape P = 64 (whose records come through the scalar cache) rather than 16.
+constexpr int ENS_MIN_CHUNK = 64, ENS_P64 = 16;
 // Launch shapes of lane shape P = 64 (choose_config)
 constexpr int SMALL_ROWS = 512;
 // Calls up to these counts complete by the finalize's word, larger ones by an
@@ -1017,7 +1020,7 @@ int Engine::start_grav_calc_clusters(int ni, const int* cluster, const int* id, 
     const int i = starts[q], e = q + 1 < starts.size() ? starts[q + 1] : ni;
     const int c = cluster[i];
     const int n = e - i;
-    const int P = n > 32 ? 64 : n > 8 ? 16 : n > 2 ? 4 : 1;
+    const int P = n > ENS_P64 ? 64 : n > 8 ? 16 : n > 2 ? 4 : 1;
     grps.push_back(EnsGroup{i, n, P, 0, 0, 0});
     gcl.push_back(c);
     work += (long)((n + P - 1) / P) * cl_n_[c];
@@ -1062,18 +1065,25 @@ int Engine::start_grav_calc_clusters(int ni, const int* cluster, const int* id, 
   }
 
   // work table: per active cluster, i-groups of P (by its active count) x j-splits
-  const long target = (long)cus_ * 4 * WAVES_PER_SIMD_TARGET;
-  const long jraw = std::max<long>(MIN_J_PER_SPLIT, (work + target - 1) / target);
-  // j per split in whole 64-interaction folds of a lane: JTILE for lane shape
-  // P = 64 (one j-lane per i-particle), 16 tiles for the smaller shapes (Q <= 16)
-  const long jch64 = (jraw + JTILE - 1) / JTILE * JTILE;
-  const long jchs = (jraw + JTILE * 16 - 1) / (JTILE * 16) * (JTILE * 16);
+  // j per split: one round of waves while that leaves an item ENS_MIN_CHUNK j, up
+  // to MIN_J_PER_SPLIT, then as many rounds as WAVES_PER_SIMD_TARGET allows (the
+  // host builds the table item by item).  26 of ~400 particles active in each of
+  // 100 clusters took 152 us in splits of 1024 j.  A split is whole sub-blocks of
+  // its lane shape's Q j-lanes.
+  const long round = (long)cus_ * 4 * 8, target = (long)cus_ * 4 * WAVES_PER_SIMD_TARGET;
+  const long jraw = std::max(std::min<long>(MIN_J_PER_SPLIT, std::max<long>(ENS_MIN_CHUNK, (work + round - 1) / round)),
+                             (work + target - 1) / target);
+  auto chunk = [&](int P) {
+    const long unit = P == 64 ? JTILE : 64 / P * FORCE_SUB;
+    return (jraw + unit - 1) / unit * unit;
+  };
+  const long jch64 = chunk(64);
   // items of lane shape P = 64 first, the smaller shapes after them: each part
   // runs in a kernel of its own, so the P = 64 part keeps its register budget
   int n64 = 0, nsm = 0;
   for (size_t q = 0; q < grps.size(); ++q) {
     EnsGroup& g = grps[q];
-    const long jch = g.P == 64 ? jch64 : jchs;
+    const long jch = chunk(g.P);
     g.S = std::max(1, (int)((cl_n_[gcl[q]] + jch - 1) / jch));
     (g.P == 64 ? n64 : nsm) += (g.n + g.P - 1) / g.P * g.S;
   }
@@ -1100,7 +1110,7 @@ int Engine::start_grav_calc_clusters(int ni, const int* cluster, const int* id, 
   for (int q = 0; q < ng; ++q) {
     const EnsGroup& g = grps[q];
     const int c = gcl[q], off = cl_off_[c], nj = cl_n_[c];
-    const long jch = g.P == 64 ? jch64 : jchs;
+    const long jch = chunk(g.P);
     EnsItem* it = items + g.first;
     for (int i0 = g.ib; i0 < g.ib + g.n; i0 += g.P) {
       const int cnt = std::min(g.P, g.ib + g.n - i0);
@@ -1161,6 +1171,7 @@ int Engine::start_grav_calc_clusters(int ni, const int* cluster, const int* id, 
   ea.ngb_cnt = cnt_d_;
   ea.ngb_list = list_d_;
   ea.ngb_on = ngb_on ? 1 : 0;
+  ea.ahead = n64 <= AHEAD_WAVES ? 1 : 0;
   FinalizeArgs fz = finalize_args(ni, ngb_on);
   fz.inorder = 0;  // ensembles: packed lists (NGB_CAP per i-particle would not fit)
   if (timing_) HIPCHK(hipEventRecord(ev_f0_, stream_), "event");

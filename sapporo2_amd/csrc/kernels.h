@@ -240,6 +240,7 @@ struct EnsArgs {
   const int4* idesc;         // per i: first item, number of splits, i-slot
   double* part; double* part_ds2; int* part_addr;   // part_fields x nitems x 64, nitems x 64
   int* ngb_cnt; int* ngb_list; int ngb_on;
+  int ahead;                 // P = 64 items load their records ahead
 };
 
 // Gathers the FP64 predicted state (pos, mass, vel, [acc]) for read-back, 10 x n

@@ -964,7 +964,7 @@ __device__ __forceinline__ void write_row(const FinalizeArgs& a, int i, const do
 // that is its i-particles' only split writes their result rows (over PCIe,
 // while other items still compute) as the finalize would: the finalize's
 // sum over one split is 0.0 + T, and its nearest neighbour the item's own.
-template <int ORDER, bool F64, int P, bool NGB>
+template <int ORDER, bool F64, int P, bool NGB, bool AHEAD = false>
 __device__ __forceinline__ void ens_item(const EnsArgs& a, const FinalizeArgs& fz,
                                          const typename RecOf<ORDER, F64>::T* __restrict__ rec, const EnsItem& it,
                                          int item) {
@@ -973,7 +973,7 @@ __device__ __forceinline__ void ens_item(const EnsArgs& a, const FinalizeArgs& f
   double dsd;
   int nnaddr, islot;
   bool writer;
-  wave_force<ORDER, F64, P, NGB>(rec, a.idr, a.ipos, a.ivel, a.iacc, a.ih2, a.iid,
+  wave_force<ORDER, F64, P, NGB, false, AHEAD>(rec, a.idr, a.ipos, a.ivel, a.iacc, a.ih2, a.iid,
                                  it.i0, it.icount, it.jb, it.je, a.eps2[it.cluster], a.ngb_cnt, a.ngb_list, T,
                                  dsd, nnaddr, islot, writer);
   if (!NGB && it.nsplit == 1) {
@@ -1000,7 +1000,7 @@ __device__ __forceinline__ void ens_item(const EnsArgs& a, const FinalizeArgs& f
 // groups in order as wave slots free up, so the short items fill the end of
 // the launch with no queue to contend for.  (A counter that every wave bumped
 // for its next item serialised the small items of large ensembles.)
-template <int ORDER, bool F64, bool NGB, bool P64>
+template <int ORDER, bool F64, bool NGB, bool P64, bool AHEAD>
 __global__ __launch_bounds__(64) void k_force_ens(EnsArgs a, FinalizeArgs fz,
                                                   const typename RecOf<ORDER, F64>::T* __restrict__ rec, int ib,
                                                   int ie) {
@@ -1021,7 +1021,7 @@ __global__ __launch_bounds__(64) void k_force_ens(EnsArgs a, FinalizeArgs fz,
   it.nsplit = __builtin_amdgcn_readfirstlane(ld.nsplit);
   it.pad = 0;
   if constexpr (P64) {
-    ens_item<ORDER, F64, 64, NGB>(a, fz, rec, it, item);
+    ens_item<ORDER, F64, 64, NGB, AHEAD>(a, fz, rec, it, item);
   } else {
     switch (it.P) {
       case 16: ens_item<ORDER, F64, 16, NGB>(a, fz, rec, it, item); break;
@@ -1471,23 +1471,23 @@ int launch_finalize(hipStream_t s, int order, bool f64, const FinalizeArgs& a) {
 
 int launch_force_ens(hipStream_t s, int order, bool f64, const EnsArgs& a, const FinalizeArgs& f, int n64) {
   if (a.nitems <= 0 || f.grid_ni <= 0) return 0;
-  const int nsmall = a.nitems - n64;
   dispatch_op(order, f64, [&](auto OR, auto FP) {
     constexpr int O = decltype(OR)::value;
     constexpr bool F = decltype(FP)::value;
     const auto* rec = reinterpret_cast<const typename RecOf<O, F>::T*>(a.rec);
-    if (n64 > 0) {
-      if (a.ngb_on)
-        hipLaunchKernelGGL((k_force_ens<O, F, true, true>), dim3(n64), dim3(64), 0, s, a, f, rec, 0, n64);
-      else
-        hipLaunchKernelGGL((k_force_ens<O, F, false, true>), dim3(n64), dim3(64), 0, s, a, f, rec, 0, n64);
-    }
-    if (nsmall > 0) {
-      if (a.ngb_on)
-        hipLaunchKernelGGL((k_force_ens<O, F, true, false>), dim3(nsmall), dim3(64), 0, s, a, f, rec, n64, a.nitems);
-      else
-        hipLaunchKernelGGL((k_force_ens<O, F, false, false>), dim3(nsmall), dim3(64), 0, s, a, f, rec, n64, a.nitems);
-    }
+    auto part = [&](auto ngb, auto p64, auto ahead, int ib, int ie) {
+      constexpr bool N = decltype(ngb)::value, P = decltype(p64)::value, A = decltype(ahead)::value;
+      if (ie > ib) hipLaunchKernelGGL((k_force_ens<O, F, N, P, A>), dim3(ie - ib), dim3(64), 0, s, a, f, rec, ib, ie);
+    };
+    auto both = [&](auto ngb) {
+      // records ahead as in the single-system launches: FP64 always, mixed where
+      // the waves leave SIMDs half empty
+      if (F || a.ahead) part(ngb, std::true_type{}, std::true_type{}, 0, n64);
+      else if constexpr (!F) part(ngb, std::true_type{}, std::false_type{}, 0, n64);
+      part(ngb, std::false_type{}, std::false_type{}, n64, a.nitems);
+    };
+    if (a.ngb_on) both(std::true_type{});
+    else both(std::false_type{});
     hipLaunchKernelGGL((k_finalize_ens<O, F>), dim3(blocks_for(f.grid_ni, 256)), dim3(256), 0, s, f, a);
     if (f.ngb_on) hipLaunchKernelGGL(k_sort_lists, dim3(blocks_for(f.grid_ni, 4)), dim3(256), 0, s, f);
   });
