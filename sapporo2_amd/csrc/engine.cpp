@@ -36,6 +36,7 @@ constexpr int MIN_J_PER_SPLIT = 512;
 // Ensembles: smallest split, and the active count from which a cluster takes lane
 // shape P = 64 (whose records come through the scalar cache) rather than 16.
 constexpr int ENS_MIN_CHUNK = 64, ENS_P64 = 16;
+constexpr int ENS_DMA_I = 1 << 18;
 // Launch shapes of lane shape P = 64 (choose_config)
 constexpr int SMALL_ROWS = 512;
 // Calls up to these counts complete by the finalize's word, larger ones by an
@@ -96,6 +97,9 @@ hipError_t hmap(T** h, T** d, size_t n, bool coherent) {
   const hipError_t e = hipHostMalloc(reinterpret_cast<void**>(h), n * sizeof(T), flags);
   if (e != hipSuccess) return e;
   return hipHostGetDevicePointer(reinterpret_cast<void**>(d), *h, 0);
+}
+inline CopySeg seg16(const void* host_mapped, void* dev, size_t bytes) {
+  return CopySeg{static_cast<const int4*>(host_mapped), static_cast<int4*>(dev), (int)((bytes + 15) / 16)};
 }
 template <typename T>
 void dfree(T*& p) {
@@ -226,7 +230,7 @@ int Engine::close() {
   slot_lists_h_.clear();
   dfree(gather_d_); gather_cap_ = 0;
   hfree(gather_h_); hfree(gaddr_h_); gather_hd_ = nullptr; gaddr_hd_ = nullptr; gather_hcap_ = 0;
-  dfree(idesc_d_); dfree(ens_eps_d_); ens_eps_cap_ = 0;
+  dfree(idesc_d_);
   hfree(ens_tab_h_); dfree(ens_tab_d_); ens_tab_cap_ = 0;
   icap_ = 0; cl_off_.clear(); cl_n_.clear(); cl_total_ = 0;
   for (hipEvent_t* e : {&ev_done_, &ev_d0_, &ev_d1_, &ev_f0_, &ev_f1_, &ev_p0_, &ev_p1_, &ev_s0_, &ev_s1_}) {
@@ -615,7 +619,7 @@ void Engine::hand_over() {
 // Staged updates, prediction of [0, pred_j1) and, for a force call, its call
 // block and counter reset (k_prep).  by_call: the caller records the call's
 // completion next, and the stage is free with it.
-int Engine::prep(int pred_j1, int call_bytes, int ni_reset, bool by_call) {
+int Engine::prep(int pred_j1, int call_bytes, int ni_reset, bool by_call, const CopySeg* more, int nmore) {
   const int n = nstaged_;
   if (n > 0 && ensure_store(max_addr_ + 1) != 0) return -1;
   Stage& sg = stage_[cur_];
@@ -632,9 +636,8 @@ int Engine::prep(int pred_j1, int call_bytes, int ni_reset, bool by_call) {
   a.new_ids = new_ids_ ? 1 : 0;
   a.ti = t_i_;
   a.pred_j1 = pred_j1;
-  a.call_h = reinterpret_cast<const int4*>(call_hd_);
-  a.call_d = reinterpret_cast<int4*>(call_d_);
-  a.call_n16 = (call_bytes + 15) / 16;
+  a.seg[0] = seg16(call_hd_, call_d_, call_bytes);
+  for (int k = 0; k < nmore; ++k) a.seg[1 + k] = more[k];
   a.ngb_cnt = cnt_d_;
   a.ni_reset = ni_reset;
   a.pack_ctr = pack_ctr_d_;
@@ -649,7 +652,8 @@ int Engine::prep(int pred_j1, int call_bytes, int ni_reset, bool by_call) {
     if (ev) HIPCHK(hipEventRecord(ev_s1_, stream_), "event");
     timed_scatter_ = ev;
     last_nupd_ = n;
-    a.nupd = a.call_n16 = a.ni_reset = a.nbits = 0;
+    a.nupd = a.ni_reset = a.nbits = 0;
+    for (CopySeg& g : a.seg) g.n16 = 0;
   }
   if (ev) HIPCHK(hipEventRecord(ev_p0_, stream_), "event");
   if (launch_prep(stream_, order_, f64_, a) != 0) return fail("prep launch", hipGetLastError());
@@ -834,10 +838,10 @@ int Engine::ensure_icap(int need) {
   hfree(ibuf_h_); hfree(iid_h_); dfree(ibuf_d_); dfree(iid_d_);
   hfree(res_h_); hfree(loff_h_); dfree(cnt_d_); dfree(idesc_d_);
   const size_t nI = (size_t)need;
-  HIPCHK(hmalloc(&ibuf_h_, IBUF_FIELDS * nI), "pinned i buffer");
-  HIPCHK(hmalloc(&iid_h_, nI), "pinned i ids");
+  HIPCHK(hmap(&ibuf_h_, &ibuf_hd_, IBUF_FIELDS * nI, true), "pinned i buffer");
+  HIPCHK(hmap(&iid_h_, &iid_hd_, nI + 4, true), "pinned i ids");  // whole 16-byte units
   HIPCHK(dmalloc(&ibuf_d_, IBUF_FIELDS * nI), "i buffer");
-  HIPCHK(dmalloc(&iid_d_, nI), "i ids");
+  HIPCHK(dmalloc(&iid_d_, nI + 4), "i ids");
   HIPCHK(hmap(&res_h_, &res_hd_, nI * out_fields(order_), coherent_), "host-mapped results");
   res_stride_ = (long)nI;
   HIPCHK(hmap(&loff_h_, &loff_hd_, nI, coherent_), "host-mapped list offsets");
@@ -1042,13 +1046,16 @@ int Engine::start_grav_calc_clusters(int ni, const int* cluster, const int* id, 
   double* bv = bx + 3 * (size_t)ni;
   double* ba = bv + 3 * (size_t)ni;
   double* bh = ba + (order_ >= ORDER_H6 ? 3 * (size_t)ni : 0);
-  // Large calls pack and upload in chunks: each chunk's copies are queued as
-  // soon as it is packed, so the transfer overlaps the packing of the rest.
+  // k_prep copies the packed inputs and the work table in the launch that predicts
+  // (with copy commands, 99436 i took 300 us for 90 us worth of transfer).  From
+  // ENS_DMA_I on packing takes long enough that chunks, each copied as soon as it
+  // is packed, are faster.
   const bool h6 = order_ >= ORDER_H6;
-  const int nchunk = ni >= (1 << 18) ? 4 : ni >= (1 << 16) ? 2 : 1;
+  const bool dma = ni >= ENS_DMA_I;
   bool ngb_on = false;
-  for (int k = 0; k < nchunk; ++k) {
-    const int b = (int)((long)ni * k / nchunk), e = (int)((long)ni * (k + 1) / nchunk);
+  if (!dma) ngb_on = pack_i(0, ni, id, xi, vi, ai, h2, bx, bv, ba, bh, iid_h_);
+  for (int k = 0; dma && k < 4; ++k) {
+    const int b = (int)((long)ni * k / 4), e = (int)((long)ni * (k + 1) / 4);
     ngb_on |= pack_i(b, e, id, xi, vi, ai, h2, bx, bv, ba, bh, iid_h_);
     const size_t n = (size_t)(e - b);
     auto up = [&](const double* h) {
@@ -1097,12 +1104,13 @@ int Engine::start_grav_calc_clusters(int ni, const int* cluster, const int* id, 
   const int ng = (int)grps.size();
   auto al = [](size_t b) { return (b + 255) / 256 * 256; };
   const size_t o_order = al(sizeof(EnsItem) * nitems), o_grp = o_order + al(sizeof(int) * nitems);
-  const size_t tab_bytes = o_grp + sizeof(EnsGroup) * ng;
+  const size_t o_eps = o_grp + al(sizeof(EnsGroup) * ng);
+  const size_t tab_bytes = o_eps + al(sizeof(double) * nc);
   if (tab_bytes > ens_tab_cap_) {
     hfree(ens_tab_h_);
     dfree(ens_tab_d_);
     ens_tab_cap_ = std::max(tab_bytes, 2 * ens_tab_cap_);
-    HIPCHK(hmalloc(&ens_tab_h_, ens_tab_cap_), "ensemble work table (host)");
+    HIPCHK(hmap(&ens_tab_h_, &ens_tab_hd_, ens_tab_cap_, true), "ensemble work table (host)");
     HIPCHK(dmalloc(&ens_tab_d_, ens_tab_cap_), "ensemble work table");
   }
   EnsItem* items = reinterpret_cast<EnsItem*>(ens_tab_h_);
@@ -1122,6 +1130,7 @@ int Engine::start_grav_calc_clusters(int ni, const int* cluster, const int* id, 
     }
   }
   memcpy(ens_tab_h_ + o_grp, grps.data(), sizeof(EnsGroup) * ng);
+  memcpy(ens_tab_h_ + o_eps, eps2c, sizeof(double) * nc);
   // launch order: longest j-range first within each part, equal lengths in
   // table order (a stable counting sort on the length)
   auto order_part = [&](int k0, int k1) {
@@ -1134,23 +1143,18 @@ int Engine::start_grav_calc_clusters(int ni, const int* cluster, const int* id, 
   };
   order_part(0, n64);
   order_part(n64, nitems);
-  if (ens_eps_cap_ < nc) {
-    dfree(ens_eps_d_);
-    ens_eps_cap_ = nc;
-    HIPCHK(dmalloc(&ens_eps_d_, (size_t)nc), "ensemble softening");
-  }
-  HIPCHK(hipMemcpyAsync(ens_tab_d_, ens_tab_h_, tab_bytes, hipMemcpyHostToDevice, stream_), "work table upload");
-  HIPCHK(hipMemcpyAsync(ens_eps_d_, eps2c, sizeof(double) * nc, hipMemcpyHostToDevice, stream_), "eps upload");
-  if (launch_ens_idesc(stream_, reinterpret_cast<const EnsGroup*>(ens_tab_d_ + o_grp), ng, ni, idesc_d_) != 0)
-    return fail("ensemble descriptor launch", hipGetLastError());
-
   if (desc_pending_ && desc_seq_ > done_seq_) HIPCHK(hipEventSynchronize(ev_desc_), "descriptor wait");
   desc_pending_ = false;
   *desc_h_ = CallDesc{t_i_, 0.0, ni, 0, 0, 0};
   done_word_ = false;
   if (timing_) HIPCHK(hipEventRecord(ev_d0_, stream_), "event");
-  if (prep(predict_ ? cl_total_ : 0, (int)sizeof(CallDesc), ngb_on ? ni : 0, true) != 0) return -1;
+  const CopySeg in[3] = {seg16(ens_tab_hd_, ens_tab_d_, tab_bytes),
+                         seg16(ibuf_hd_, ibuf_d_, sizeof(double) * (size_t)((h2 ? bh + ni : bh) - bx)),
+                         seg16(iid_hd_, iid_d_, sizeof(int) * (size_t)ni)};
+  if (prep(predict_ ? cl_total_ : 0, (int)sizeof(CallDesc), ngb_on ? ni : 0, true, in, dma ? 1 : 3) != 0) return -1;
   predict_ = false;
+  if (launch_ens_idesc(stream_, reinterpret_cast<const EnsGroup*>(ens_tab_d_ + o_grp), ng, ni, idesc_d_) != 0)
+    return fail("ensemble descriptor launch", hipGetLastError());
   if (ensure_partials((size_t)nitems * 64) != 0) return -1;
   EnsArgs ea{};
   ea.rec = st_.rec;
@@ -1160,7 +1164,7 @@ int Engine::start_grav_calc_clusters(int ni, const int* cluster, const int* id, 
   ea.iacc = ibuf_d_ + 6 * (size_t)ni;
   ea.ih2 = ibuf_d_ + (bh - bx);
   ea.iid = iid_d_;
-  ea.eps2 = ens_eps_d_;
+  ea.eps2 = reinterpret_cast<const double*>(ens_tab_d_ + o_eps);
   ea.items = reinterpret_cast<const EnsItem*>(ens_tab_d_);
   ea.nitems = nitems;
   ea.order = reinterpret_cast<const int*>(ens_tab_d_ + o_order);

@@ -140,7 +140,8 @@ class Engine {
   int stage_block(int n, const int* addr, const int* id, const F& fill);
   int stage_row(int addr, int id);
   void hand_over();
-  int prep(int pred_j1, int call_bytes, int ni_reset, bool by_call);
+  int prep(int pred_j1, int call_bytes, int ni_reset, bool by_call, const sapk::CopySeg* more = nullptr,
+           int nmore = 0);
   int predict_range(int j0, int j1);
   bool pack_i(int i0, int i1, const int* id, const double (*xi)[3], const double (*vi)[3], const double (*ai)[3],
               const double* h2, double* bx, double* bv, double* ba, double* bh, int* bid);
@@ -207,7 +208,7 @@ class Engine {
   bool predict_ = false;
 
   // i-particles and results
-  double* ibuf_h_ = nullptr; int* iid_h_ = nullptr;
+  double* ibuf_h_ = nullptr; double* ibuf_hd_ = nullptr; int* iid_h_ = nullptr; int* iid_hd_ = nullptr;
   double* ibuf_d_ = nullptr; int* iid_d_ = nullptr;
   double* part_d_ = nullptr; double* pds2_d_ = nullptr; int* paddr_d_ = nullptr;
   size_t part_cap_ = 0;
@@ -273,9 +274,8 @@ class Engine {
   int cl_total_ = 0;
   // work table of an ensemble call: [items | launch order | groups], built in
   // pinned host memory and uploaded with one copy
-  char* ens_tab_h_ = nullptr; char* ens_tab_d_ = nullptr; size_t ens_tab_cap_ = 0;
+  char* ens_tab_h_ = nullptr; char* ens_tab_hd_ = nullptr; char* ens_tab_d_ = nullptr; size_t ens_tab_cap_ = 0;
   int4* idesc_d_ = nullptr;
-  double* ens_eps_d_ = nullptr; int ens_eps_cap_ = 0;
 
   struct TuneEntry { int order, prec, ngb, li, lj, P, jlog; };
   std::vector<TuneEntry> tune_;

@@ -106,11 +106,14 @@ struct PredictArgs {
 };
 
 // One launch before a directly launched call's force kernel: applies the staged
-// updates, predicts [0, pred_j1), copies the call block (descriptor, i ids, i
-// doubles) to the device and clears the neighbour counters.  Work-groups take
-// one role each: [0, nb_upd) updates, then nb_copy for the call block, the rest
-// predict.  Updates and call block are read from pinned host memory.
+// updates, predicts [0, pred_j1), copies the call's inputs (descriptor, i ids, i
+// doubles, an ensemble's work table) to the device and clears the neighbour
+// counters.  Work-groups take one role each: [0, nb_upd) updates, then nb_copy
+// for the inputs, the rest predict.  Updates and inputs are read from pinned
+// host memory.
 constexpr int PREP_ROWS = 64;   // update rows per work-group
+constexpr int PREP_SEGS = 4;
+struct CopySeg { const int4* src; int4* dst; int n16; };   // host-mapped, device, 16-byte units
 struct PrepArgs {
   StoreView st;
   const double* rows_d;   // staged rows [0, nd), already on the device
@@ -121,9 +124,7 @@ struct PrepArgs {
   int new_ids;            // some update changes an address's id: widen its tile's id range
   double ti;
   int pred_j1;
-  const int4* call_h;     // call block, host-mapped, and its device copy, in 16-byte units
-  int4* call_d;
-  int call_n16;
+  CopySeg seg[PREP_SEGS];
   int* ngb_cnt;           // zeroed for [0, ni_reset), with *pack_ctr
   int ni_reset;
   int* pack_ctr;
