@@ -1422,13 +1422,15 @@ int Engine::grav_calc_scratch(void* scratch, size_t bytes, int nj, int ni, const
   p += al(sizeof(double) * r);
   int* paddr = reinterpret_cast<int*>(p);
   const CallDesc v{t_i_, eps2, ni, 0, 0, 0};
-  if (launch_write_desc(s, cd, v) != 0) return fail("descriptor launch", hipGetLastError());
+  // the descriptor goes with the prediction when there is one
+  if (!predict_ && launch_write_desc(s, cd, v) != 0) return fail("descriptor launch", hipGetLastError());
   if (predict_) {
     PredictArgs pa{};
     pa.st = st_;
     pa.j0 = 0;
     pa.j1 = nj;
-    pa.cd = cd;
+    pa.desc = v;
+    pa.desc_out = cd;
     if (launch_predict(s, order_, f64_, pa) != 0) return fail("predict launch", hipGetLastError());
     predict_ = false;
     jhost_valid_ = false;

@@ -102,7 +102,9 @@ struct ScatterArgs {
 struct PredictArgs {
   StoreView st;
   int j0, j1;            // predict addresses [j0, j1)
-  const CallDesc* cd;    // ti
+  const CallDesc* cd;    // ti; null: it is in desc, which is written to desc_out
+  CallDesc desc;
+  CallDesc* desc_out;
 };
 
 // One launch before a directly launched call's force kernel: applies the staged

@@ -161,11 +161,13 @@ __device__ __forceinline__ void tile_id_range(const StoreView& st, int j) {
 template <int ORDER, bool F64>
 __global__ __launch_bounds__(256) void k_predict(PredictArgs a) {
   const int j = a.j0 + blockIdx.x * blockDim.x + threadIdx.x;
+  if (!a.cd && blockIdx.x == 0 && threadIdx.x == 0) *a.desc_out = a.desc;
+  const double ti = a.cd ? a.cd->ti : a.desc.ti;
   tile_id_range(a.st, j);
   if (j >= a.j1) return;
   const size_t cap = (size_t)a.st.cap;
   double p[3], v[3], ac[3];
-  predict_one<ORDER>([&](int f) { return a.st.raw[f * cap + j]; }, a.cd->ti, p, v, ac);
+  predict_one<ORDER>([&](int f) { return a.st.raw[f * cap + j]; }, ti, p, v, ac);
   put_pred<ORDER, F64>(a.st, j, p, v, ac, a.st.raw[RF_M * cap + j], a.st.id[j]);
 }
 
