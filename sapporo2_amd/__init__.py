@@ -393,7 +393,7 @@ class Engine:
         return P.value, S.value, jc.value
 
     def load_tuning(self, path):
-        """Load a launch-shape table (None or a missing file: heuristic shapes)."""
+        """Load a launch-shape table (None or a missing file: the built-in rule)."""
         return self._L.sapamd_load_tuning(self._h, None if path is None else str(path).encode())
 
     @property

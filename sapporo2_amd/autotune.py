@@ -4,14 +4,15 @@ For each system size N (a Plummer sphere), integration order, working precision,
 neighbour-list mode and active-count bucket ni = 2^k (k = 0 .. 14), it times candidate
 lane shapes P (i-particles per wave) and j-splits S, and keeps the shape with the
 smallest device time of the whole call (scatter/reset, force, finalize: the engine's
-device window).  The result is a text table the engine reads at open(); a call uses the
-entry of its bucket at the nearest log2(nj):
+device window).  The result is a text table that replaces the engine's built-in launch-shape rule
+when it is loaded ($SAPPORO2_AMD_TUNE at open, or load_tuning); a call then uses the entry of
+its bucket at the nearest log2(nj):
 
     # order precision ngb log2(ni) log2(nj) P log2(j per split)
     1 1 1 14 17 64 10
 
 usage (on the GPU): python -m sapporo2_amd.autotune [--n 8192,131072,262144,1048576] [--out PATH]
-The default output is tune/<arch>.txt beside the library, the file the engine loads.
+The default output is tune/gfx950.txt beside the library.
 """
 from __future__ import annotations
 

@@ -58,6 +58,7 @@ constexpr int BATCH_ROWS = 16384;  // rows a batch stages at a time
 // Rows from which staging uses the host threads: waking them costs ~50 us after
 // a long call, a row ~10 ns on the caller (2500 rows: 70 us with them, 20 without).
 constexpr size_t PAR_ROWS = 6144;
+constexpr int BITS_ROWS = 4096;  // updates marked for the predictor at ~1 ns each
 // Upload block of a single-system call, one host->device copy: the call
 // descriptor, then the i ids, then the i doubles.  The ids region is sized by
 // the power-of-two bucket of ni, so every offset depends on the bucket only
@@ -368,7 +369,7 @@ int Engine::set_no_time() {
 
 namespace {
 // Row of one update: the raw fields in RawField order, then (address, id).
-inline void fill_row(double* u, int order, int addr, int id, double tj, double dtj, double mass, const double* a,
+__attribute__((always_inline)) inline void fill_row(double* u, int order, int addr, int id, double tj, double dtj, double mass, const double* a,
                      const double* jrk, const double* v, const double* x, const double* snp, const double* crk,
                      double eps) {
   u[RF_T] = tj; u[RF_DT] = dtj; u[RF_M] = mass; u[RF_EPS] = eps;
@@ -394,13 +395,17 @@ int Engine::open_stage() {
   if (nstaged_ != 0) return 0;
   Stage& sg = stage_[cur_];
   if (sg.busy && wait_stage(sg) != 0) return -1;
-  auto clear = [&](size_t b, size_t e) {
-    for (size_t k = b; k < e; ++k) __atomic_store_n(&sg.bits[sg.addr[k] >> 5], 0u, __ATOMIC_RELAXED);
-  };
-  if (sg.addr.size() >= PAR_ROWS) par_for(sg.addr.size(), clear);
-  else clear(0, sg.addr.size());
+  if (sg.bits_set)
+    for (const int a : sg.addr) sg.bits[a >> 5] = 0;
+  sg.bits_set = false;
   sg.addr.clear();
   return 0;
+}
+
+// The stage's addresses as a bit set.
+void Engine::set_bits(Stage& sg) {
+  for (const int a : sg.addr) sg.bits[a >> 5] |= 1u << (a & 31);
+  sg.bits_set = true;
 }
 
 // Capacity for an address beyond the host maps.
@@ -420,7 +425,7 @@ int Engine::admit(int addr) {
 
 // Row of the current stage for an update of addr (-1 on error); the caller
 // fills it.
-inline int Engine::stage_row(int addr, int id) {
+__attribute__((always_inline)) inline int Engine::stage_row(int addr, int id) {
   if ((unsigned)addr >= addr_.size() && admit(addr) != 0) return -1;
   if (nstaged_ == 0 && open_stage() != 0) return -1;
   Stage* sg = &stage_[cur_];
@@ -436,7 +441,6 @@ inline int Engine::stage_row(int addr, int id) {
     k = nstaged_++;
     as.slot = k;
     sg->addr.push_back(addr);
-    sg->bits[addr >> 5] |= 1u << (addr & 31);
   } else if (k < flushed_) {
     flushed_ = k;  // already copied: copy again from this row
   }
@@ -555,7 +559,6 @@ int Engine::stage_block(int n, const int* addr, const int* id, const F& fill) {
       ch |= was == SLOT_NEW || __atomic_load_n(&as[ad].id, __ATOMIC_RELAXED) != id[k];
       if (was < 0) __atomic_store_n(&as[ad].slot, base + (int)k, __ATOMIC_RELAXED);
       __atomic_store_n(&as[ad].id, id[k], __ATOMIC_RELAXED);
-      __atomic_fetch_or(&sg.bits[ad >> 5], 1u << (ad & 31), __ATOMIC_RELAXED);
       sg.addr[(size_t)base + k] = ad;
       mx = std::max(mx, ad);
     }
@@ -629,7 +632,12 @@ int Engine::prep(int pred_j1, int call_bytes, int ni_reset, bool by_call, const 
   a.rows_h = sg.dd;
   a.nd = flushed_;
   a.nupd = n;
-  if (n > 0 && pred_j1 > 0) {
+  // Updates and prediction in one launch, unless ids change (the tile id ranges
+  // are rebuilt from the updated store) or marking the addresses would cost the
+  // host more than the launch.
+  const bool apart = n > 0 && pred_j1 > 0 && (new_ids_ || n > BITS_ROWS);
+  if (n > 0 && pred_j1 > 0 && !apart) {
+    set_bits(sg);
     a.bits = sg.bits_d;
     a.nbits = (int)std::min<size_t>(sg.words * 32, INT_MAX);
   }
@@ -643,16 +651,15 @@ int Engine::prep(int pred_j1, int call_bytes, int ni_reset, bool by_call, const 
   a.pack_ctr = pack_ctr_d_;
   const bool ev = timing_;
   timed_scatter_ = timed_predict_ = false;
-  if (n > 0 && pred_j1 > 0 && new_ids_) {
-    // ids change: the tile id ranges are rebuilt from the updated store
+  if (apart) {
     PrepArgs u = a;
-    u.pred_j1 = u.nbits = 0;
+    u.pred_j1 = 0;
     if (ev) HIPCHK(hipEventRecord(ev_s0_, stream_), "event");
     if (launch_prep(stream_, order_, f64_, u) != 0) return fail("update launch", hipGetLastError());
     if (ev) HIPCHK(hipEventRecord(ev_s1_, stream_), "event");
     timed_scatter_ = ev;
     last_nupd_ = n;
-    a.nupd = a.ni_reset = a.nbits = 0;
+    a.nupd = a.ni_reset = 0;
     for (CopySeg& g : a.seg) g.n16 = 0;
   }
   if (ev) HIPCHK(hipEventRecord(ev_p0_, stream_), "event");
@@ -1268,7 +1275,8 @@ int Engine::start_grav_calc(int nj, int ni, const int* id, const double (*xi)[3]
     if (launch_call_graph(grid_ni, nj, cfg, ngb_on, predict, sblocks, finalize_threads(bucket)) != 0) return -1;
     timed_predict_ = timed_force_ = false;
   } else {
-    if (cfg.small && predict && !new_ids_ && nstaged_ <= SMALL_UPD && flushed_ == 0 && max_addr_ < nj) {
+    if (cfg.small && predict && !new_ids_ && nstaged_ <= SMALL_UPD && flushed_ == 0 &&
+        (nstaged_ == 0 || max_addr_ < nj)) {
       if (call_small(nj, cfg, ngb_on, bucket) != 0) return -1;
     } else {
       if (prep(predict ? nj : 0, (int)nbytes, ngb_on ? ni : 0, true) != 0) return -1;
@@ -1298,7 +1306,7 @@ int Engine::start_grav_calc(int nj, int ni, const int* id, const double (*xi)[3]
 int Engine::call_small(int nj, const ForceConfig& cfg, bool ngb_on, int bucket) {
   const int ni = desc_h_->ni;
   int* cnt = cnt_small_d_ + (small_flip_ ? SMALL_NI : 0);
-  const Stage& sg = stage_[cur_];
+  Stage& sg = stage_[cur_];
   const ptrdiff_t alias = reinterpret_cast<char*>(call_hd_) - reinterpret_cast<char*>(call_d_);
   SmallArgs a{};
   a.f = force_args(ni, nj, ngb_on);
@@ -1312,7 +1320,10 @@ int Engine::call_small(int nj, const ForceConfig& cfg, bool ngb_on, int bucket) 
   a.st = st_;
   a.rows_h = sg.dd;
   a.bits = sg.bits_d;
-  a.nbits = nstaged_ > 0 ? (int)std::min<size_t>(sg.words * 32, INT_MAX) : 0;
+  if (nstaged_ > SMALL_ARG) {
+    set_bits(sg);
+    a.nbits = (int)std::min<size_t>(sg.words * 32, INT_MAX);
+  }
   a.nupd = nstaged_;
   a.ti = t_i_;
   for (int k = 0; k < std::min(nstaged_, SMALL_ARG); ++k) a.addr[k] = sg.addr[k];

@@ -136,6 +136,7 @@ class Engine {
   int grow_maps();
   int admit(int addr);
   int open_stage();
+  void set_bits(Stage& sg);
   template <typename F>
   int stage_block(int n, const int* addr, const int* id, const F& fill);
   int stage_row(int addr, int id);
@@ -182,9 +183,10 @@ class Engine {
     double* d = nullptr;      // cap rows of nf doubles + one (address, id) int pair
     double* dd = nullptr;     // its device alias
     int cap = 0;
-    // addresses of its rows, in row order, and as a bit set (host-mapped: host
-    // pointer, device alias, words); both are cleared when the stage is reused
+    // addresses of its rows, in row order, and, once bits_set, as a bit set (host-
+    // mapped: host pointer, device alias, words); cleared when the stage is reused
     std::vector<int> addr;
+    bool bits_set = false;
     unsigned* bits = nullptr; unsigned* bits_d = nullptr; size_t words = 0;
     hipEvent_t ev = nullptr;  // completion of the copy that last read it
     bool busy = false;

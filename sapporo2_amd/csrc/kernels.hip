@@ -179,8 +179,8 @@ __global__ __launch_bounds__(256) void k_predict(PredictArgs a) {
 // bit is set: the work-group that holds such an update writes its stored fields
 // and its predicted record from the staged row, so the roles never write the
 // same address and need no order among them.  The tile id ranges are the
-// predictor's alone: a call whose updates change an id runs the updates in a
-// launch of their own before it (new_ids).
+// predictor's alone: a call whose updates change an id, or are many, runs the
+// updates in a launch of their own before it.
 template <int ORDER, bool F64>
 __global__ __launch_bounds__(256) void k_prep(PrepArgs a) {
   constexpr int NF = raw_fields(ORDER), NR = NF + 1;
@@ -219,31 +219,38 @@ __global__ __launch_bounds__(256) void k_prep(PrepArgs a) {
   b -= a.nb_upd;
   if (b < a.nb_copy) {
     const int stride = a.nb_copy * 256;
-#pragma unroll
-    for (int g = 0; g < PREP_SEGS; ++g) {
-      const CopySeg& sg = a.seg[g];
+    auto copy = [&](const int4* __restrict__ src, int4* __restrict__ dst, int n16) {
       int k = b * 256 + t;
-      for (; k + 3 * stride < sg.n16; k += 4 * stride) {  // four reads over PCIe in flight
-        int4 v[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) v[u] = sg.src[k + u * stride];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) sg.dst[k + u * stride] = v[u];
+      for (; k + 3 * stride < n16; k += 4 * stride) {  // four reads over PCIe in flight
+        const int4 v0 = src[k], v1 = src[k + stride], v2 = src[k + 2 * stride], v3 = src[k + 3 * stride];
+        dst[k] = v0; dst[k + stride] = v1; dst[k + 2 * stride] = v2; dst[k + 3 * stride] = v3;
       }
-      for (; k < sg.n16; k += stride) sg.dst[k] = sg.src[k];
-    }
+      for (; k < n16; k += stride) dst[k] = src[k];
+    };
+    static_assert(PREP_SEGS == 4, "segments");
+    copy(a.seg[0].src, a.seg[0].dst, a.seg[0].n16);
+    copy(a.seg[1].src, a.seg[1].dst, a.seg[1].n16);
+    copy(a.seg[2].src, a.seg[2].dst, a.seg[2].n16);
+    copy(a.seg[3].src, a.seg[3].dst, a.seg[3].n16);
     for (int k = b * 256 + t; k < a.ni_reset; k += stride) a.ngb_cnt[k] = 0;
     if (b == 0 && t == 0 && a.ni_reset > 0) *a.pack_ctr = 0;
     return;
   }
   b -= a.nb_copy;
   const int j = b * 256 + t;
+  // the stored fields are loaded while the bits come over PCIe
+  double raw[NF];
+  if (j < a.pred_j1) {
+#pragma unroll
+    for (int f = 0; f < NF; ++f)
+      if (f != RF_DT && f != RF_EPS) raw[f] = a.st.raw[(size_t)f * cap + j];
+  }
   const bool skip = j < a.nbits && (a.bits[j >> 5] >> (j & 31) & 1u);
   tile_id_range(a.st, j);
   if (j >= a.pred_j1 || skip) return;
   double p[3], v[3], ac[3];
-  predict_one<ORDER>([&](int f) { return a.st.raw[f * cap + j]; }, a.ti, p, v, ac);
-  put_pred<ORDER, F64>(a.st, j, p, v, ac, a.st.raw[RF_M * cap + j], a.st.id[j]);
+  predict_one<ORDER>([&](int f) { return raw[f]; }, a.ti, p, v, ac);
+  put_pred<ORDER, F64>(a.st, j, p, v, ac, raw[RF_M], a.st.id[j]);
 }
 
 // ---------------------------------------------------------------------------
