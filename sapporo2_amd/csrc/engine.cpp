@@ -57,7 +57,7 @@ constexpr int EARLY_FLUSH_ROWS = 4096;
 constexpr int BATCH_ROWS = 16384;  // rows a batch stages at a time
 // Rows from which staging uses the host threads: waking them costs ~50 us after
 // a long call, a row ~10 ns on the caller (2500 rows: 70 us with them, 20 without).
-constexpr size_t PAR_ROWS = 6144;
+constexpr size_t PAR_ROWS = 6144, PAR_RELEASE = 65536;
 constexpr int BITS_ROWS = 4096;  // updates marked for the predictor at ~1 ns each
 // Upload block of a single-system call, one host->device copy: the call
 // descriptor, then the i ids, then the i doubles.  The ids region is sized by
@@ -213,7 +213,7 @@ int Engine::close() {
   for (auto& s : stage_) {
     hfree(s.d); s.dd = nullptr; s.cap = 0; s.busy = s.by_call = false;
     hfree(s.bits); s.bits_d = nullptr; s.words = 0;
-    s.addr.clear();
+    s.addr.clear(); s.handed = 0; s.bits_set = false;
     if (s.ev) (void)hipEventDestroy(s.ev);
     s.ev = nullptr;
   }
@@ -321,6 +321,7 @@ int Engine::grow_staging(int need) {
     s.d = d;
     s.dd = dd;
     s.cap = nc;
+    s.addr.resize((size_t)nc);
   }
   return ensure_bits(nj_max_);
 }
@@ -396,15 +397,14 @@ int Engine::open_stage() {
   Stage& sg = stage_[cur_];
   if (sg.busy && wait_stage(sg) != 0) return -1;
   if (sg.bits_set)
-    for (const int a : sg.addr) sg.bits[a >> 5] = 0;
+    for (int k = 0; k < sg.handed; ++k) sg.bits[sg.addr[k] >> 5] = 0;
   sg.bits_set = false;
-  sg.addr.clear();
   return 0;
 }
 
-// The stage's addresses as a bit set.
+// The current stage's addresses as a bit set.
 void Engine::set_bits(Stage& sg) {
-  for (const int a : sg.addr) sg.bits[a >> 5] |= 1u << (a & 31);
+  for (int k = 0; k < nstaged_; ++k) sg.bits[sg.addr[k] >> 5] |= 1u << (sg.addr[k] & 31);
   sg.bits_set = true;
 }
 
@@ -431,8 +431,10 @@ __attribute__((always_inline)) inline int Engine::stage_row(int addr, int id) {
   Stage* sg = &stage_[cur_];
   AddrState& as = addr_[addr];
   int k = as.slot;
-  new_ids_ |= k == SLOT_NEW || as.id != id;
-  as.id = id;
+  if (__builtin_expect(k == SLOT_NEW || as.id != id, 0)) {
+    new_ids_ = true;
+    as.id = id;
+  }
   if (k < 0) {
     if (nstaged_ >= sg->cap) {
       if (grow_staging(nstaged_ + 1) != 0) return -1;
@@ -440,7 +442,7 @@ __attribute__((always_inline)) inline int Engine::stage_row(int addr, int id) {
     }
     k = nstaged_++;
     as.slot = k;
-    sg->addr.push_back(addr);
+    sg->addr[k] = addr;
   } else if (k < flushed_) {
     flushed_ = k;  // already copied: copy again from this row
   }
@@ -546,7 +548,6 @@ int Engine::stage_block(int n, const int* addr, const int* id, const F& fill) {
   if (nstaged_ + n > stage_[cur_].cap && grow_staging(nstaged_ + n) != 0) return -1;
   Stage& sg = stage_[cur_];
   const int base = nstaged_;
-  sg.addr.resize((size_t)base + n);
   AddrState* as = addr_.data();
   std::atomic<bool> again{false}, changed{false};
   std::atomic<int> top{max_addr_};
@@ -578,7 +579,6 @@ int Engine::stage_block(int n, const int* addr, const int* id, const F& fill) {
   if (again.load()) {
     for (int k = 0; k < n; ++k)
       if (as[addr[k]].slot >= base) as[addr[k]].slot = SLOT_NONE;
-    sg.addr.resize((size_t)base);
     new_ids_ = true;  // the ids before this block are overwritten
     return 0;
   }
@@ -607,12 +607,13 @@ int Engine::upload_updates(int* nupd) {
 // The staged rows are the device's from here on; staging goes on in the other
 // stage.
 void Engine::hand_over() {
-  const std::vector<int>& staged = stage_[cur_].addr;
+  Stage& sg = stage_[cur_];
   auto release = [&](size_t b, size_t e) {
-    for (size_t k = b; k < e; ++k) addr_[staged[k]].slot = SLOT_NONE;
+    for (size_t k = b; k < e; ++k) addr_[sg.addr[k]].slot = SLOT_NONE;
   };
-  if (staged.size() >= PAR_ROWS) par_for(staged.size(), release);
-  else release(0, staged.size());
+  if ((size_t)nstaged_ >= PAR_RELEASE) par_for((size_t)nstaged_, release);
+  else release(0, (size_t)nstaged_);
+  sg.handed = nstaged_;
   nstaged_ = 0;
   flushed_ = 0;
   new_ids_ = false;

@@ -185,7 +185,8 @@ class Engine {
     int cap = 0;
     // addresses of its rows, in row order, and, once bits_set, as a bit set (host-
     // mapped: host pointer, device alias, words); cleared when the stage is reused
-    std::vector<int> addr;
+    std::vector<int> addr;    // as many as rows
+    int handed = 0;           // rows of the last flush from this stage
     bool bits_set = false;
     unsigned* bits = nullptr; unsigned* bits_d = nullptr; size_t words = 0;
     hipEvent_t ev = nullptr;  // completion of the copy that last read it
