@@ -119,7 +119,13 @@ Engine::~Engine() {
   if (open_) close();
 }
 
+// A failure between a call's first device work and its completion record leaves
+// nothing that would tell when that work has read its pinned memory: wait for it.
 int Engine::fail(const char* what, hipError_t e) {
+  if (queued_ && !capturing_) {
+    (void)hipStreamSynchronize(stream_);
+    queued_ = false;
+  }
   err_ = what;
   if (e != hipSuccess) {
     err_ += ": ";
@@ -240,7 +246,7 @@ int Engine::close() {
   }
   if (stream_) (void)hipStreamDestroy(stream_);
   stream_ = nullptr;
-  open_ = inflight_ = have_results_ = ngb_fetched_ = jhost_valid_ = false;
+  open_ = inflight_ = queued_ = have_results_ = ngb_fetched_ = jhost_valid_ = false;
   addr_.clear();
   nstaged_ = 0;
   return 0;
@@ -490,9 +496,11 @@ int Engine::copy_staged() {
   }
   Stage& sg = stage_[cur_];
   const size_t o = (size_t)flushed_ * nr;
+  queued_ = true;
   HIPCHK(hipMemcpyAsync(upd_d_ + o, sg.d + o, sizeof(double) * ((size_t)n * nr - o), hipMemcpyHostToDevice,
                         stream_), "update upload");
   HIPCHK(hipEventRecord(sg.ev, stream_), "event");
+  queued_ = false;
   sg.busy = true;
   sg.by_call = false;
   sg.seq = ++rec_seq_;
@@ -652,6 +660,7 @@ int Engine::prep(int pred_j1, int call_bytes, int ni_reset, bool by_call, const 
   a.pack_ctr = pack_ctr_d_;
   const bool ev = timing_;
   timed_scatter_ = timed_predict_ = false;
+  queued_ = true;
   if (apart) {
     PrepArgs u = a;
     u.pred_j1 = 0;
@@ -676,6 +685,7 @@ int Engine::prep(int pred_j1, int call_bytes, int ni_reset, bool by_call, const 
     sg.seq = ++rec_seq_;
     hand_over();
   }
+  if (!by_call) queued_ = false;
   return 0;
 }
 
@@ -1062,6 +1072,7 @@ int Engine::start_grav_calc_clusters(int ni, const int* cluster, const int* id, 
   const bool dma = ni >= ENS_DMA_I;
   bool ngb_on = false;
   if (!dma) ngb_on = pack_i(0, ni, id, xi, vi, ai, h2, bx, bv, ba, bh, iid_h_);
+  queued_ = dma;
   for (int k = 0; dma && k < 4; ++k) {
     const int b = (int)((long)ni * k / 4), e = (int)((long)ni * (k + 1) / 4);
     ngb_on |= pack_i(b, e, id, xi, vi, ai, h2, bx, bv, ba, bh, iid_h_);
@@ -1151,6 +1162,7 @@ int Engine::start_grav_calc_clusters(int ni, const int* cluster, const int* id, 
   };
   order_part(0, n64);
   order_part(n64, nitems);
+  if (ensure_partials((size_t)nitems * 64) != 0) return -1;
   if (desc_pending_ && desc_seq_ > done_seq_) HIPCHK(hipEventSynchronize(ev_desc_), "descriptor wait");
   desc_pending_ = false;
   *desc_h_ = CallDesc{t_i_, 0.0, ni, 0, 0, 0};
@@ -1163,7 +1175,6 @@ int Engine::start_grav_calc_clusters(int ni, const int* cluster, const int* id, 
   predict_ = false;
   if (launch_ens_idesc(stream_, reinterpret_cast<const EnsGroup*>(ens_tab_d_ + o_grp), ng, ni, idesc_d_) != 0)
     return fail("ensemble descriptor launch", hipGetLastError());
-  if (ensure_partials((size_t)nitems * 64) != 0) return -1;
   EnsArgs ea{};
   ea.rec = st_.rec;
   ea.idr = st_.idr;
@@ -1196,6 +1207,7 @@ int Engine::start_grav_calc_clusters(int ni, const int* cluster, const int* id, 
   timed_force_ = timing_;
   HIPCHK(hipEventRecord(ev_done_, stream_), "event");
   done_rec_seq_ = ++rec_seq_;
+  queued_ = false;
   inflight_ = true;
   have_results_ = true;
   ngb_fetched_ = false;
@@ -1256,8 +1268,10 @@ int Engine::start_grav_calc(int nj, int ni, const int* id, const double (*xi)[3]
   desc_h_->seq = next_seq();
   const size_t nbytes = (size_t)((char*)(bx + nd) - (char*)call_h_);
   if (graphs_) {
+    queued_ = true;
     HIPCHK(hipMemcpyAsync(call_d_, call_h_, nbytes, hipMemcpyHostToDevice, stream_), "call upload");
     HIPCHK(hipEventRecord(ev_desc_, stream_), "event");
+    queued_ = false;
     desc_pending_ = true;
     desc_seq_ = ++rec_seq_;
   }
@@ -1288,6 +1302,7 @@ int Engine::start_grav_calc(int nj, int ni, const int* id, const double (*xi)[3]
   if (timing_) HIPCHK(hipEventRecord(ev_d1_, stream_), "event");
   if (!done_word_) HIPCHK(hipEventRecord(ev_done_, stream_), "event");
   done_rec_seq_ = ++rec_seq_;
+  queued_ = false;
   inflight_ = true;
   have_results_ = true;
   ngb_fetched_ = false;
@@ -1329,10 +1344,11 @@ int Engine::call_small(int nj, const ForceConfig& cfg, bool ngb_on, int bucket) 
   a.ti = t_i_;
   for (int k = 0; k < std::min(nstaged_, SMALL_ARG); ++k) a.addr[k] = sg.addr[k];
   a.cnt_clear = cnt_small_d_ + (small_flip_ ? 0 : SMALL_NI);
-  small_flip_ = !small_flip_;
   timed_scatter_ = timed_predict_ = false;
+  queued_ = true;
   if (timing_) HIPCHK(hipEventRecord(ev_f0_, stream_), "event");
   if (launch_force_small(stream_, order_, f64_, a, cfg, true) != 0) return fail("force launch", hipGetLastError());
+  small_flip_ = !small_flip_;
   if (timing_) HIPCHK(hipEventRecord(ev_f1_, stream_), "event");
   FinalizeArgs fz = finalize_args(ni, ngb_on);
   fz.cd = nullptr;

@@ -234,6 +234,7 @@ class Engine {
   hipEvent_t ev_s0_ = nullptr, ev_s1_ = nullptr;
   bool timed_scatter_ = false;
   int last_nupd_ = 0;
+  bool queued_ = false;       // device work is queued whose completion has no record yet
   bool inflight_ = false, have_results_ = false, ngb_fetched_ = false, ngb_on_last_ = false;
   bool timed_predict_ = false, timed_force_ = false;
   bool capturing_ = false;

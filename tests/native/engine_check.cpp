@@ -1,0 +1,158 @@
+// Checks of the host engine against a HIP runtime of the test's own (fake_hip.h):
+// one check per argument.
+#include "fake_hip.h"
+
+#include <chrono>
+#include <set>
+
+#include "engine.h"
+
+using namespace sap;
+using namespace sapk;
+
+namespace {
+
+int bad = 0;
+#define EXPECT(c, ...)                                            \
+  do {                                                            \
+    if (!(c)) {                                                   \
+      ++bad;                                                      \
+      std::printf("%s:%d: " #c " does not hold: ", __FILE__, __LINE__); \
+      std::printf(__VA_ARGS__);                                   \
+      std::printf("\n");                                          \
+    }                                                             \
+  } while (0)
+
+// A program: n particles, each send recorded so that the store can be compared.
+struct Program {
+  Engine e;
+  int order;
+  std::vector<double> x;  // last x sent, by address
+  std::vector<int> id;
+  Program(int n, int order_ = ORDER_H4, int prec = PREC_DS) : order(order_), x(n, 0.0), id(n, 0) {
+    if (e.open(0, order, prec) != 0) std::abort();
+    std::vector<int> a(n);
+    std::vector<double> m(n, 1.0), p(3 * (size_t)n);
+    for (int k = 0; k < n; ++k) { a[k] = k; id[k] = 10 + k; x[k] = p[3 * (size_t)k] = k; }
+    if (e.set_j_particles(n, a.data(), id.data(), nullptr, nullptr, m.data(), nullptr, nullptr, nullptr, p.data(),
+                          nullptr, nullptr, nullptr) != 0)
+      std::abort();
+    e.set_time(0.0);
+    if (e.force_prediction(n) != 0) std::abort();
+  }
+  void send(int a, double v, int new_id = -1) {
+    if (new_id >= 0) id[a] = new_id;
+    x[a] = v;
+    const double p[3] = {v, 0, 0}, z[3] = {0, 0, 0};
+    EXPECT(e.set_j_particle(a, id[a], 0, 0, 1, z, z, z, p, z, z, 0) == 0, "send %d", a);
+  }
+  void batch(const std::vector<int>& a, double v) {
+    const int n = (int)a.size();
+    std::vector<int> ids(n);
+    std::vector<double> m(n, 1.0), p(3 * (size_t)n, 0.0);
+    for (int k = 0; k < n; ++k) { ids[k] = id[a[k]]; p[3 * (size_t)k] = x[a[k]] = v + k; }
+    EXPECT(e.set_j_particles(n, a.data(), ids.data(), nullptr, nullptr, m.data(), nullptr, nullptr, nullptr, p.data(),
+                             nullptr, nullptr, nullptr) == 0, "batch of %d", n);
+  }
+  int call(int nj, int ni, bool lists = false, bool predict = true) {
+    std::vector<int> ids(ni, -5);
+    std::vector<double> p(3 * (size_t)ni, 0.5), h(ni, 1.0);
+    predict ? e.set_time(1.0) : e.set_no_time();
+    const auto* v = reinterpret_cast<const double(*)[3]>(p.data());
+    return e.start_grav_calc(nj, ni, ids.data(), v, v, v, 1e-4, lists ? h.data() : nullptr);
+  }
+  int results(int nj, int ni) {
+    std::vector<double> a(3 * (size_t)ni);
+    return e.get_grav_results(nj, ni, reinterpret_cast<double(*)[3]>(a.data()), nullptr, nullptr, nullptr, nullptr,
+                              nullptr, nullptr, false);
+  }
+  // the store holds what was sent
+  void check(const char* label) {
+    EXPECT(e.force_prediction(0) == 0, "%s", label);
+    EXPECT(e.synchronize() == 0, "%s", label);
+    const StoreView& st = fake::last_store;
+    int wrong = 0;
+    for (size_t a = 0; a < x.size(); ++a)
+      wrong += st.raw[(size_t)RF_X * st.cap + a] != x[a] || st.id[a] != id[a];
+    EXPECT(wrong == 0, "%s: %d addresses of the store differ from what was sent", label, wrong);
+    EXPECT(fake::violations == 0, "%s", label);
+    fake::violations = 0;
+  }
+};
+
+int ens_call(Program& p, const std::vector<int>& nj, int per) {
+  std::vector<int> c, ids;
+  for (size_t k = 0; k < nj.size(); ++k)
+    for (int i = 0; i < per; ++i) { c.push_back((int)k); ids.push_back(-5); }
+  const int ni = (int)c.size();
+  std::vector<double> x(3 * (size_t)ni, 0.5), eps(nj.size(), 1e-4);
+  const auto* v = reinterpret_cast<const double(*)[3]>(x.data());
+  p.e.set_time(1.0);
+  return p.e.start_grav_calc_clusters(ni, c.data(), ids.data(), v, v, v, eps.data(), nullptr);
+}
+
+}  // namespace
+
+struct Fault {
+  const char* what;  // fake::fails name, and which of the call's requests of that name fails
+  int nth, ni, lists;
+  bool ens;
+};
+
+// Calls that fail, each followed by sends into both stages and by calls that succeed.
+void fail_and_go_on(const Fault* at, int cases) {
+  for (int q = 0; q < cases; ++q) {
+    const Fault& f = at[q];
+    Program p(std::max(3000, f.ni));
+    const int np = (int)p.x.size();
+    const std::vector<int> cl(4, 700);
+    if (f.ens) EXPECT(p.e.set_clusters(4, cl.data()) == 0, "clusters");
+    char label[96];
+    std::snprintf(label, sizeof label, "%s %d of a call of %d%s", f.what, f.nth, f.ni, f.ens ? " (ensemble)" : "");
+    bool reached = false;
+    for (int r = 0; r < 3; ++r) {
+      // "prep" 2: ids change, so that updates and prediction are two launches
+      const bool ids = f.nth == 2 && std::strcmp(f.what, "prep") == 0;
+      for (int k = 0; k < 40; ++k) p.send(3 * k + r, 1000.0 * r + k, ids ? 90000 + 100 * r + k : -1);
+      fake::fail_in[f.what] = f.nth;
+      const int rc = f.ens ? ens_call(p, cl, f.ni) : p.call(np, f.ni, f.lists != 0);
+      const bool hit = fake::fail_in[f.what] == 0;  // memory that is there is not asked for again
+      fake::fail_in.clear();
+      reached |= hit;
+      EXPECT((rc != 0) == hit, "%s: returns %d", label, rc);
+      for (int k = 0; k < 40; ++k) p.send(3 * k + 1, -1.0 - k - 50 * r);
+      EXPECT(p.e.force_prediction(0) == 0, "%s: flush", label);
+      for (int k = 0; k < 40; ++k) p.send(3 * k + 2, -2.0 - k - 50 * r);
+      EXPECT((f.ens ? ens_call(p, cl, 40) : p.call(np, 70, f.lists != 0)) == 0, "%s: the next call", label);
+      EXPECT(p.results(np, 3) == 0, "%s: the next results", label);
+      EXPECT(p.call(np, 5, true) == 0 && p.results(np, 5) == 0, "%s: a small call", label);
+    }
+    EXPECT(reached, "%s: not reached", label);
+    p.check(label);
+  }
+}
+
+// A call that fails after device work was queued: the memory which that work reads
+// is not written before it has run, and the next calls are as any other.
+void failed_calls() {
+  const Fault at[] = {{"idesc", 1, 3, 0, true},      {"ens", 1, 3, 0, true},       {"event", 1, 3, 0, true},
+                      {"force", 1, 100, 0, false},   {"finalize", 1, 100, 1, false}, {"event", 1, 5000, 0, false},
+                      {"small", 1, 5, 1, false},     {"finalize", 1, 5, 1, false}, {"prep", 1, 100, 1, false},
+                      {"prep", 2, 100, 0, false}};
+  fail_and_go_on(at, sizeof at / sizeof *at);
+}
+
+int main(int argc, char** argv) {
+  const std::string want = argc > 1 ? argv[1] : "";
+  const struct { const char* name; void (*f)(); } checks[] = {
+      {"failed_calls", failed_calls},
+  };
+  int ran = 0;
+  for (const auto& c : checks)
+    if (want.empty() || want == c.name) {
+      c.f();
+      ++ran;
+    }
+  std::printf("%s: %s\n", want.c_str(), bad || !ran || fake::violations ? "FAIL" : "ok");
+  return bad || !ran || fake::violations;
+}
