@@ -489,6 +489,7 @@ int Engine::copy_staged() {
     if (stream_) HIPCHK(hipStreamSynchronize(stream_), "staging grow sync");
     dfree(upd_d_);
     const int nc = std::max(n, upd_cap_d_ * 2);
+    upd_cap_d_ = 0;
     HIPCHK(dmalloc(&upd_d_, (size_t)nc * nr), "device staging");
     upd_cap_d_ = nc;
     flushed_ = 0;
@@ -732,6 +733,7 @@ int Engine::ensure_partials(size_t entries) {
   dfree(pds2_d_);
   dfree(paddr_d_);
   const size_t nc = std::max(entries, part_cap_ + part_cap_ / 2);
+  part_cap_ = 0;
   HIPCHK(dmalloc(&part_d_, nc * part_fields(order_)), "partials");
   HIPCHK(dmalloc(&pds2_d_, nc), "partials");
   HIPCHK(dmalloc(&paddr_d_, nc), "partials");
@@ -852,7 +854,8 @@ ForceConfig Engine::choose_config(int ni, int nj, bool ngb) const {
 int Engine::ensure_icap(int need) {
   if (need <= icap_) return 0;
   if (stream_) HIPCHK(hipStreamSynchronize(stream_), "i-buffer grow sync");
-  inflight_ = false;
+  inflight_ = have_results_ = false;
+  icap_ = 0;
   hfree(ibuf_h_); hfree(iid_h_); dfree(ibuf_d_); dfree(iid_d_);
   hfree(res_h_); hfree(loff_h_); dfree(cnt_d_); dfree(idesc_d_);
   const size_t nI = (size_t)need;
@@ -867,7 +870,6 @@ int Engine::ensure_icap(int need) {
   HIPCHK(dmalloc(&idesc_d_, nI), "ensemble i descriptors");
   HIPCHK(hipMemsetAsync(cnt_d_, 0, nI * sizeof(int), stream_), "memset");
   icap_ = need;
-  have_results_ = false;
   ++gen_;
   return 0;
 }
@@ -876,11 +878,11 @@ int Engine::ensure_icap(int need) {
 int Engine::ensure_lists(int need) {
   if (need <= list_cap_) return 0;
   if (stream_) HIPCHK(hipStreamSynchronize(stream_), "list grow sync");
-  inflight_ = false;
+  inflight_ = have_results_ = false;
+  list_cap_ = 0;
   dfree(list_d_);
   HIPCHK(dmalloc(&list_d_, (size_t)need * NGB_CAP), "neighbour lists");
   list_cap_ = need;
-  have_results_ = false;
   ++gen_;
   return 0;
 }
@@ -890,11 +892,11 @@ int Engine::ensure_lists(int need) {
 int Engine::ensure_packed(long need) {
   if (need <= packed_cap_) return 0;
   if (stream_) HIPCHK(hipStreamSynchronize(stream_), "packed-list grow sync");
-  inflight_ = false;
+  inflight_ = have_results_ = false;
+  packed_cap_ = 0;
   hfree(packed_h_);
   HIPCHK(hmap(&packed_h_, &packed_hd_, (size_t)need, coherent_), "host-mapped packed lists");
   packed_cap_ = need;
-  have_results_ = false;
   ++gen_;
   return 0;
 }
@@ -1128,9 +1130,11 @@ int Engine::start_grav_calc_clusters(int ni, const int* cluster, const int* id, 
   if (tab_bytes > ens_tab_cap_) {
     hfree(ens_tab_h_);
     dfree(ens_tab_d_);
-    ens_tab_cap_ = std::max(tab_bytes, 2 * ens_tab_cap_);
-    HIPCHK(hmap(&ens_tab_h_, &ens_tab_hd_, ens_tab_cap_, true), "ensemble work table (host)");
-    HIPCHK(dmalloc(&ens_tab_d_, ens_tab_cap_), "ensemble work table");
+    const size_t cap = std::max(tab_bytes, 2 * ens_tab_cap_);
+    ens_tab_cap_ = 0;
+    HIPCHK(hmap(&ens_tab_h_, &ens_tab_hd_, cap, true), "ensemble work table (host)");
+    HIPCHK(dmalloc(&ens_tab_d_, cap), "ensemble work table");
+    ens_tab_cap_ = cap;
   }
   EnsItem* items = reinterpret_cast<EnsItem*>(ens_tab_h_);
   int* order = reinterpret_cast<int*>(ens_tab_h_ + o_order);
@@ -1749,6 +1753,7 @@ int Engine::fetch_j_host(int need) {
   if (ensure_store(n) != 0) return -1;
   if (gather_cap_ < (size_t)n) {
     dfree(gather_d_);
+    gather_cap_ = 0;
     HIPCHK(dmalloc(&gather_d_, (size_t)n * 10), "gather buffer");
     gather_cap_ = n;
   }

@@ -163,7 +163,7 @@ hipError_t hipHostFree(void* p) { std::free(p); return hipSuccess; }
 hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind k, hipStream_t) {
   if (fake::fails("memcpy")) return hipErrorUnknown;
   // a host source may be written again behind the copy: rows are copied anew then
-  fake::submit([=] { std::memcpy(d, s, n); });
+  fake::submit([=] { if (n) std::memcpy(d, s, n); });
   (void)k;
   return hipSuccess;
 }

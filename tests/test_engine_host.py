@@ -29,7 +29,7 @@ def harness(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("check", ["failed_calls"])
+@pytest.mark.parametrize("check", ["failed_calls", "failed_growth"])
 def test_engine(harness, check):
     r = subprocess.run([harness, check], capture_output=True, text=True, timeout=300)
     assert r.returncode == 0 and "ok" in r.stdout, (r.stdout + r.stderr)[-4000:]
