@@ -57,6 +57,9 @@ constexpr int EARLY_FLUSH_ROWS = 4096;
 constexpr int BATCH_ROWS = 16384;  // rows a batch stages at a time
 // Rows from which staging uses the host threads: waking them costs ~50 us after
 // a long call, a row ~10 ns on the caller (2500 rows: 70 us with them, 20 without).
+// From PAR_RELEASE rows staged there, their addresses are also released there; those
+// of rows that the caller staged are released by the caller, whose next sends read
+// them (with the map in other cores' caches 262143 sends took 4.3-5.1 ms for 2.9-3.6).
 constexpr size_t PAR_ROWS = 6144, PAR_RELEASE = 65536;
 constexpr int BITS_ROWS = 4096;  // updates marked for the predictor at ~1 ns each
 // Upload block of a single-system call, one host->device copy: the call
@@ -249,6 +252,7 @@ int Engine::close() {
   open_ = inflight_ = queued_ = have_results_ = ngb_fetched_ = jhost_valid_ = false;
   addr_.clear();
   nstaged_ = 0;
+  par_staged_ = 0;
   return 0;
 }
 
@@ -592,6 +596,7 @@ int Engine::stage_block(int n, const int* addr, const int* id, const F& fill) {
     return 0;
   }
   nstaged_ = base + n;
+  par_staged_ += (size_t)n;
   new_ids_ |= changed.load();
   max_addr_ = top.load();
   jhost_valid_ = false;
@@ -620,10 +625,11 @@ void Engine::hand_over() {
   auto release = [&](size_t b, size_t e) {
     for (size_t k = b; k < e; ++k) addr_[sg.addr[k]].slot = SLOT_NONE;
   };
-  if ((size_t)nstaged_ >= PAR_RELEASE) par_for((size_t)nstaged_, release);
+  if (par_staged_ >= PAR_RELEASE) par_for((size_t)nstaged_, release);
   else release(0, (size_t)nstaged_);
   sg.handed = nstaged_;
   nstaged_ = 0;
+  par_staged_ = 0;
   flushed_ = 0;
   new_ids_ = false;
   cur_ ^= 1;

@@ -196,6 +196,7 @@ class Engine {
   };
   Stage stage_[2];
   int cur_ = 0, nstaged_ = 0;
+  size_t par_staged_ = 0;     // staged rows that the host threads staged
   int flushed_ = 0;           // staged rows [0, flushed_) already copied to the device (early flush)
   // per address: its staged row (SLOT_NONE: not staged, SLOT_NEW: nor was its id
   // ever staged, or a load replaced it) and the id last staged for it

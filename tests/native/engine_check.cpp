@@ -31,6 +31,7 @@ struct Program {
   std::vector<int> id;
   Program(int n, int order_ = ORDER_H4, int prec = PREC_DS) : order(order_), x(n, 0.0), id(n, 0) {
     if (e.open(0, order, prec) != 0) std::abort();
+    if (n == 0) return;
     std::vector<int> a(n);
     std::vector<double> m(n, 1.0), p(3 * (size_t)n);
     for (int k = 0; k < n; ++k) { a[k] = k; id[k] = 10 + k; x[k] = p[3 * (size_t)k] = k; }
@@ -157,11 +158,33 @@ void failed_growth() {
   fail_and_go_on(at.data(), (int)at.size());
 }
 
+// A program that sends its particles one by one has its addresses released on its own
+// thread, however many: the host threads (started at their first use) are not.
+void send_release() {
+  const int n = 131072;
+  Program p(0);
+  p.x.assign(n, 0.0);
+  p.id.assign(n, 7);
+  for (int r = 0; r < 2; ++r) {
+    for (int a = 0; a < n; ++a) p.send(a, 1.0 + r + a);
+    EXPECT(p.call(n, 100) == 0 && p.results(n, 100) == 0, "call");
+  }
+  int threads = 0;
+  if (FILE* f = std::fopen("/proc/self/status", "r")) {
+    char line[256];
+    while (std::fgets(line, sizeof line, f)) std::sscanf(line, "Threads: %d", &threads);
+    std::fclose(f);
+  }
+  EXPECT(threads == 1, "%d threads", threads);
+  p.check("sends");
+}
+
 int main(int argc, char** argv) {
   const std::string want = argc > 1 ? argv[1] : "";
   const struct { const char* name; void (*f)(); } checks[] = {
       {"failed_calls", failed_calls},
       {"failed_growth", failed_growth},
+      {"send_release", send_release},
   };
   int ran = 0;
   for (const auto& c : checks)

@@ -29,8 +29,9 @@ def harness(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("check", ["failed_calls", "failed_growth"])
+@pytest.mark.parametrize("check", ["failed_calls", "failed_growth", "send_release"])
 def test_engine(harness, check):
-    r = subprocess.run([harness, check], capture_output=True, text=True, timeout=300)
+    env = dict(os.environ, SAPPORO2_AMD_HOST_THREADS="4")
+    r = subprocess.run([harness, check], capture_output=True, text=True, env=env, timeout=300)
     assert r.returncode == 0 and "ok" in r.stdout, (r.stdout + r.stderr)[-4000:]
     assert "runtime error" not in r.stderr, r.stderr[-4000:]
