@@ -441,15 +441,15 @@ __attribute__((always_inline)) inline int Engine::stage_row(int addr, int id) {
   Stage* sg = &stage_[cur_];
   AddrState& as = addr_[addr];
   int k = as.slot;
+  if (k < 0 && nstaged_ >= sg->cap) {
+    if (grow_staging(nstaged_ + 1) != 0) return -1;
+    sg = &stage_[cur_];
+  }
   if (__builtin_expect(k == SLOT_NEW || as.id != id, 0)) {
     new_ids_ = true;
     as.id = id;
   }
   if (k < 0) {
-    if (nstaged_ >= sg->cap) {
-      if (grow_staging(nstaged_ + 1) != 0) return -1;
-      sg = &stage_[cur_];
-    }
     k = nstaged_++;
     as.slot = k;
     sg->addr[k] = addr;

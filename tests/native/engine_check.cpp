@@ -179,12 +179,41 @@ void send_release() {
   p.check("sends");
 }
 
+// A send that fails leaves its address's id as it was: the next send of that id writes it.
+void failed_send() {
+  const int n = 1500;
+  Program p(0);
+  p.x.assign(n, 0.0);
+  p.id.assign(n, 7);
+  for (int a = 0; a < n; ++a) {
+    p.send(a, a);
+    if (a % 500 == 499) EXPECT(p.e.force_prediction(0) == 0, "flush");
+  }
+  int failed = 0;
+  for (int a = 0; a < n; ++a) {
+    // 1024 rows are staged: this send asks for more
+    if (a == 1024) fake::fail_in["hostmalloc"] = 1;
+    const double x[3] = {p.x[a] = 3.0 * a, 0, 0}, z[3] = {0, 0, 0};
+    p.id[a] = 50000 + a;
+    if (p.e.set_j_particle(a, p.id[a], 0, 0, 1, z, z, z, x, z, z, 0) != 0) {
+      ++failed;
+      EXPECT(p.e.force_prediction(0) == 0, "flush");
+      p.send(a, p.x[a]);
+      EXPECT(p.call(n, 5) == 0 && p.results(n, 5) == 0, "call");
+    }
+  }
+  fake::fail_in.clear();
+  EXPECT(failed == 1, "%d sends failed", failed);
+  p.check("after a failed send");
+}
+
 int main(int argc, char** argv) {
   const std::string want = argc > 1 ? argv[1] : "";
   const struct { const char* name; void (*f)(); } checks[] = {
       {"failed_calls", failed_calls},
       {"failed_growth", failed_growth},
       {"send_release", send_release},
+      {"failed_send", failed_send},
   };
   int ran = 0;
   for (const auto& c : checks)
