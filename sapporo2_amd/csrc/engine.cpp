@@ -1942,7 +1942,7 @@ int Engine::load_state(const void* buf, long long bytes) {
   if (h.ncl && set_clusters(h.ncl, sizes.data()) != 0) return -1;
   if (cl_total_ > h.n) return fail("load_state: corrupt cluster sizes");
   nj_max_ = std::max({h.nj_max, h.max_addr + 1, cl_total_});  // the source's logical capacity
-  if ((int)addr_.size() < nj_max_ && grow_maps() != 0) return -1;
+  if (grow_maps() != 0) return -1;  // or shrinks them: sends beyond it are refused
   std::fill(addr_.begin(), addr_.end(), AddrState{});  // the dump's ids are not looked at here
   if (ensure_store(std::max(h.n, 1)) != 0) return -1;
   // clear the whole store: addresses beyond the dump's were never set there

@@ -179,6 +179,24 @@ void send_release() {
   p.check("sends");
 }
 
+// A load takes the dump's capacity: addresses beyond it are refused as on an engine
+// that never held more, whatever this one held before.
+void load_capacity() {
+  Program small(1000);
+  std::vector<char> dump((size_t)small.e.state_bytes());
+  EXPECT(small.e.save_state(dump.data(), (long long)dump.size()) == 0, "save");
+  Program p(60000);
+  EXPECT(p.e.load_state(dump.data(), (long long)dump.size()) == 0, "load");
+  const double z[3] = {0, 0, 0};
+  for (Engine* e : {&small.e, &p.e})
+    EXPECT(e->set_j_particle(50000, 1, 0, 0, 1, z, z, z, z, z, z, 0) != 0, "address beyond the dump's capacity");
+  p.x.assign(1000, 0.0);
+  p.id.assign(1000, 0);
+  for (int k = 0; k < 1000; ++k) { p.x[k] = k; p.id[k] = 10 + k; }
+  p.send(999, 5.0, 12);
+  p.check("after a load");
+}
+
 // A send that fails leaves its address's id as it was: the next send of that id writes it.
 void failed_send() {
   const int n = 1500;
@@ -213,6 +231,7 @@ int main(int argc, char** argv) {
       {"failed_calls", failed_calls},
       {"failed_growth", failed_growth},
       {"send_release", send_release},
+      {"load_capacity", load_capacity},
       {"failed_send", failed_send},
   };
   int ran = 0;
