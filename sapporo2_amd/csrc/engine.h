@@ -100,6 +100,7 @@ class Engine {
   void set_split_major(bool on) { ovr_smajor_ = on ? 1 : 0; }
   void set_ngb_pipeline(bool on) { ovr_pipe_ = on ? 1 : 0; }
   sapk::ForceConfig choose_config(int ni, int nj, bool ngb) const;
+  sapk::ForceConfig split_config(int P, long S, int ni, int nj) const;
   // Launch-shape table written by sapporo2_amd/autotune.py: lines
   // "order precision ngb log2(ni bucket) log2(nj) P log2(j per split)".
   int load_tuning(const char* path);

@@ -171,15 +171,27 @@ struct SmallArgs {
 };
 
 // Launch geometry of one force call: each wave owns P i-particles and Q = 64/P
-// j-lanes per i-particle over one of S contiguous j-ranges of jchunk.
-// smajor: wave-to-split mapping; pipe: neighbour-id stores deferred by one group;
+// j-lanes per i-particle over one of S contiguous j-ranges of up to jchunk
+// (Splits).  smajor: wave-to-split mapping; pipe: neighbour-id stores deferred by one group;
 // ahead (P = 64): records loaded ahead of the pairs.  small: k_force_small, S
 // work-groups of jchunk j (whole tiles of 256), one partial row each.
 struct ForceConfig { int P; int S; int jchunk; int smajor; int pipe; int ahead; int small; };
 
-// Iterations of a lane that the pair loop takes at a time; a j-split is a whole
-// number of them (SUB * Q j), except for what the last split has left.
+// Iterations of a lane that the pair loop takes at a time.
 constexpr int FORCE_SUB = 16;
+
+// The j-ranges of a launch: nj in units of FORCE_SUB iterations (of one, where a
+// range is shorter than that), q or q + 1 units each, so that ranges differ by one
+// unit at most and only a launch of fewer units than ranges has empty ones.
+struct Splits {
+  int unit, q, r;
+  __host__ __device__ int begin(int s) const { return unit * (s * q + (s < r ? s : r)); }
+};
+inline Splits make_splits(int P, int S, int nj) {
+  const int Q = 64 / P, unit = (long)nj >= (long)S * Q * FORCE_SUB ? Q * FORCE_SUB : Q;
+  const int n = (nj + unit - 1) / unit;
+  return Splits{unit, n / S, n % S};
+}
 
 // Partial-sum rows a force launch writes per i-particle.  With S a multiple of
 // 4 and split-minor wave order the 4 waves of a work-group are 4 consecutive

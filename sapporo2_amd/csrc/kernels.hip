@@ -717,7 +717,7 @@ __global__ __launch_bounds__(256) void k_force(
     const typename RecOf<ORDER, F64>::T* __restrict__ rec, const int2* __restrict__ idr, const int nj,
     const double* __restrict__ ibuf, const int* __restrict__ iid, const CallDesc* __restrict__ cd,
     double* __restrict__ part, double* __restrict__ part_ds2, int* __restrict__ part_addr,
-    int* __restrict__ ngb_cnt, int* __restrict__ ngb_list, const int S, const int jchunk, const int smajor,
+    int* __restrict__ ngb_cnt, int* __restrict__ ngb_list, const int S, const Splits sp, const int smajor,
     const int blockred) {
   constexpr int NF = nf<ORDER>();
   // the call's values come from the descriptor; the grid may cover more
@@ -737,8 +737,8 @@ __global__ __launch_bounds__(256) void k_force(
   // scalar-cache lines; otherwise consecutive waves walk the splits of one group
   const int g = smajor ? wave % G : wave / S;
   const int sidx = smajor ? wave / G : wave - g * S;
-  const int jb = sidx * jchunk;
-  const int je = min(nj, jb + jchunk);
+  const int jb = sp.begin(sidx);
+  const int je = min(nj, sp.begin(sidx + 1));
   double T[NF];
   double dsd;
   int nnaddr, islot;
@@ -1426,9 +1426,10 @@ template <int OR, bool FP, int P, bool PIPE, bool AHEAD>
 static void launch_force_w(hipStream_t s, const ForceArgs& a, const ForceConfig& c) {
   const long G = (a.grid_ni + P - 1) / P;
   const dim3 nb(blocks_for(G * c.S, 4)), bs(256);
+  const Splits sp = make_splits(P, c.S, a.nj);
   const auto* rec = reinterpret_cast<const typename RecOf<OR, FP>::T*>(a.rec);
 #define SAPK_FORCE_ARGS rec, a.idr, a.nj, a.ibuf, a.iid, a.cd, a.part, a.part_ds2, \
-                        a.part_addr, a.ngb_cnt, a.ngb_list, c.S, c.jchunk, c.smajor, partial_rows(c) != c.S ? 1 : 0
+                        a.part_addr, a.ngb_cnt, a.ngb_list, c.S, sp, c.smajor, partial_rows(c) != c.S ? 1 : 0
   if (a.ngb_on) hipLaunchKernelGGL((k_force<OR, FP, P, true, PIPE, AHEAD>), nb, bs, 0, s, SAPK_FORCE_ARGS);
   else hipLaunchKernelGGL((k_force<OR, FP, P, false, false, AHEAD>), nb, bs, 0, s, SAPK_FORCE_ARGS);
 #undef SAPK_FORCE_ARGS
@@ -1484,7 +1485,7 @@ int launch_force(hipStream_t s, int order, bool f64, const ForceArgs& a, const F
     sm.tiles = c.jchunk / 256;
     return launch_force_small(s, order, f64, sm, c, false);
   }
-  if (c.S <= 0 || c.jchunk <= 0 || (long)c.S * c.jchunk < a.nj) return -3;
+  if (c.S <= 0) return -3;
   int rc = 0;
   dispatch_op(order, f64, [&](auto OR, auto FP) { rc = launch_force_t<decltype(OR)::value, decltype(FP)::value>(s, a, c); });
   return rc;

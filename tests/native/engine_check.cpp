@@ -225,6 +225,48 @@ void failed_send() {
   p.check("after a failed send");
 }
 
+// Work-groups go to the 8 XCDs in turn: the j that a launch gives them.
+double xcd_balance(const ForceConfig& c, int ni, int nj) {
+  const int G = (ni + c.P - 1) / c.P, nb = c.S / 4;
+  const Splits sp = make_splits(c.P, c.S, nj);
+  std::vector<double> j(8, 0.0);
+  for (int g = 0; g < G; ++g)
+    for (int b = 0; b < nb; ++b)
+      j[(size_t)(g * nb + b) % 8] += std::min(nj, sp.begin(4 * b + 4)) - std::min(nj, sp.begin(4 * b));
+  double top = 0, sum = 0;
+  for (double v : j) { top = std::max(top, v); sum += v; }
+  return top * 8 / sum;
+}
+
+// Large calls of any size give the 8 XCDs the same work, to the ranges' unit; splits
+// cover the j once, in order.
+void xcd_shapes() {
+  for (int f64 = 0; f64 < 2; ++f64) {
+    Engine e;
+    EXPECT(e.open(0, ORDER_H4, f64 ? PREC_DOUBLE : PREC_DS) == 0, "open");
+    for (int nj : {65536, 100003, 131072, 200003, 262144, 1048577})
+      for (int ni = 2000; ni <= NPIPES; ni += 237) {
+        const ForceConfig c = e.choose_config(ni, nj, true);
+        const double b = xcd_balance(c, ni, nj);
+        EXPECT(b < 1.02, "%d i x %d j, S = %d: the busiest XCD has %.3f of the mean", ni, nj, c.S, b);
+      }
+    for (int nj : {1, 15, 16, 17, 63, 64, 65, 1000, 4097, 131071})
+      for (int S : {1, 3, 16, 33, 200, 1000})
+        for (int P : {64, 16, 4, 1}) {
+          e.set_force_override(P, S);
+          const ForceConfig c = e.choose_config(100, nj, true);
+          const Splits sp = make_splits(c.P, c.S, nj);
+          int longest = 0;
+          for (int k = 0; k < c.S; ++k) {
+            EXPECT(sp.begin(k + 1) >= sp.begin(k), "order");
+            longest = std::max(longest, sp.begin(k + 1) - sp.begin(k));
+          }
+          EXPECT(sp.begin(0) == 0 && sp.begin(c.S) >= nj && sp.begin(c.S) - nj < sp.unit, "cover %d", nj);
+          EXPECT(longest == c.jchunk, "longest range %d, jchunk %d", longest, c.jchunk);
+        }
+  }
+}
+
 int main(int argc, char** argv) {
   const std::string want = argc > 1 ? argv[1] : "";
   const struct { const char* name; void (*f)(); } checks[] = {
@@ -233,6 +275,7 @@ int main(int argc, char** argv) {
       {"send_release", send_release},
       {"load_capacity", load_capacity},
       {"failed_send", failed_send},
+      {"xcd_shapes", xcd_shapes},
   };
   int ran = 0;
   for (const auto& c : checks)
