@@ -1450,9 +1450,15 @@ int Engine::grav_calc_scratch(void* scratch, size_t bytes, int nj, int ni, const
     const size_t r = (size_t)partial_rows(c) * ni;
     return al(sizeof(CallDesc)) + al(sizeof(double) * NF * r) + al(sizeof(double) * r) + al(sizeof(int) * r);
   };
-  while (need(cfg) > bytes && cfg.S > 1) {
-    cfg.jchunk *= 2;
-    cfg.S = (nj + cfg.jchunk - 1) / cfg.jchunk;
+  // Half the splits until the rows fit, in whole work-groups (which write one row for
+  // four splits; a count that was none wrote four times the rows and was halved
+  // further), while there are many in whole eights of these.  us with such a count and
+  // now: 8192 i x 200003 j H4 mixed 1355, 1134, FP64 2342, 1844, H6 mixed 2302, 1661.
+  // Halves keep the ranges of a power of two in j at whole tiles (16384 x 131072: 128
+  // splits 1379, as many as fit, 224, 1498 against 1460 on another box).
+  while (need(cfg) > bytes && cfg.S > 4) {
+    const long S = cfg.S / 2;
+    cfg = split_config(cfg.P, S >= 128 ? (S + 31) / 32 * 32 : S, ni, nj);
   }
   if (need(cfg) > bytes) return fail("grav_calc_noalloc: call too large for the scratch region");
   const size_t r = (size_t)partial_rows(cfg) * ni;

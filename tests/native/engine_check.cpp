@@ -267,6 +267,42 @@ void xcd_shapes() {
   }
 }
 
+// The allocation-free call: rows within the scratch region, and no fewer splits than a
+// halving needs for that (a split count that is no whole work-group writes four times
+// the rows).
+void noalloc_shapes() {
+  const size_t bytes = size_t(64) << 20;
+  std::vector<char> scratch(bytes);
+  fake::device_mem[scratch.data()] = bytes;
+  std::vector<int> ids(NPIPES, 1);
+  std::vector<double> in(10 * NPIPES, 0.0), out(13 * NPIPES);
+  for (int order : {ORDER_H4, ORDER_H6}) {
+    Program p(1000, order);
+    for (int nj : {100003, 131072, 200003, 300000}) {
+      std::vector<int> a(1, nj - 1), id(1, 5);
+      std::vector<double> m(1, 1.0), x(3, 0.0);
+      EXPECT(p.e.set_j_particles(1, a.data(), id.data(), nullptr, nullptr, m.data(), nullptr, nullptr, nullptr, x.data(),
+                                 nullptr, nullptr, nullptr) == 0, "send");
+      p.e.set_time(0.0);
+      EXPECT(p.e.force_prediction(nj) == 0, "flush");
+      for (int ni : {65, 1000, 4096, 5000, 8192, 12345, 15000, 16384}) {
+        const ForceConfig direct = p.e.choose_config(ni, nj, false);
+        p.e.set_time(1.0);
+        EXPECT(p.e.grav_calc_scratch(scratch.data(), bytes, nj, ni, ids.data(), in.data(), 1e-4, out.data(), nullptr) == 0,
+               "%d x %d", ni, nj);
+        const ForceConfig c = fake::last_cfg;
+        const double row = ni * (8.0 * (part_fields(order) + 1) + 4), rows = partial_rows(c);
+        EXPECT(c.S == direct.S || rows * 2.3 * row > (double)bytes, "%d x %d: %d splits, %g rows of %g", ni, nj, c.S,
+               rows, row);
+        EXPECT(xcd_balance(c, ni, nj) < 1.02, "%d x %d: XCDs", ni, nj);
+        p.e.synchronize();
+      }
+    }
+  }
+  fake::device_mem.erase(scratch.data());
+  EXPECT(fake::violations == 0, "rows");
+}
+
 int main(int argc, char** argv) {
   const std::string want = argc > 1 ? argv[1] : "";
   const struct { const char* name; void (*f)(); } checks[] = {
@@ -276,6 +312,7 @@ int main(int argc, char** argv) {
       {"load_capacity", load_capacity},
       {"failed_send", failed_send},
       {"xcd_shapes", xcd_shapes},
+      {"noalloc_shapes", noalloc_shapes},
   };
   int ran = 0;
   for (const auto& c : checks)

@@ -29,7 +29,8 @@ def harness(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("check", ["failed_calls", "failed_growth", "send_release", "failed_send", "load_capacity", "xcd_shapes"])
+@pytest.mark.parametrize("check", ["failed_calls", "failed_growth", "send_release", "failed_send", "load_capacity", "xcd_shapes",
+                                   "noalloc_shapes"])
 def test_engine(harness, check):
     env = dict(os.environ, SAPPORO2_AMD_HOST_THREADS="4")
     r = subprocess.run([harness, check], capture_output=True, text=True, env=env, timeout=300)

@@ -144,3 +144,29 @@ def test_noalloc_matches_regular_entry(prec):
             assert isinstance(_noalloc(eng, hip, n, ids[s2], px[s2], pv[s2], eps2), dict)
     finally:
         hip.free_all()
+
+
+@pytest.mark.parametrize("prec", [sa.DOUBLESINGLE, sa.DOUBLE])
+@pytest.mark.parametrize("ni", [15001, 16384])
+def test_noalloc_coarsened_split_of_odd_nj(prec, ni):
+    """Rows beyond the scratch array at a j count that is no power of two: fewer splits,
+    results as the regular call's."""
+    n, eps2 = 70003, 1e-6
+    m, x, v = ics.plummer(n, seed=303)
+    ids = np.arange(n, dtype=np.int32)
+    hip = Hip()
+    try:
+        with sa.Engine(sa.FOURTH, prec) as eng:
+            eng.set_j_particles(np.arange(n), ids, m, x, v)
+            eng.set_time(0.0)
+            eng.force_prediction(n)
+            _say(f"noalloc coarsened prec={prec} ni={ni}")
+            s = np.sort(np.random.Generator(np.random.PCG64(304)).choice(n, ni, replace=False))
+            eng.start_grav_calc(n, ids[s], x[s], v[s], eps2, None)
+            reg = eng.get_grav_results(n, ni)
+            got = _noalloc(eng, hip, n, ids[s], x[s], v[s], eps2)
+            check_forces(got, reg, 1, TOL[prec], label=f"noalloc coarsened prec={prec} ni={ni}")
+            assert np.array_equal(got["nnb"], reg["nnb"])
+            assert np.array_equal(got["dsmin"], reg["dsmin"], equal_nan=True)
+    finally:
+        hip.free_all()
