@@ -1808,29 +1808,46 @@ int Engine::retrieve_predicted_j_particles(int n, const int* addr, double* mass,
   if (flush_updates() != 0) return -1;
   for (int k = 0; k < n; ++k)
     if (addr[k] < 0 || addr[k] > max_addr_) return fail("retrieve_predicted_j_particles: address never set");
-  // addresses and rows go through pinned memory that the kernel reads and writes
-  if (gather_hcap_ < (size_t)n) {
+  // Addresses and rows go through pinned memory that the kernel reads and writes: up to
+  // NPIPES the call block, which no call uses now (two pinned allocations made the
+  // first pick-up of 2500 on an engine 700 us for 100-200), beyond that their own.
+  double *rows_h = reinterpret_cast<double*>(reinterpret_cast<char*>(call_h_) + CALL_HDR + call_ids_bytes(NPIPES));
+  int* addr_h = reinterpret_cast<int*>(reinterpret_cast<char*>(call_h_) + CALL_HDR);
+  const ptrdiff_t alias = reinterpret_cast<char*>(call_hd_) - reinterpret_cast<char*>(call_h_);
+  double* rows_hd = reinterpret_cast<double*>(reinterpret_cast<char*>(rows_h) + alias);
+  int* addr_hd = reinterpret_cast<int*>(reinterpret_cast<char*>(addr_h) + alias);
+  static_assert(IBUF_FIELDS >= 10, "gathered rows in the call block");
+  if (n <= NPIPES) {
+    if (desc_pending_ && desc_seq_ > done_seq_) HIPCHK(hipEventSynchronize(ev_desc_), "call block wait");
+    desc_pending_ = false;
+  } else if (gather_hcap_ < (size_t)n) {
     hfree(gather_h_);
     hfree(gaddr_h_);
     gather_hcap_ = 0;
-    const size_t nc = std::max<size_t>(n, 1024);
+    const size_t nc = (size_t)n;
     HIPCHK(hmap(&gather_h_, &gather_hd_, nc * 10, true), "pinned gather rows");
     HIPCHK(hmap(&gaddr_h_, &gaddr_hd_, nc, true), "pinned gather addresses");
     gather_hcap_ = nc;
   }
-  memcpy(gaddr_h_, addr, sizeof(int) * (size_t)n);
+  if (n > NPIPES) {
+    rows_h = gather_h_;
+    addr_h = gaddr_h_;
+    rows_hd = gather_hd_;
+    addr_hd = gaddr_hd_;
+  }
+  memcpy(addr_h, addr, sizeof(int) * (size_t)n);
   GatherArgs g{};
   g.st = st_;
   g.n = n;
-  g.out = gather_hd_;
-  g.addr = gaddr_hd_;
+  g.out = rows_hd;
+  g.addr = addr_hd;
   g.done = done_hd_;
   g.done_ctr = done_ctr_d_;
   g.seq = next_seq();
   if (launch_gather_pred(stream_, order_, f64_, g) != 0) return fail("gather launch", hipGetLastError());
   if (wait_word() != 0) return -1;
   HIPCHK(hipGetLastError(), "device error");
-  const double* p = gather_h_;
+  const double* p = rows_h;
   auto rows = [&](size_t b, size_t e) {
     auto vec = [&](double (*dst)[3], int f) {
       if (!dst) return;

@@ -303,6 +303,34 @@ void noalloc_shapes() {
   EXPECT(fake::violations == 0, "rows");
 }
 
+// Picking up the active particles of a step asks for no memory, between calls with and
+// without graphs; more than a call's worth of them does once.
+void pick_up() {
+  const int n = 40000;
+  for (int graphs = 0; graphs < 2; ++graphs) {
+    Program p(n);
+    p.e.set_graphs(graphs != 0);
+    for (int m : {1, 2500, NPIPES, 30000}) {
+      p.send(m / 2, 4.0 * m);
+      EXPECT(p.call(n, 100) == 0, "call");
+      std::vector<int> a(m);
+      for (int k = 0; k < m; ++k) a[k] = m - 1 - k;
+      std::vector<double> x(3 * (size_t)m), mass(m);
+      const int before = fake::host_allocs;
+      const size_t bytes = fake::device_bytes;
+      EXPECT(p.e.retrieve_predicted_j_particles(m, a.data(), mass.data(), reinterpret_cast<double(*)[3]>(x.data()),
+                                                nullptr, nullptr) == 0, "pick-up of %d", m);
+      EXPECT((fake::host_allocs == before) == (m <= NPIPES), "%d: %d pinned allocations", m, fake::host_allocs - before);
+      EXPECT(fake::device_bytes == bytes, "%d: device memory", m);
+      int wrong = 0;
+      for (int k = 0; k < m; ++k) wrong += x[3 * (size_t)k] != p.x[a[k]];
+      EXPECT(wrong == 0, "%d of %d rows", wrong, m);
+      EXPECT(p.results(n, 100) == 0 && p.call(n, 5) == 0 && p.results(n, 5) == 0, "calls after it");
+    }
+    p.check("pick-up");
+  }
+}
+
 int main(int argc, char** argv) {
   const std::string want = argc > 1 ? argv[1] : "";
   const struct { const char* name; void (*f)(); } checks[] = {
@@ -313,6 +341,7 @@ int main(int argc, char** argv) {
       {"failed_send", failed_send},
       {"xcd_shapes", xcd_shapes},
       {"noalloc_shapes", noalloc_shapes},
+      {"pick_up", pick_up},
   };
   int ran = 0;
   for (const auto& c : checks)
