@@ -1297,7 +1297,7 @@ int Engine::start_grav_calc(int nj, int ni, const int* id, const double (*xi)[3]
   // bucket share a captured sequence); direct launches cover ni exactly.  The
   // finalize shape follows the bucket in both cases, so results agree.
   const int grid_ni = graphs_ ? std::min(bucket, NPIPES) : ni;
-  if (ensure_partials((size_t)cfg.S * grid_ni) != 0) return -1;
+  if (ensure_partials((size_t)partial_rows(cfg) * grid_ni) != 0) return -1;
   // device window: all device work (after the host->device copies of a replayed call)
   if (timing_) HIPCHK(hipEventRecord(ev_d0_, stream_), "event");
   if (graphs_) {

@@ -331,6 +331,18 @@ void pick_up() {
   }
 }
 
+// An engine's partial rows take what its calls write.
+void scratch_size() {
+  for (int ni : {100, 5000, 16384}) {
+    Program p(131072);
+    EXPECT(p.call(131072, ni) == 0 && p.results(131072, ni) == 0, "call");
+    const size_t want = (size_t)partial_rows(fake::last_cfg) * ni * part_fields(ORDER_H4) * 8;
+    const size_t got = fake::bytes_from(fake::last_force.part);
+    EXPECT(got == want, "%d: %zu bytes of rows, %zu are written", ni, got, want);
+    p.check("rows");
+  }
+}
+
 int main(int argc, char** argv) {
   const std::string want = argc > 1 ? argv[1] : "";
   const struct { const char* name; void (*f)(); } checks[] = {
@@ -342,6 +354,7 @@ int main(int argc, char** argv) {
       {"xcd_shapes", xcd_shapes},
       {"noalloc_shapes", noalloc_shapes},
       {"pick_up", pick_up},
+      {"scratch_size", scratch_size},
   };
   int ran = 0;
   for (const auto& c : checks)
