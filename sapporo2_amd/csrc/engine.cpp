@@ -802,7 +802,8 @@ ForceConfig Engine::choose_config(int ni, int nj, bool ngb) const {
       jchunk_t = 1L << best->jlog;
     }
   }
-  if (plain && jchunk_t == 0 && !ovr_smajor_ && !ovr_pipe_) {
+  const bool rule = plain && jchunk_t == 0 && !ovr_smajor_ && !ovr_pipe_;
+  if (rule) {
     if (ni <= SMALL_NI) {
       // At most SMALL_ROWS work-groups, each one row for the finalize to read.
       const int ntiles = (nj + 255) / 256, tiles = (ntiles + SMALL_ROWS - 1) / SMALL_ROWS;
@@ -814,7 +815,7 @@ ForceConfig Engine::choose_config(int ni, int nj, bool ngb) const {
   const int Q = 64 / P;
   const long G = (ni + P - 1) / P;
   long S;
-  if (P == 64 && plain && jchunk_t == 0) {
+  if (rule) {
     // One round of waves (8 per SIMD mixed, 5 in FP64) while that leaves a wave
     // MIN_CHUNK j or more; the fixed cost of a wave (its i-particles, cold
     // records, epilogue) is then small against its pairs.  More i-groups take

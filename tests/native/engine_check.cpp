@@ -343,6 +343,21 @@ void scratch_size() {
   }
 }
 
+// Split-major order and pipelined list stores keep the general shapes at every active
+// count: at least 512 j a split (split-major launches write a row for each).
+void mode_shapes() {
+  Engine e;
+  EXPECT(e.open(0, ORDER_H4, PREC_DS) == 0, "open");
+  for (int mode = 0; mode < 2; ++mode) {
+    e.set_split_major(mode == 0);
+    e.set_ngb_pipeline(mode == 1);
+    for (int ni : {1, 20, 33, 64, 65, 333, 5000, 16384}) {
+      const ForceConfig c = e.choose_config(ni, 131072, true);
+      EXPECT(c.small == 0 && c.jchunk >= 512, "%d i: %d splits of %d", ni, c.S, c.jchunk);
+    }
+  }
+}
+
 int main(int argc, char** argv) {
   const std::string want = argc > 1 ? argv[1] : "";
   const struct { const char* name; void (*f)(); } checks[] = {
@@ -355,6 +370,7 @@ int main(int argc, char** argv) {
       {"noalloc_shapes", noalloc_shapes},
       {"pick_up", pick_up},
       {"scratch_size", scratch_size},
+      {"mode_shapes", mode_shapes},
   };
   int ran = 0;
   for (const auto& c : checks)
