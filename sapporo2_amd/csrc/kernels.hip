@@ -503,17 +503,26 @@ constexpr int SUB = FORCE_SUB;
 static_assert(KT % SUB == 0 && SUB % 4 == 0, "fold");
 
 // J-records on their way through the scalar cache (lane shape P = 64): JU
-// consecutive records held in SGPRs, as one or two wide scalar loads.
+// consecutive records held in SGPRs, as one or two wide scalar loads.  Units lie at
+// multiples of their size, which is what the loads' types claim: 96-byte units are
+// aligned to 32 bytes, not to the 64 of a 16-register load.
 typedef int v8i __attribute__((ext_vector_type(8)));
 typedef int v16i __attribute__((ext_vector_type(16)));
+typedef v16i v16i_at32 __attribute__((aligned(32)));
 template <typename Rec> struct JUnit {
   static constexpr int JU = sizeof(Rec) == 48 ? 2 : 1;
   static constexpr bool TAIL = sizeof(Rec) * JU == 96;
+  static_assert(sizeof(Rec) * JU % (TAIL ? alignof(v16i_at32) : alignof(v16i)) == 0 &&
+                sizeof(Rec) * JU % alignof(v8i) == 0, "unit alignment");
   v16i h;
   v8i t;
   __device__ __forceinline__ void load(const Rec* __restrict__ p) {
-    h = *reinterpret_cast<const v16i*>(p);
-    if constexpr (TAIL) t = *reinterpret_cast<const v8i*>(reinterpret_cast<const char*>(p) + 64);
+    if constexpr (TAIL) {
+      h = *reinterpret_cast<const v16i_at32*>(p);
+      t = *reinterpret_cast<const v8i*>(reinterpret_cast<const char*>(p) + 64);
+    } else {
+      h = *reinterpret_cast<const v16i*>(p);
+    }
   }
   // The loads have arrived (scalar loads return out of order: a wait is for
   // all of them, so this comes before the next unit's loads are issued).
