@@ -62,3 +62,23 @@ def test_split_counts(prec, S):
         eng.set_force_override(64, S)
         sel = np.arange(0, n, 19)
         _check(eng, sa.FOURTH, prec, sys_, sel, n, True, f"splits prec={prec} S={S}")
+
+
+@pytest.mark.parametrize("order", [sa.FOURTH, sa.SIXTH])
+def test_mixed_without_records_ahead(order):
+    """More waves than take their records ahead in mixed precision (4096): the kernel of
+    large calls, at counts that leave remainders of i-groups, splits and tiles."""
+    n = 9000
+    m, x, v, ids, h2 = plummer_system(n, seed=94)
+    h2 = h2.copy()
+    h2[::7] = 4.0                                   # most of the system
+    rng = np.random.Generator(np.random.PCG64(95))
+    z = np.zeros((n, 3))
+    with sa.Engine(order, sa.DOUBLESINGLE) as eng:
+        load_engine(eng, m, x, v, ids, z, z, *([z, z] if order >= sa.SIXTH else [None, None]))
+        eng.set_time(0.0)
+        for ni, nj, lists in [(4097, 8991, True), (4097, 8991, False), (8191, 8999, True), (6001, 8977, False)]:
+            sel = np.sort(rng.choice(n, ni, replace=False))
+            _check(eng, order, sa.DOUBLESINGLE, (m, x, v, ids, h2), sel, nj, lists, f"full chip order={order} ni={ni} nj={nj}")
+            P, S, _ = eng.last_config()
+            assert P == 64 and (ni + 63) // 64 * S > 4096

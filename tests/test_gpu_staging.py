@@ -11,7 +11,7 @@ import pytest
 
 import oracle
 import sapporo2_amd as sa
-from _util import load_engine, plummer_system, random_derivs
+from _util import check_forces, load_engine, plummer_system, random_derivs
 
 pytestmark = pytest.mark.gpu
 
@@ -84,3 +84,38 @@ def test_update_routes_agree(order, prec):
                 assert np.array_equal(got["pos"], px) and np.array_equal(got["vel"], pv), r
                 if order >= sa.SIXTH:
                     assert np.array_equal(got["acc"], pa), r
+
+
+@pytest.mark.parametrize("prec", [sa.DOUBLESINGLE, sa.DOUBLE])
+@pytest.mark.parametrize("n,upd,again", [(7001, 4096, 1000), (7001, 4096, 4095), (7001, 7001, 0), (4000, 4000, 0)])
+def test_part_sent_early_and_all_updated(prec, n, upd, again):
+    """Rows partly on the device when the launch that predicts reads them (4096 sends are
+    copied ahead, sending one of them again takes back its row and those behind it), and
+    every predicted particle an update, in one launch (4000) and in two (7001)."""
+    m, x, v, ids, _ = plummer_system(n, seed=74)
+    acc, jrk, _, _ = random_derivs(n, 75, 0.3)
+    rng = np.random.Generator(np.random.PCG64(76))
+    tj = -rng.uniform(0, 1.0 / 256, n)
+    x = x.copy()
+    with sa.Engine(sa.FOURTH, prec) as a:
+        load_engine(a, m, x, v, ids, acc, jrk, tj=tj)
+        a.force_prediction(n)
+        print(f"staging prec={prec} n={n} updates={upd} again={again}", flush=True)
+        u = np.sort(rng.choice(n, upd, replace=False))
+        x[u] += 1e-3 * rng.normal(size=(upd, 3))
+        for q in u:
+            a.set_j_particle(q, ids[q], tj[q], 0.0, m[q], acc[q], jrk[q], v[q], x[q])
+        if again:
+            q = u[again]
+            x[q] += 0.25
+            a.set_j_particle(q, ids[q], tj[q], 0.0, m[q], acc[q], jrk[q], v[q], x[q])
+        ti = 1.0 / 512
+        a.set_time(ti)
+        sel = np.sort(rng.choice(n, 100, replace=False))
+        a.start_grav_calc(n, ids[sel], x[sel], v[sel], 1e-4)
+        res = a.get_grav_results(n, len(sel))
+        px, pv, _ = oracle.predict(sa.FOURTH, ti, tj, x, v, acc, jrk, None, None)
+        got = a.retrieve_predicted_j_particles(np.arange(n))
+        assert np.array_equal(got["pos"], px) and np.array_equal(got["vel"], pv)
+        ref = oracle.force(sa.FOURTH, x[sel], v[sel], ids[sel], px, pv, m, ids, 1e-4)
+        check_forces(res, ref, sa.FOURTH, 1e-6 if prec == sa.DOUBLESINGLE else 1e-12, label=f"n={n} updates={upd}")
