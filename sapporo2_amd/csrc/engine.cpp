@@ -524,6 +524,7 @@ int Engine::set_j_particles(int n, const int* addr, const int* id, const double*
     amax = std::max(amax, addr[k]);
     amin = std::min(amin, addr[k]);
   }
+  if (amax == INT_MAX) return fail("set_j_particles: address out of range");
   if (amax >= nj_max_) nj_max_ = amax + 1;
   if ((int)addr_.size() < nj_max_ && grow_maps() != 0) return -1;
   // On the host threads a block at a time: a block's copy is under way while the

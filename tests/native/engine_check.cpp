@@ -358,6 +358,28 @@ void mode_shapes() {
   }
 }
 
+// A batch with an address that no store can hold is refused, large batches like small
+// ones, and leaves the engine as it was.
+void batch_range() {
+  Program p(9000);
+  for (int n : {3, 7000}) {
+    std::vector<int> a(n), id(n, 1);
+    std::vector<double> m(n, 1.0), x(3 * (size_t)n, 0.0);
+    for (int k = 0; k < n; ++k) a[k] = k;
+    for (int wrong : {INT_MAX, -1}) {
+      a[0] = wrong;  // first: nothing of the batch is staged
+      EXPECT(p.e.set_j_particles(n, a.data(), id.data(), nullptr, nullptr, m.data(), nullptr, nullptr, nullptr, x.data(),
+                                 nullptr, nullptr, nullptr) != 0, "address %d in a batch of %d", wrong, n);
+    }
+  }
+  p.send(8999, 2.0, 3);
+  std::vector<int> a(7000);
+  for (int k = 0; k < 7000; ++k) a[k] = 2 * k % 9000 + (k >= 4500);
+  p.batch(a, 0.5);
+  EXPECT(p.call(9000, 100) == 0 && p.results(9000, 100) == 0, "call");
+  p.check("after refused batches");
+}
+
 int main(int argc, char** argv) {
   const std::string want = argc > 1 ? argv[1] : "";
   const struct { const char* name; void (*f)(); } checks[] = {
@@ -371,6 +393,7 @@ int main(int argc, char** argv) {
       {"pick_up", pick_up},
       {"scratch_size", scratch_size},
       {"mode_shapes", mode_shapes},
+      {"batch_range", batch_range},
   };
   int ran = 0;
   for (const auto& c : checks)

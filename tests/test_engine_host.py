@@ -30,7 +30,8 @@ def harness(tmp_path_factory):
 
 
 @pytest.mark.parametrize("check", ["failed_calls", "failed_growth", "send_release", "failed_send", "load_capacity", "xcd_shapes",
-                                   "noalloc_shapes", "pick_up", "scratch_size", "mode_shapes"])
+                                   "noalloc_shapes", "pick_up", "scratch_size", "mode_shapes",
+                                   "batch_range"])
 def test_engine(harness, check):
     env = dict(os.environ, SAPPORO2_AMD_HOST_THREADS="4")
     r = subprocess.run([harness, check], capture_output=True, text=True, env=env, timeout=300)
