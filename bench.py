@@ -57,7 +57,8 @@ FLOP_PER_INTERACTION = 60.0          # test_gravity_block.cpp:271
 # the updates and copies the call's inputs from host memory), per j-particle: reads
 # t, m, x, v, a, j (14 doubles) and the id; writes the working-precision record (48 B mixed,
 # 64 B FP64) and, mixed only, the FP64 predicted position and velocity kept for read-back.
-# Scatter (a launch of its own only where updates change ids), per staged update: reads the row
+# Scatter (a launch of its own where updates change ids or are more than 4096; up to then they
+# are applied in the predictor's), per staged update: reads the row
 # (16 doubles and the address/id pair), writes the 16 raw fields and the id.
 PREDICT_BYTES = {"mixed": 116 + 48 + 48, "fp64": 116 + 64}
 SCATTER_BYTES = 136 + 128 + 4

@@ -125,9 +125,10 @@ int sapamd_retrieve_predicted_j_particles(sapamd_engine *e, int n, const int *ad
 int sapamd_graph_count(sapamd_engine *e);
 float sapamd_last_force_ms(sapamd_engine *e);
 float sapamd_last_predict_ms(sapamd_engine *e);
-/* time of the launch that applied the last call's j-updates (timing on) and, in
- * *nupd (may be NULL), their number; 0 when the call had none or applied them in
- * the predictor's launch (updates that change no id) */
+/* time of the launch that applied the last call's j-updates by themselves (timing
+ * on) and, in *nupd (may be NULL), their number: with a prediction, updates that
+ * change an id or more than 4096.  0 when the call had none or applied them in the
+ * launch that predicts (or computes the forces), or predicted nothing */
 float sapamd_last_scatter_ms(sapamd_engine *e, int *nupd);
 /* finalize kernel time of the last call (timing on): reduction of the partial
  * sums, list sort, and the result and list writes into host memory */

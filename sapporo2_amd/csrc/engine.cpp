@@ -749,9 +749,7 @@ int Engine::ensure_partials(size_t entries) {
   return 0;
 }
 
-// Launch shape: P i-particles per wave (64 unless fewer are active), S j-splits
-// so that about WAVES_PER_SIMD_TARGET waves per SIMD exist, each split at least
-// MIN_ITERS_PER_LANE iterations per lane.
+// Launch-shape table for choose_config; returns its entries.
 int Engine::load_tuning(const char* path) {
   tune_.clear();
   tune_path_.clear();
@@ -817,8 +815,11 @@ ForceConfig Engine::choose_config(int ni, int nj, bool ngb) const {
   const long G = (ni + P - 1) / P;
   long S;
   if (rule) {
-    // One round of waves (8 per SIMD mixed, 5 in FP64) while that leaves a wave
-    // MIN_CHUNK j or more; the fixed cost of a wave (its i-particles, cold
+    // One round of waves while that leaves a wave MIN_CHUNK j or more, 8 per SIMD
+    // mixed and 5 in FP64 as Hermite-4 with lists keeps resident.  (Mixed with
+    // records ahead 7, Hermite-6 with lists 6; Hermite-6 mixed 7, with lists 6;
+    // FP64 without lists 6; Hermite-6 FP64 4: there a round here is up to 1.33 of
+    // the chip's.)  The fixed cost of a wave (its i-particles, cold
     // records, epilogue) is then small against its pairs.  More i-groups take
     // several rounds of MAX_CHUNK j, so that the last round is short, up to
     // MAX_WAVES, where the partial rows begin to cost more than the balance gains.
@@ -1296,8 +1297,8 @@ int Engine::start_grav_calc(int nj, int ni, const int* id, const double (*xi)[3]
   predict_ = false;  // reference 698
   const ForceConfig cfg = choose_config(ni, nj, ngb_on);
   // With graphs the grid covers the power-of-two bucket of ni (calls of one
-  // bucket share a captured sequence); direct launches cover ni exactly.  The
-  // finalize shape follows the bucket in both cases, so results agree.
+  // bucket and launch shape share a captured sequence); direct launches cover ni
+  // exactly.  The finalize shape follows the bucket in both cases, so results agree.
   const int grid_ni = graphs_ ? std::min(bucket, NPIPES) : ni;
   if (ensure_partials((size_t)partial_rows(cfg) * grid_ni) != 0) return -1;
   // device window: all device work (after the host->device copies of a replayed call)

@@ -7,12 +7,14 @@
 //     in pinned host memory, large ones sent ahead with asynchronous copies, and
 //     applied by a kernel (no per-particle map lookups on the device);
 //   * each force call is prep (updates, prediction, inputs) -> force -> finalize
-//     on one HIP stream; the finalize writes the result rows and the sorted, packed
+//     on one HIP stream, a call of few i-particles (updates, prediction, forces)
+//     -> finalize; the finalize writes the result rows and the sorted, packed
 //     neighbour lists straight into host-mapped pinned memory, so lasthalf and
-//     read_neighbour_list wait for one completion event and copy nothing.  The
-//     kernels take the call's values (block time, softening, counts) from a
-//     small device-side descriptor, so with graphs on the sequence is captured
-//     once per launch shape and replayed (one graph launch per call).
+//     read_neighbour_list wait for the call (a word that the finalize writes, or
+//     an event) and copy nothing.  With graphs on the kernels take the call's
+//     values (block time, softening, counts) from a small device-side descriptor,
+//     and the sequence is captured once per launch shape and replayed (one graph
+//     launch per call); direct calls pass some of them by value.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -107,13 +109,14 @@ class Engine {
   int tuning_entries() const { return (int)tune_.size(); }
   const char* tuning_path() const { return tune_path_.c_str(); }
   void set_timing(bool on) { timing_ = on; }
-  // Capture scatter..finalize as a hipGraph per launch shape and replay it.
+  // Capture scatter..finalize as a hipGraph per launch shape (of a power-of-two bucket of ni) and replay it.
   void set_graphs(bool on) { graphs_ = on; }
   bool graphs() const { return graphs_; }
   int graph_count() const { return (int)graph_cache_.size(); }
   float last_force_ms();          // force kernel time of the last call (timing on)
-  float last_predict_ms();        // predictor time of the last call (timing on, 0 if none)
-  // time of the last call's update launch and its update count (timing on; 0 if none or fused with the prediction)
+  float last_predict_ms();        // predictor time of the last call (timing on; 0 if none or in the force launch)
+  // time of the last call's update launch and its update count (timing on; 0 where the prediction's launch, or
+  // one without a prediction, applied them)
   float last_scatter_ms(int* nupd);
   float last_finalize_ms();       // finalize (reduction, list sort, host writes) time of the last call (timing on)
   float last_device_ms();         // prep..finalize (lists packed) device time of the last call (timing on)
